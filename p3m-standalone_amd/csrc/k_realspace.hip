@@ -446,26 +446,58 @@ __device__ __forceinline__ void load_erfcx_table(RsShared<FP32, VJP> &sh) {
 }
 
 // Work-item claims of the persistent grids: a claim takes `per` consecutive
-// items with one device atomic on the shared counter, which is a serial point
-// (190k single-item claims of sparse cells took most of a 2.2 ms batched
-// launch).  per = total / (8 grid), at least 1, leaves a wavefront about
-// eight claims, for the balance of clustered systems.
-__device__ __forceinline__ int claim_size(int total) { return max(1, total / ((int)gridDim.x * 8)); }
+// items.  A wavefront's first claim is its block index (no memory access),
+// the later ones take a device atomic on the shared counter, which counts
+// from the grid's first claims on.  The counter is a serial point (about
+// 18 ns an atomic): with a first claim by atomic, the 8192 wavefronts of the
+// grid took 150 us for that alone, whatever the system.  per = total /
+// (8 grid), at least 1, leaves a wavefront about eight claims, for the
+// balance of clustered systems.
+struct Claims {
+    int next, end, per, total;
+};
+__device__ __forceinline__ Claims first_claim(int total) {
+    Claims c;
+    c.total = total;
+    c.per = max(1, total / ((int)gridDim.x * 8));
+    c.next = (int)min((long)total, (long)blockIdx.x * c.per);
+    c.end = min(total, c.next + c.per);
+    return c;
+}
 
-// this wavefront's next item (next, end: its current claim), total when the
-// items are exhausted
-__device__ __forceinline__ int next_item(int *counter, int total, int per, int &next, int &end) {
-    if (next >= end) {
+// this wavefront's next item, total when the items are exhausted
+__device__ __forceinline__ int next_item(int *counter, Claims &c) {
+    if (c.next >= c.end) {
+        const int given = (int)gridDim.x * c.per; // by block index
+        if (given >= c.total || c.next >= c.total)
+            return c.total;
         int first = 0;
         if (threadIdx.x == 0)
-            first = atomicAdd(counter, per);
+            first = atomicAdd(counter, c.per);
         first = __builtin_amdgcn_readfirstlane(first);
-        if (first >= total)
-            return total;
-        next = first;
-        end = min(total, first + per);
+        if (first >= c.total - given)
+            return c.total;
+        c.next = given + first;
+        c.end = min(c.total, c.next + c.per);
     }
-    return next++;
+    return c.next++;
+}
+
+// Units of the half shell per work item: when the items are fewer than the
+// GPU has wavefront slots, an item's neighbour cells are dealt out to
+// 2^split_bits wavefronts (each walks every 2^split_bits-th live cell and
+// adds its share of the forces), so that a small system's chain of windows
+// is shared.  With the first claims by block index, whole steps: 1,000
+// particles FP64 159 -> 120 us, 7,777 mixed 192 -> 149 us, 100,000 mixed
+// 240 -> 154 us, a batch of 24 small systems 542 -> 455 us; a million
+// particles 6.26 -> 6.15 ms.
+constexpr int kMaxSplitBits = 4;
+constexpr int kSplitUnits = 4096; // about the resident wavefronts
+__device__ __forceinline__ int split_bits_of(int total) {
+    int b = 0;
+    while (b < kMaxSplitBits && (total << b) < kSplitUnits)
+        b++;
+    return b;
 }
 
 // index of the periodic image shift (wx, wy, wz) in {-1, 0, 1}^3
@@ -762,10 +794,9 @@ k_realspace(int n, const double4 *__restrict__ sorted, const float4 *__restrict_
     const int total = istart[ncell];
     double en_tot = 0.0;
     load_erfcx_table(sh);
-    const int per = claim_size(total);
-    int next = 0, end = 0;
+    Claims claims = first_claim(total);
     for (;;) {
-        const int item = next_item(counter, total, per, next, end);
+        const int item = next_item(counter, claims);
         if (item >= total)
             break;
         const int home = __float_as_int(bbox[2 * item].w), chunk = __float_as_int(bbox[2 * item + 1].w);
@@ -796,10 +827,9 @@ k_realspace_vjp(int n, const double4 *__restrict__ sorted, const float4 *__restr
     const int total = istart[ncell];
     double en_unused = 0.0;
     load_erfcx_table(sh);
-    const int per = claim_size(total);
-    int next = 0, end = 0;
+    Claims claims = first_claim(total);
     for (;;) {
-        const int item = next_item(counter, total, per, next, end);
+        const int item = next_item(counter, claims);
         if (item >= total)
             break;
         const int home = __float_as_int(bbox[2 * item].w), chunk = __float_as_int(bbox[2 * item + 1].w);
@@ -892,7 +922,7 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
                     const float4 *__restrict__ sorted32, const int4 *__restrict__ sortedq,
                     const int *__restrict__ start, const int *__restrict__ istart,
                     const float4 *__restrict__ bbox, int nc, int reach, double L, double rcut,
-                    double alpha, long stride,
+                    double alpha, long stride, int split_bits, int part,
                     double *__restrict__ fs, RsHalfShared<FP32> &sh, double &en_tot) {
     const int lane = threadIdx.x;
     const double two_a_spi = 2.0 * alpha / sqrt_pi();
@@ -1258,6 +1288,16 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
     // kept in LDS for the walk (read back uniformly), not in registers
     sh.cells[lane] = make_int4(cjb, cje, citem, (int)cinfo);
     unsigned long long cells = __ballot(live);
+    if (split_bits > 0) {
+        // this unit's share of the live cells, dealt out in turn
+        const int rank = (int)__builtin_amdgcn_mbcnt_hi((unsigned int)(cells >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo((unsigned int)cells, 0u));
+        cells = __ballot(live && (rank & ((1 << split_bits) - 1)) == part);
+        if (cells == 0) {
+            __syncthreads();
+            return;
+        }
+    }
     while (cells) {
         const int k = __builtin_ctzll(cells);
         cells &= cells - 1;
@@ -1383,16 +1423,17 @@ k_realspace_half(const double4 *__restrict__ sorted, const float4 *__restrict__ 
             sh.tab[k] = (&p3m::kErfcxDoubleCoef[0][0])[k];
     }
     __syncthreads();
-    const int per = claim_size(total);
-    int next = 0, end = 0;
+    const int sb = split_bits_of(total);
+    Claims claims = first_claim(total << sb);
     for (;;) {
-        const int item = next_item(counter, total, per, next, end);
-        if (item >= total)
+        const int unit = next_item(counter, claims);
+        if (unit >= claims.total)
             break;
+        const int item = unit >> sb;
         // the item's cell and chunk, stored with its box
         const int home = __float_as_int(bbox[2 * item].w), chunk = __float_as_int(bbox[2 * item + 1].w);
         realspace_item_half<FP32, true>(home, chunk, 0, sorted, sorted32, sortedq, start, istart, bbox, nc, reach, L,
-                                        rcut, alpha, stride, fs, sh, en_tot);
+                                        rcut, alpha, stride, sb, unit & ((1 << sb) - 1), fs, sh, en_tot);
     }
     if (energy != nullptr) {
         for (int off = 32; off > 0; off >>= 1)
@@ -1567,7 +1608,7 @@ extern "C" int p3mk_realspace_vjp(p3mk_cells *c, int n, double L, const double *
         P3MK_TRY(p3mk_alloc((void **)&a.gsorted, sizeof(double4) * ((size_t)c->nmax + kPad)));
     P3MK_TRY(build_cells(c, n, L, x, y, z, q, rcut, g, qu));
     const bool all_cells = (2 * c->reach + 1 > c->nc);
-    const dim3 grid((unsigned)c->grid);
+    const dim3 grid((unsigned)std::min<long>(c->grid, a.max_items));
     hipStream_t s = p3mk_stream(qu);
     if (all_cells)
         hipLaunchKernelGGL(k_realspace_vjp<true>, grid, dim3(kWave), 0, s, n, a.sorted, a.sorted32,
@@ -1588,7 +1629,9 @@ extern "C" int p3mk_realspace(p3mk_cells *c, int n, double L, const double *x, c
     CellArrays &a = c->a;
     hipStream_t s = p3mk_stream(qu);
     const bool all_cells = (2 * c->reach + 1 > c->nc);
-    const dim3 grid((unsigned)c->grid);
+    // no more wavefronts than units (half shell) or items can be
+    const long units = all_cells ? a.max_items : a.max_items << kMaxSplitBits;
+    const dim3 grid((unsigned)std::min<long>(c->grid, units));
     if (!all_cells) {
         // half shell: forces summed in sorted order, then added by perm
         P3MK_TRY(build_cells(c, n, L, x, y, z, q, rcut, nullptr, qu));
@@ -1684,10 +1727,9 @@ k_brealspace(const BSys *__restrict__ sys, const int *__restrict__ cell0s, int n
     __shared__ RsShared<FP32> sh;
     const int total = istart[ncell];
     load_erfcx_table(sh);
-    const int per = claim_size(total);
-    int next = 0, end = 0;
+    Claims claims = first_claim(total);
     for (;;) {
-        const int item = next_item(counter, total, per, next, end);
+        const int item = next_item(counter, claims);
         if (item >= total)
             break;
         const int home = __float_as_int(bbox[2 * item].w), chunk = __float_as_int(bbox[2 * item + 1].w);
@@ -1728,12 +1770,13 @@ k_brealspace_half(const BSys *__restrict__ sys, const int *__restrict__ cell0s, 
             sh.tab[k] = (&p3m::kErfcxDoubleCoef[0][0])[k];
     }
     __syncthreads();
-    const int per = claim_size(total);
-    int next = 0, end = 0;
+    const int sb = split_bits_of(total);
+    Claims claims = first_claim(total << sb);
     for (;;) {
-        const int item = next_item(counter, total, per, next, end);
-        if (item >= total)
+        const int unit = next_item(counter, claims);
+        if (unit >= claims.total)
             break;
+        const int item = unit >> sb;
         const int home = __float_as_int(bbox[2 * item].w), chunk = __float_as_int(bbox[2 * item + 1].w);
         const int s = p3m::fft::prefix_slot(cell0s, nsys, (long)home);
         const BSys &S = sys[s];
@@ -1741,7 +1784,8 @@ k_brealspace_half(const BSys *__restrict__ sys, const int *__restrict__ cell0s, 
             continue; // no real-space part, or nearest images (k_brealspace)
         double en = 0.0;
         realspace_item_half<FP32, FP32>(home - S.cell0, chunk, S.cell0, sorted, sorted32, sortedq, start,
-                                  istart, bbox, S.nc, S.reach, S.L, S.rcut, S.alpha, ntot, fs, sh, en);
+                                  istart, bbox, S.nc, S.reach, S.L, S.rcut, S.alpha, ntot, sb,
+                                  unit & ((1 << sb) - 1), fs, sh, en);
         if (energy != nullptr) {
             for (int off = 32; off > 0; off >>= 1)
                 en += __shfl_down(en, off, kWave);

@@ -227,3 +227,41 @@ def test_stage_ring_pair_kernel_times(pkg):
     assert len(pairs) == 3
     assert all(0.0 < pairs[k] <= stages[k, 4] for k in (0, 1))
     assert pairs[2] == 0.0
+
+
+@pytest.mark.parametrize("prec_name", ["FP64", "MIXED"])
+@pytest.mark.parametrize("cells,per_cell", [(3, 37), (6, 9), (8, 8), (13, 4), (16, 3), (17, 3)])
+def test_items_dealt_to_several_wavefronts(pkg, orc, cells, per_cell, prec_name):
+    """Systems of few work items, whose neighbour cells are dealt out to 16,
+    8, 4, 2 or one wavefront per item (items from 27 to above 4096, one cell
+    of 150 particles among them so that items of one cell differ in chunks):
+    sums of up to 16 shares per particle, so the tolerance is that of the
+    other real-space tests (FP64 1e-13; mixed 1e-6 by the fixed-point quantum
+    at these densities' closest pairs, kept above 0.05)."""
+    import torch
+
+    rcut, alpha = 3.0, 1.0
+    L = rcut * cells * 1.001
+    rng = np.random.default_rng(100 + cells)
+    side = int(round((per_cell * cells ** 3) ** (1.0 / 3.0)))
+    lattice = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    p = (lattice + 0.5 + 0.6 * (rng.uniform(size=lattice.shape) - 0.5)) * (L / side)
+    p = np.concatenate([p, rng.uniform(0.05, 2.9, (150, 3))])
+    gap = np.linalg.norm(p[-150:, None] - p[None], axis=2)
+    gap[np.arange(150), np.arange(len(p) - 150, len(p))] = 1.0
+    p = np.delete(p, len(p) - 150 + np.nonzero(gap.min(1) < 0.05)[0], axis=0)
+    n = len(p)
+    q = np.where(np.arange(n) % 2 == 0, 1.0, -1.0)
+    s = {"x": p[:, 0].copy(), "y": p[:, 1].copy(), "z": p[:, 2].copy(), "q": q, "L": float(L)}
+    fr_ref, _ = orc.realteil(s, rcut, alpha, cells=True)
+    solver = pkg.Solver(7, pkg.HostSystem.from_dict(s), pkg.parameters(16, 3, alpha, rcut),
+                        getattr(pkg, prec_name))
+    dev = {k: torch.tensor(s[k], dtype=torch.float64, device="cuda") for k in "xyzq"}
+    fr = torch.zeros(3 * n, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    solver.realteil_device(n, L, *[dev[k].data_ptr() for k in "xyzq"], rcut, alpha, fr.data_ptr(), None)
+    solver.synchronize()
+    err = rel_err(fr.cpu().numpy().reshape(3, n), fr_ref)
+    print("cells %d n %d %s rel err %.2e" % (cells, n, prec_name, err))
+    assert err < (1e-13 if prec_name == "FP64" else 1e-6)
+    solver.close()
