@@ -12,6 +12,7 @@
 #include <cmath>
 
 #include "fft_tiles.hpp"
+#include "fft_two.hpp"
 #include "k_internal.hpp"
 
 namespace p3m {
@@ -26,9 +27,11 @@ struct BSys {
     long tile0;         // first global tile index
     int p0, n;          // particle slots [p0, p0 + n) in the concatenated arrays
     fft::Radices rp;
+    fft::TwoPlan two;   // M as two factors (r1 = 0: per-radix passes by rp)
     void *buf[kNumBuf]; // mesh, spec0..2, F0..2 (element type of the batch)
     const double *G, *Dn, *selfb;
     const void *tw;     // twiddles exp(-2 pi i k / M), batch precision
+    const double2 *tw64; // the same in FP64 (two-factor passes)
     double prefac;      // back-interpolation prefactor (ad: includes nothing else)
     // real space
     int cell0, nc, reach, small;

@@ -39,6 +39,15 @@ __device__ __forceinline__ long line_start(const LineMap &m, long L) {
     return a * m.sa + (L - a * m.C);
 }
 
+// an element of a mesh to and from the FP64 registers of the passes
+template <typename V> __device__ __forceinline__ double2 widen(V v) { return make_double2(v.x, v.y); }
+template <typename V> __device__ __forceinline__ V narrow(double2 v) {
+    V r;
+    r.x = (decltype(V::x))v.x;
+    r.y = (decltype(V::x))v.y;
+    return r;
+}
+
 template <typename V> __device__ __forceinline__ V twid(const V *tw, int idx, int inv) {
     V w = tw[idx];
     if (inv)
@@ -151,8 +160,7 @@ __device__ __forceinline__ void butterfly(const V *__restrict__ src, V *__restri
 // m < 8 / R) and, after the last pass, its outputs in natural order.  A
 // pass computes in registers; between passes the outputs go through one LDS
 // line (positions of the autosort Stockham, as butterfly() writes them) and
-// back.  The radix sequence is make_radices', so the results equal the LDS
-// tile passes' bit for bit.
+// back.  The radix sequence is make_radices'.
 template <int N> struct P2Plan;
 template <> struct P2Plan<16> { static constexpr int np = 2, r[3] = {8, 2, 1}; };
 template <> struct P2Plan<32> { static constexpr int np = 2, r[3] = {8, 4, 1}; };
@@ -188,7 +196,7 @@ __device__ __forceinline__ void p2_pass(V v[8], int t, int Ns, const V *__restri
 
 // the outputs of a pass to their autosort positions in the LDS line
 template <int N, int R, typename V>
-__device__ __forceinline__ void p2_write(V *line, const V v[8], int t, int Ns) {
+__device__ __forceinline__ void p2_write(V *line, const double2 v[8], int t, int Ns) {
     constexpr int TPL = N / 8, B = 8 / R;
 #pragma unroll
     for (int m = 0; m < B; m++) {
@@ -196,22 +204,24 @@ __device__ __forceinline__ void p2_write(V *line, const V v[8], int t, int Ns) {
         const int base = (j / Ns) * Ns * R + (j & (Ns - 1));
 #pragma unroll
         for (int r = 0; r < R; r++)
-            line[base + r * Ns] = v[m + r * B];
+            line[base + r * Ns] = narrow<V>(v[m + r * B]);
     }
 }
 
 template <int N, typename V>
-__device__ __forceinline__ void p2_read(const V *line, V v[8], int t) {
+__device__ __forceinline__ void p2_read(const V *line, double2 v[8], int t) {
     constexpr int TPL = N / 8;
 #pragma unroll
     for (int s = 0; s < 8; s++)
-        v[s] = line[t + TPL * s];
+        v[s] = widen(line[t + TPL * s]);
 }
 
 // all passes of the plan on the registers of thread t; `line` is its line's
-// LDS row (N + 1 values), shared by the N / 8 threads of the line
+// LDS row (N + 1 values), shared by the N / 8 threads of the line.  The FP32
+// form, too, computes in FP64 registers (the FP32 rate; its rounded twiddles
+// would leave errors common to all points of a radix).
 template <int N, typename V>
-__device__ __forceinline__ void p2_fft(V v[8], V *line, int t, const V *__restrict__ tw, int inv) {
+__device__ __forceinline__ void p2_fft(double2 v[8], V *line, int t, const double2 *__restrict__ tw, int inv) {
     using Pl = P2Plan<N>;
     p2_pass<N, Pl::r[0]>(v, t, 1, tw, inv);
     p2_write<N, Pl::r[0]>(line, v, t, 1);

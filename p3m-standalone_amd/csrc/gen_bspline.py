@@ -119,8 +119,10 @@ def main(out=sys.stdout):
               " * Cardinal B-spline charge-assignment weights of order P (cao):\n"
               " *   w[j]  = W_j(x)  = B_P(x - j + (P-1)/2),  x in [-1/2, 1/2]\n"
               " *   dw[j] = W'_j(x),  d2w[j] = W''_j(x)\n"
-              " * evaluated as integer-coefficient Horner polynomials times 1/D_P,\n"
-              " * D_P = 2^(P-1) (P-1)!. */\n")
+              " * each times D_P = 2^(P-1) (P-1)!: integer-coefficient Horner polynomials.\n"
+              " * The caller multiplies the product of three by inv_den^3 (stencil_norm)\n"
+              " * in FP64, once per particle: a rounded FP32 1/D_P in every weight scales\n"
+              " * all of them by the same error. */\n")
     out.write("#pragma once\n\nnamespace p3m {\n\n")
     out.write("template <int P, typename T> struct Bspline;\n\n")
     for p in range(1, MAX_ORDER + 1):
@@ -131,7 +133,7 @@ def main(out=sys.stdout):
         if p == 1:
             out.write("    (void)x;\n")
         for j in range(p):
-            out.write("    o[%d] = (%s) * T(inv_den);\n" % (j, _horner(w[j])))
+            out.write("    o[%d] = (%s);\n" % (j, _horner(w[j])))
         out.write("  }\n")
         out.write("  __host__ __device__ static inline void dw(T x, T *o) {\n")
         if p <= 2:
@@ -140,7 +142,7 @@ def main(out=sys.stdout):
             if p == 1:
                 out.write("    o[%d] = T(0.0);\n" % j)
             else:
-                out.write("    o[%d] = (%s) * T(inv_den);\n" % (j, _horner(dw[j][:p - 1])))
+                out.write("    o[%d] = (%s);\n" % (j, _horner(dw[j][:p - 1])))
         out.write("  }\n")
         out.write("  __host__ __device__ static inline void d2w(T x, T *o) {\n")
         if p <= 3:
@@ -149,8 +151,11 @@ def main(out=sys.stdout):
             if p <= 2:
                 out.write("    o[%d] = T(0.0);\n" % j)
             else:
-                out.write("    o[%d] = (%s) * T(inv_den);\n" % (j, _horner(d2w[j][:p - 2])))
+                out.write("    o[%d] = (%s);\n" % (j, _horner(d2w[j][:p - 2])))
         out.write("  }\n};\n\n")
+    out.write("// 1/D_P^3, the norm of a product of three weights\n"
+              "template <int P> constexpr double stencil_norm =\n"
+              "    Bspline<P, double>::inv_den * Bspline<P, double>::inv_den * Bspline<P, double>::inv_den;\n\n")
     out.write("}  // namespace p3m\n")
 
 

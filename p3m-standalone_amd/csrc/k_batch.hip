@@ -218,6 +218,7 @@ extern "C" int p3mk_batch_create(p3mk_batch **out, int r2c, int interlaced, int 
         S.p0 = (int)ntot;
         S.n = I.n;
         S.rp = rp;
+        S.two = fft::make_two(I.M);
         S.prefac = I.prefac;
         S.rcut = I.rcut;
         S.alpha = I.alpha;
@@ -315,6 +316,7 @@ extern "C" int p3mk_batch_create(p3mk_batch **out, int r2c, int interlaced, int 
             p3mk_batch_destroy(b);
             return p3mk_fail(P3MK_EDEVICE, "twiddle upload", (int)e);
         }
+        S.tw64 = (const double2 *)tw;
         S.tw = fp32 ? (const void *)(tw + align256(sizeof(double2) * S.M)) : (const void *)tw;
     }
     // per-particle system ids and prefix arrays

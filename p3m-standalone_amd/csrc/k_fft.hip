@@ -1,10 +1,10 @@
 // Mixed-radix Stockham FFT for the P3M meshes (radices 2,3,4,5,7,8,11,13).
 //
 // A 3D transform is three passes of batched 1D transforms, one per axis.
-// Each workgroup loads a tile of `lt` lines into LDS (coalesced: along the
-// line for the contiguous z axis, across neighbouring lines for the strided
-// y and x axes), runs all radix passes in LDS (autosort Stockham, two
-// ping-pong buffers) and writes the tile back.  The x pass of the forward
+// Lengths 16 ... 256 of powers of two hold their lines in registers (p2_fft,
+// below), lengths with two factors up to 16 take two register stages
+// (fft_two.hpp); the rest (162, 200, 220, above 256, ...) one pass per radix
+// through two LDS buffers (fft_tiles.hpp).  The x pass of the forward
 // transform is fused with the multiplication by the influence function (and,
 // for ik, the gradient i 2pi/L Dn) and with the x pass of the backward
 // transform, so the spectrum never makes an extra round trip through HBM.
@@ -19,6 +19,7 @@
 #include "batch_desc.hpp"
 #include "device_common.hpp"
 #include "fft_tiles.hpp"
+#include "fft_two_launch.hpp"
 #include "k_internal.hpp"
 
 using namespace p3m;
@@ -41,7 +42,7 @@ k_fft_pass(c2_t<T> *data, LineMap m, Radices rp, const c2_t<T> *__restrict__ tw,
 // neighbouring lines.
 template <int N, typename T, bool CONTIG>
 __global__ void __launch_bounds__(kThreads)
-k_fft_p2(c2_t<T> *data, LineMap m, const c2_t<T> *__restrict__ tw, int inv) {
+k_fft_p2(c2_t<T> *data, LineMap m, const double2 *__restrict__ tw, int inv) {
     using V = c2_t<T>;
     constexpr int TPL = N / 8, LPW = kThreads / TPL, PITCH = N + 1;
     __shared__ V buf[LPW * PITCH];
@@ -51,32 +52,33 @@ k_fft_p2(c2_t<T> *data, LineMap m, const c2_t<T> *__restrict__ tw, int inv) {
     const long L = (long)blockIdx.x * LPW + l;
     const bool ok = L < m.nlines;
     const long base = ok ? line_start(m, L) : 0;
-    V v[8];
+    V in[8];
 #pragma unroll
     for (int s = 0; s < 8; s++) {
-        if (ok) {
-            v[s] = data[base + (long)(t + TPL * s) * m.es];
-        } else {
-            v[s].x = T(0);
-            v[s].y = T(0);
-        }
+        in[s].x = in[s].y = T(0);
+        if (ok)
+            in[s] = data[base + (long)(t + TPL * s) * m.es];
     }
+    double2 v[8];
+#pragma unroll
+    for (int s = 0; s < 8; s++)
+        v[s] = widen(in[s]);
     p2_fft<N>(v, buf + l * PITCH, t, tw, inv);
     if (ok) {
 #pragma unroll
         for (int s = 0; s < 8; s++)
-            data[base + (long)(t + TPL * s) * m.es] = v[s];
+            data[base + (long)(t + TPL * s) * m.es] = narrow<V>(v[s]);
     }
 }
 
 // The fused x pass (convolve_x_tile) for power-of-two meshes on registers:
-// forward along x, X <- G X (FP64 product rounded to T), then for nout == 1
+// forward along x, X <- G X, then for nout == 1
 // backward into out0, for nout == 3 backward of i (2 pi / L) Dn[n_d] X into
 // out_d.  Lines c = j W + k (strided by nl = M W), element e = n_x.
 template <int N, typename T>
 __global__ void __launch_bounds__(kThreads)
 k_convolve_p2(const c2_t<T> *in, c2_t<T> *out0, c2_t<T> *out1, c2_t<T> *out2, long nl, int W,
-              const c2_t<T> *__restrict__ tw, const double *__restrict__ G,
+              const double2 *__restrict__ tw, const double *__restrict__ G,
               const double *__restrict__ Dn, double twopi_L, int nout) {
     using V = c2_t<T>;
     constexpr int TPL = N / 8, LPW = kThreads / TPL, PITCH = N + 1;
@@ -86,50 +88,51 @@ k_convolve_p2(const c2_t<T> *in, c2_t<T> *out0, c2_t<T> *out1, c2_t<T> *out2, lo
     const long L = (long)blockIdx.x * LPW + l;
     const bool ok = L < nl;
     const int j = ok ? (int)(L / W) : 0, k = ok ? (int)(L - (long)j * W) : 0;
-    V v[8];
+    V x[8];
 #pragma unroll
     for (int s = 0; s < 8; s++) {
-        if (ok) {
-            v[s] = in[L + (long)(t + TPL * s) * nl];
-        } else {
-            v[s].x = T(0);
-            v[s].y = T(0);
-        }
+        x[s].x = x[s].y = T(0);
+        if (ok)
+            x[s] = in[L + (long)(t + TPL * s) * nl];
     }
+    double2 v[8];
+#pragma unroll
+    for (int s = 0; s < 8; s++)
+        v[s] = widen(x[s]);
     V *line = buf + l * PITCH;
     p2_fft<N>(v, line, t, tw, 0);
 #pragma unroll
     for (int s = 0; s < 8; s++) {
         const int e = t + TPL * s;
         const double g = ok ? G[((long)e * N + j) * N + k] : 0.0;
-        v[s].x = (T)((double)v[s].x * g);
-        v[s].y = (T)((double)v[s].y * g);
+        v[s].x *= g;
+        v[s].y *= g;
     }
     if (nout == 1) {
         p2_fft<N>(v, line, t, tw, 1);
         if (ok) {
 #pragma unroll
             for (int s = 0; s < 8; s++)
-                out0[L + (long)(t + TPL * s) * nl] = v[s];
+                out0[L + (long)(t + TPL * s) * nl] = narrow<V>(v[s]);
         }
         return;
     }
     V *outs[3] = {out0, out1, out2};
     for (int d = 0; d < 3; d++) {
-        V w[8];
+        double2 w[8];
 #pragma unroll
         for (int s = 0; s < 8; s++) {
             const int e = t + TPL * s;
             const int nd = (d == 0) ? e : ((d == 1) ? j : k);
             const double f = twopi_L * Dn[nd];
-            w[s].x = (T)(-f * (double)v[s].y);
-            w[s].y = (T)(f * (double)v[s].x);
+            w[s].x = -f * v[s].y;
+            w[s].y = f * v[s].x;
         }
         p2_fft<N>(w, line, t, tw, 1);
         if (ok) {
 #pragma unroll
             for (int s = 0; s < 8; s++)
-                outs[d][L + (long)(t + TPL * s) * nl] = w[s];
+                outs[d][L + (long)(t + TPL * s) * nl] = narrow<V>(w[s]);
         }
     }
 }
@@ -176,6 +179,7 @@ struct p3mk_fft {
     p3mk_geom g;
     int M, H;
     Radices rp;
+    TwoPlan two;
     double2 *tw64;
     float2 *tw32;
 };
@@ -204,6 +208,7 @@ extern "C" int p3mk_fft_create(p3mk_fft **out, const p3mk_geom *g) {
     f->M = g->M;
     f->H = g->M / 2 + 1;
     f->rp = rp;
+    f->two = make_two(g->M);
     f->tw64 = nullptr;
     f->tw32 = nullptr;
     const int n = g->M;
@@ -265,7 +270,7 @@ template <int N, typename T>
 int pass_p2(p3mk_fft *f, c2_t<T> *data, const LineMap &m, int inv, bool contig, p3mk_queue *q) {
     constexpr int LPW = kThreads / (N / 8);
     const long blocks = (m.nlines + LPW - 1) / LPW;
-    const c2_t<T> *tw = sizeof(T) == 8 ? (const c2_t<T> *)f->tw64 : (const c2_t<T> *)f->tw32;
+    const double2 *tw = f->tw64;
     if (contig)
         hipLaunchKernelGGL((k_fft_p2<N, T, true>), dim3((unsigned)blocks), dim3(kThreads), 0,
                            p3mk_stream(q), data, m, tw, inv);
@@ -285,10 +290,12 @@ int pass(p3mk_fft *f, c2_t<T> *data, const LineMap &m, int inv, bool contig, p3m
     case 256: return pass_p2<256, T>(f, data, m, inv, contig, q);
     default: break;
     }
+    const c2_t<T> *tw = sizeof(T) == 8 ? (const c2_t<T> *)f->tw64 : (const c2_t<T> *)f->tw32;
+    if (f->two.r1 > 0)
+        return two_pass<T>(f->two, data, m, f->tw64, inv, contig, p3mk_stream(q));
     const int lt = launch_lines<T>(m.n, 2, m.nlines);
     const size_t lds = 2 * (size_t)lt * (m.n + 1) * sizeof(c2_t<T>);
     const long blocks = (m.nlines + lt - 1) / lt;
-    const c2_t<T> *tw = sizeof(T) == 8 ? (const c2_t<T> *)f->tw64 : (const c2_t<T> *)f->tw32;
     hipLaunchKernelGGL(k_fft_pass<T>, dim3((unsigned)blocks), dim3(kThreads), lds, p3mk_stream(q),
                        data, m, f->rp, tw, inv, lt, contig ? 1 : 0);
     return p3mk_launch_check("fft pass");
@@ -306,11 +313,15 @@ template <typename T> int forward_zy(p3mk_fft *f, void *mesh, void *spec, p3mk_q
         return pass<T>(f, d, y, 0, false, q);
     }
     const long nl = (long)M * M;
-    const int lt = launch_lines<T>(M, 2, nl);
-    const size_t lds = 2 * (size_t)lt * (M + 1) * sizeof(V);
-    hipLaunchKernelGGL(k_fft_r2c_z<T>, dim3((unsigned)((nl + lt - 1) / lt)), dim3(kThreads), lds,
-                       p3mk_stream(q), (const T *)mesh, (V *)spec, nl, M, f->rp, tw, lt);
-    P3MK_TRY(p3mk_launch_check("fft r2c"));
+    if (f->two.r1 > 0) {
+        P3MK_TRY(two_r2c<T>(f->two, (const T *)mesh, (V *)spec, nl, f->tw64, p3mk_stream(q)));
+    } else {
+        const int lt = launch_lines<T>(M, 2, nl);
+        const size_t lds = 2 * (size_t)lt * (M + 1) * sizeof(V);
+        hipLaunchKernelGGL(k_fft_r2c_z<T>, dim3((unsigned)((nl + lt - 1) / lt)), dim3(kThreads), lds,
+                           p3mk_stream(q), (const T *)mesh, (V *)spec, nl, M, f->rp, tw, lt);
+        P3MK_TRY(p3mk_launch_check("fft r2c"));
+    }
     LineMap y = {M, H, H, (long)M * H, (long)M * H};
     return pass<T>(f, (V *)spec, y, 0, false, q);
 }
@@ -329,6 +340,8 @@ template <typename T> int backward_yz(p3mk_fft *f, void *spec, void *mesh, p3mk_
     LineMap y = {M, H, H, (long)M * H, (long)M * H};
     P3MK_TRY(pass<T>(f, (V *)spec, y, 1, false, q));
     const long nl = (long)M * M;
+    if (f->two.r1 > 0)
+        return two_c2r<T>(f->two, (const V *)spec, (T *)mesh, nl, f->tw64, p3mk_stream(q));
     const int lt = launch_lines<T>(M, 2, nl);
     const size_t lds = 2 * (size_t)lt * (M + 1) * sizeof(V);
     hipLaunchKernelGGL(k_fft_c2r_z<T>, dim3((unsigned)((nl + lt - 1) / lt)), dim3(kThreads), lds,
@@ -341,7 +354,7 @@ int convolve_p2(p3mk_fft *f, int nout, const double *G, const double *Dn, void *
                 void *const out[3], long nl, int W, p3mk_queue *q) {
     using V = c2_t<T>;
     constexpr int LPW = kThreads / (N / 8);
-    const c2_t<T> *tw = sizeof(T) == 8 ? (const V *)f->tw64 : (const V *)f->tw32;
+    const double2 *tw = f->tw64;
     V *o0 = (V *)out[0];
     V *o1 = nout == 3 ? (V *)out[1] : nullptr;
     V *o2 = nout == 3 ? (V *)out[2] : nullptr;
@@ -366,12 +379,15 @@ int convolve(p3mk_fft *f, int nout, const double *G, const double *Dn, void *spe
     case 256: return convolve_p2<256, T>(f, nout, G, Dn, spec, out, nl, W, q);
     default: break;
     }
+    const c2_t<T> *tw = sizeof(T) == 8 ? (const V *)f->tw64 : (const V *)f->tw32;
+    const double twopi_L = 2.0 * 3.14159265358979323846 / f->g.L;
+    if (f->two.r1 > 0)
+        return two_convolve<T>(f->two, (const V *)spec, (V *const *)out, nout, nl, W, f->tw64, G, Dn, twopi_L,
+                               p3mk_stream(q));
     LineMap x = {M, nl, nl, 0, nl};
     const int nbuf = (nout == 3) ? 3 : 2;
     const int lt = launch_lines<T>(M, nbuf, nl);
     const size_t lds = (size_t)nbuf * lt * (M + 1) * sizeof(V);
-    const c2_t<T> *tw = sizeof(T) == 8 ? (const V *)f->tw64 : (const V *)f->tw32;
-    const double twopi_L = 2.0 * 3.14159265358979323846 / f->g.L;
     V *o0 = (V *)out[0];
     V *o1 = nout == 3 ? (V *)out[1] : nullptr;
     V *o2 = nout == 3 ? (V *)out[2] : nullptr;
@@ -388,11 +404,14 @@ int divergence(p3mk_fft *f, const double *G, const double *Dn, void *const in[3]
     const int M = f->M;
     const int W = f->g.r2c ? f->H : M;
     const long nl = (long)M * W;
+    const c2_t<T> *tw = sizeof(T) == 8 ? (const V *)f->tw64 : (const V *)f->tw32;
+    const double twopi_L = 2.0 * 3.14159265358979323846 / f->g.L;
+    if (f->two.r1 > 0)
+        return two_divergence<T>(f->two, (const V *const *)in, (V *)out, nl, W, f->tw64, G, Dn, twopi_L,
+                                 p3mk_stream(q));
     LineMap x = {M, nl, nl, 0, nl};
     const int lt = launch_lines<T>(M, 3, nl);
     const size_t lds = (size_t)3 * lt * (M + 1) * sizeof(V);
-    const c2_t<T> *tw = sizeof(T) == 8 ? (const V *)f->tw64 : (const V *)f->tw32;
-    const double twopi_L = 2.0 * 3.14159265358979323846 / f->g.L;
     hipLaunchKernelGGL(k_divergence_x<T>, dim3((unsigned)((nl + lt - 1) / lt)), dim3(kThreads), lds,
                        p3mk_stream(q), (const V *)in[0], (const V *)in[1], (const V *)in[2],
                        (V *)out, x, W, f->rp, tw, G, Dn, twopi_L, lt);
@@ -402,89 +421,23 @@ int divergence(p3mk_fft *f, const double *G, const double *Dn, void *const in[3]
 }  // namespace
 
 // ---- batched passes over many systems ------------------------------------
-//
-// Block b belongs to the system s with blk[s] <= b < blk[s+1]; its tile
-// starts at line (b - blk[s]) * lt(M_s).  Buffers are the systems' own.
-
-namespace {
-
-template <typename T>
-__global__ void __launch_bounds__(kThreads)
-k_bfft_pass(const BSys *__restrict__ sys, const long *__restrict__ blk, int nsys, int axis, int slot,
-            int inv, int r2c) {
-    extern __shared__ unsigned char smem[];
-    using V = c2_t<T>;
-    const int s = prefix_slot(blk, nsys, (long)blockIdx.x);
-    const BSys &S = sys[s];
-    const int M = S.M, W = r2c ? M / 2 + 1 : M;
-    LineMap m;
-    if (axis == kPassZ)
-        m = {M, 1, 1, M, (long)M * M};
-    else
-        m = {M, W, W, (long)M * W, (long)M * W};
-    const int lt = batch_tile_lines<T>(M, 2);
-    fft_pass_tile<T>((V *)S.buf[slot], m, S.rp, (const V *)S.tw, inv, lt, axis == kPassZ ? 1 : 0,
-                     (long)(blockIdx.x - blk[s]) * lt, smem);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kThreads)
-k_bfft_r2c_z(const BSys *__restrict__ sys, const long *__restrict__ blk, int nsys, int in_slot,
-             int out_slot) {
-    extern __shared__ unsigned char smem[];
-    using V = c2_t<T>;
-    const int s = prefix_slot(blk, nsys, (long)blockIdx.x);
-    const BSys &S = sys[s];
-    const int M = S.M, lt = batch_tile_lines<T>(M, 2);
-    fft_r2c_z_tile<T>((const T *)S.buf[in_slot], (V *)S.buf[out_slot], (long)M * M, M, S.rp,
-                      (const V *)S.tw, lt, (long)(blockIdx.x - blk[s]) * lt, smem);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kThreads)
-k_bfft_c2r_z(const BSys *__restrict__ sys, const long *__restrict__ blk, int nsys, int in_slot,
-             int out_slot) {
-    extern __shared__ unsigned char smem[];
-    using V = c2_t<T>;
-    const int s = prefix_slot(blk, nsys, (long)blockIdx.x);
-    const BSys &S = sys[s];
-    const int M = S.M, lt = batch_tile_lines<T>(M, 2);
-    fft_c2r_z_tile<T>((const V *)S.buf[in_slot], (T *)S.buf[out_slot], (long)M * M, M, S.rp,
-                      (const V *)S.tw, lt, (long)(blockIdx.x - blk[s]) * lt, smem);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kThreads)
-k_bconvolve_x(const BSys *__restrict__ sys, const long *__restrict__ blk, int nsys, int nout,
-              int in_slot, int out_slot, int r2c) {
-    extern __shared__ unsigned char smem[];
-    using V = c2_t<T>;
-    const int s = prefix_slot(blk, nsys, (long)blockIdx.x);
-    const BSys &S = sys[s];
-    const int M = S.M, W = r2c ? M / 2 + 1 : M;
-    const long nl = (long)M * W;
-    const LineMap m = {M, nl, nl, 0, nl};
-    const int lt = batch_tile_lines<T>(M, nout == 3 ? 3 : 2);
-    V *o0 = (V *)S.buf[out_slot];
-    V *o1 = nout == 3 ? (V *)S.buf[out_slot + 1] : nullptr;
-    V *o2 = nout == 3 ? (V *)S.buf[out_slot + 2] : nullptr;
-    convolve_x_tile<T>((const V *)S.buf[in_slot], o0, o1, o2, m, W, S.rp, (const V *)S.tw, S.G, S.Dn,
-                       2.0 * 3.14159265358979323846 / S.L, nout, lt,
-                       (long)(blockIdx.x - blk[s]) * lt, smem);
-}
-
-}  // namespace
 
 namespace p3m {
 
 int bfft_lines_per_tile(const BForm &f, int M, int kind) {
+    const int lg = btwo_lg(make_two(M));
+    if (lg >= 0)
+        return 1 << lg;
     const int nbuf = (kind == kPassX && !f.ad) ? 3 : 2;
     return f.fp32 ? batch_tile_lines<float>(M, nbuf) : batch_tile_lines<double>(M, nbuf);
 }
 
 size_t bfft_lds_bytes(const BForm &f, int M, int kind) {
-    const int nbuf = (kind == kPassX && !f.ad) ? 3 : 2;
     const size_t v = f.fp32 ? sizeof(float2) : sizeof(double2);
+    const TwoPlan two = make_two(M);
+    if (two.r1 > 0)
+        return (size_t)two_lds_points(two, 1 << btwo_lg(two)) * v;
+    const int nbuf = (kind == kPassX && !f.ad) ? 3 : 2;
     return (size_t)nbuf * bfft_lines_per_tile(f, M, kind) * (M + 1) * v;
 }
 
@@ -492,53 +445,36 @@ int bfft_pass(const BForm &f, const BSys *sys, const long *blk, int nsys, long n
               int slot, int inv, p3mk_queue *q) {
     if (nblocks <= 0)
         return P3MK_OK;
-    if (f.fp32)
-        hipLaunchKernelGGL(k_bfft_pass<float>, dim3((unsigned)nblocks), dim3(kThreads), lds,
-                           p3mk_stream(q), sys, blk, nsys, axis, slot, inv, f.r2c);
-    else
-        hipLaunchKernelGGL(k_bfft_pass<double>, dim3((unsigned)nblocks), dim3(kThreads), lds,
-                           p3mk_stream(q), sys, blk, nsys, axis, slot, inv, f.r2c);
-    return p3mk_launch_check("batched fft pass");
+    hipStream_t st = p3mk_stream(q);
+    return f.fp32 ? btwo_pass<float>(sys, blk, nsys, nblocks, lds, axis, slot, inv, f.r2c, st)
+                  : btwo_pass<double>(sys, blk, nsys, nblocks, lds, axis, slot, inv, f.r2c, st);
 }
 
 int bfft_r2c_z(const BForm &f, const BSys *sys, const long *blk, int nsys, long nblocks, size_t lds, int in_slot,
                int out_slot, p3mk_queue *q) {
     if (nblocks <= 0)
         return P3MK_OK;
-    if (f.fp32)
-        hipLaunchKernelGGL(k_bfft_r2c_z<float>, dim3((unsigned)nblocks), dim3(kThreads), lds,
-                           p3mk_stream(q), sys, blk, nsys, in_slot, out_slot);
-    else
-        hipLaunchKernelGGL(k_bfft_r2c_z<double>, dim3((unsigned)nblocks), dim3(kThreads), lds,
-                           p3mk_stream(q), sys, blk, nsys, in_slot, out_slot);
-    return p3mk_launch_check("batched fft r2c");
+    hipStream_t st = p3mk_stream(q);
+    return f.fp32 ? btwo_r2c<float>(sys, blk, nsys, nblocks, lds, in_slot, out_slot, st)
+                  : btwo_r2c<double>(sys, blk, nsys, nblocks, lds, in_slot, out_slot, st);
 }
 
 int bfft_c2r_z(const BForm &f, const BSys *sys, const long *blk, int nsys, long nblocks, size_t lds, int in_slot,
                int out_slot, p3mk_queue *q) {
     if (nblocks <= 0)
         return P3MK_OK;
-    if (f.fp32)
-        hipLaunchKernelGGL(k_bfft_c2r_z<float>, dim3((unsigned)nblocks), dim3(kThreads), lds,
-                           p3mk_stream(q), sys, blk, nsys, in_slot, out_slot);
-    else
-        hipLaunchKernelGGL(k_bfft_c2r_z<double>, dim3((unsigned)nblocks), dim3(kThreads), lds,
-                           p3mk_stream(q), sys, blk, nsys, in_slot, out_slot);
-    return p3mk_launch_check("batched fft c2r");
+    hipStream_t st = p3mk_stream(q);
+    return f.fp32 ? btwo_c2r<float>(sys, blk, nsys, nblocks, lds, in_slot, out_slot, st)
+                  : btwo_c2r<double>(sys, blk, nsys, nblocks, lds, in_slot, out_slot, st);
 }
 
 int bfft_convolve_x(const BForm &f, const BSys *sys, const long *blk, int nsys, long nblocks, size_t lds,
                     int nout, int in_slot, int out_slot, p3mk_queue *q) {
     if (nblocks <= 0)
         return P3MK_OK;
-    if (f.fp32)
-        hipLaunchKernelGGL(k_bconvolve_x<float>, dim3((unsigned)nblocks), dim3(kThreads), lds,
-                           p3mk_stream(q), sys, blk, nsys, nout, in_slot, out_slot, f.r2c);
-    else
-        hipLaunchKernelGGL(k_bconvolve_x<double>, dim3((unsigned)nblocks), dim3(kThreads),
-                           lds, p3mk_stream(q), sys, blk, nsys, nout, in_slot, out_slot,
-                           f.r2c);
-    return p3mk_launch_check("batched convolve");
+    hipStream_t st = p3mk_stream(q);
+    return f.fp32 ? btwo_convolve<float>(sys, blk, nsys, nblocks, lds, nout, in_slot, out_slot, f.r2c, st)
+                  : btwo_convolve<double>(sys, blk, nsys, nblocks, lds, nout, in_slot, out_slot, f.r2c, st);
 }
 
 }  // namespace p3m

@@ -162,9 +162,10 @@ assign_rows_item(const double4 *__restrict__ sorted, int pb, int pe, long tl, in
             const double gq = gn;
             fetch(rd + 1, rn, gn);
             if (lane < nb) {
-                T qv = (T)r.w;
+                const double qn = r.w * stencil_norm<P>;
+                T qv = (T)qn;
                 if (MODE == kWeighted)
-                    qv = (T)(r.w * gq);
+                    qv = (T)(qn * gq);
                 int c0, c1, c2;
                 T w0[P], w1[P], w2[P];
                 axis_weights<P, T>(r.x, Hi, half, M, c0, w0);
@@ -257,10 +258,11 @@ assign_item(const double4 *__restrict__ sorted, int pb, int pe, long tl, int nt,
     __syncthreads();
     for (int p = pb + threadIdx.x; p < pe; p += blockDim.x) {
         const double4 r = sorted[p];
-        T qv = (T)r.w;
+        const double qn = r.w * stencil_norm<P>;
+        T qv = (T)qn;
         T g0 = T(0), g1 = T(0), g2 = T(0);
         if (MODE == kWeighted) {
-            qv = (T)(r.w * gv[perm[p]]);
+            qv = (T)(qn * gv[perm[p]]);
         } else if (MODE == kDipole) {
             const int i = perm[p];
             g0 = (T)gv[i];
@@ -375,7 +377,7 @@ interp_ik_item(const double4 *__restrict__ sorted, const int *__restrict__ perm,
     const int npts = R * R * R;
     const int tz = (int)(tl % nt), ty = (int)((tl / nt) % nt), tx = (int)(tl / ((long)nt * nt));
     const int t0x = tx * Tt, t0y = ty * Tt, t0z = tz * Tt;
-    const double sc = IL ? 0.5 * prefac : prefac;
+    const double sc = (IL ? 0.5 * prefac : prefac) * stencil_norm<P>;
     for (int d = 0; d < 3; d++) {
         const T *F = d == 0 ? F0 : (d == 1 ? F1 : F2);
         for (int k = threadIdx.x; k < npts; k += blockDim.x) {
@@ -502,7 +504,7 @@ interp_ad_item(const double4 *__restrict__ sorted, const int *__restrict__ perm,
                 F[2] += (double)w0[a] * (double)sz;
             }
         }
-        const double scale = (IL ? 0.5 * prefac : prefac) * (r.w * Leni);
+        const double scale = (IL ? 0.5 * prefac : prefac) * stencil_norm<P> * (r.w * Leni);
         const int i = perm[p];
         fk[i] -= scale * F[0];
         fk[stride + i] -= scale * F[1];

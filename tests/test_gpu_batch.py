@@ -208,3 +208,23 @@ def test_batch_time_pairs(pkg):
     after = run_batch(torch, batch, dev, graph=True)[0]
     assert rel_err(after, before) < 1e-6
     batch.close()
+
+
+@pytest.mark.parametrize("method", [0, 3, 6])
+def test_batch_mesh_splits(pkg, orc, method):
+    """One launch over meshes of different factor splits, a mesh without one
+    (162, one pass per radix) among them: each system against the oracle."""
+    import torch
+
+    systems, data = make_batch_systems(6, seed=77)
+    for s, M in zip(systems, (16, 26, 44, 36, 162, 90)):
+        s["M"], s["cao"] = M, 4
+    batch = pkg.Batch(method, systems, pkg.FP64)
+    dev = device_arrays(torch, data)
+    f, fk, fr = run_batch(torch, batch, dev)[:3]
+    for k, (s, d) in enumerate(zip(systems, data)):
+        sysd = dict(d, L=s["L"])
+        G = orc.influence(method, s["M"], s["cao"], s["L"], s["alpha"])
+        ref, _ = orc.kspace_force(method, sysd, s["M"], s["cao"], s["alpha"], G=G)
+        assert rel_err(per_system(fk, batch.offsets, k), ref) < 1e-12
+    batch.close()

@@ -442,6 +442,59 @@ def test_fft_r2c_zy_vs_numpy(pkg, M, fp32):
         rig.close()
 
 
+@pytest.mark.parametrize("fp32", [0, 1])
+@pytest.mark.parametrize("M", [4, 6, 10, 14, 26, 32, 50, 90, 104, 112, 120, 150, 156, 160, 162, 220, 256])
+def test_fft_factor_splits(pkg, M, fp32):
+    """Two-factor passes over every radix 2 ... 16 (4 = 2 x 2 to 160 = 10 x 16,
+    156 = 12 x 13), the meshes left to one pass per radix (162 and 220 have
+    no split with factors up to 16) and powers of two: z and y passes and
+    their inverses, c2c and r2c, against numpy in FP64.  FP64: 1e-14 as the
+    other transforms; FP32 storage with FP64 arithmetic rounds each value
+    twice per axis (stage and store) at 2^-24 / sqrt(3): 2 axes stay below
+    4e-7 with the meshes of one pass per radix in FP32."""
+    fn = _fft_api(pkg)
+    rdt, cdt = (np.float32, np.complex64) if fp32 else (np.float64, np.complex128)
+    rng = np.random.default_rng(300 + M)
+    tol = 4e-7 if fp32 else 1e-14
+    n0 = min(M, 32)  # planes checked (the passes do not mix x planes)
+    for r2c in (0, 1):
+        H = M // 2 + 1 if r2c else M
+        a = rng.standard_normal((M, M, M)).astype(rdt)
+        if not r2c:
+            a = (a + 1j * rng.standard_normal((M, M, M))).astype(cdt)
+        spec = np.empty((M, M, H), dtype=cdt)
+        rig = _FftRig(fn, M, r2c, fp32, [a.nbytes, spec.nbytes])
+        try:
+            out = 1 if r2c else 0
+            rig.put(0, a)
+            assert fn["p3mk_fft_forward_zy"](rig.plan, rig.bufs[0], rig.bufs[out], rig.q) == 0
+            rig.get(out, spec)
+            wide = a[:n0].astype(np.float64 if r2c else np.complex128)
+            ref = np.fft.fft(np.fft.rfft(wide, axis=2) if r2c else np.fft.fft(wide, axis=2), axis=1)
+            ef = rel_err(spec[:n0].astype(np.complex128), ref)
+            assert fn["p3mk_fft_backward_yz"](rig.plan, rig.bufs[out], rig.bufs[0], rig.q) == 0
+            back = rig.get(0, np.empty_like(a))
+            eb = rel_err(back[:n0].astype(wide.dtype), M * M * wide)
+            print("M %d fp32 %d r2c %d: forward %.2e, round trip %.2e" % (M, fp32, r2c, ef, eb))
+            assert ef < tol
+            assert eb < 2 * tol
+        finally:
+            rig.close()
+
+
+@pytest.mark.parametrize("method,M", [(0, 10), (0, 26), (3, 90), (1, 28), (6, 44), (6, 150), (6, 110)])
+def test_kspace_force_mesh_splits(pkg, orc, method, M):
+    """The fused x pass (and its gradient form) over two-factor meshes,
+    against the oracle at the FP64 tolerance."""
+    cao, L, alpha = 4, 10.0, 0.9
+    s = random_system(300, L, seed=M, charges="normal")
+    fk, _ = orc.kspace_force(method, s, M, cao, alpha)
+    solver = pkg.Solver(method, pkg.HostSystem.from_dict(s), pkg.parameters(M, cao, alpha))
+    got = solver.kspace_force().kspace()
+    assert rel_err(got, fk) < 1e-12
+    solver.close()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,fp32", [(64, 1), (128, 1), (128, 0)])
 def test_fft_c2c_zy_vs_numpy(pkg, M, fp32):
