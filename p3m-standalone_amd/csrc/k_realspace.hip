@@ -72,6 +72,15 @@ constexpr int kMfmaMinCell = 4;
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
 
+// Order of LDS accesses within the single wavefront of a workgroup: its LDS
+// instructions are performed in program order, so the compiler is all that
+// has to be held.  A workgroup barrier here would also wait for the device
+// atomics in flight (the reaction sums go to memory, microseconds away).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ double fold(double r, double L) {
     // into [0, L); identity for positions already inside the box
     if (r >= 0.0 && r < L)
@@ -442,7 +451,7 @@ __device__ __forceinline__ void load_erfcx_table(RsShared<FP32, VJP> &sh) {
         for (int k = threadIdx.x; k < kErfcxTab; k += blockDim.x)
             sh.tab[k] = (&p3m::kErfcxDoubleCoef[0][0])[k];
     }
-    __syncthreads();
+    wave_sync();
 }
 
 // Work-item claims of the persistent grids: a claim takes `per` consecutive
@@ -622,7 +631,7 @@ realspace_item(int home, int chunk, int cell0, const double4 *__restrict__ sorte
     }
     fill_shifts(sh, L);
     int count = 0; // wave-uniform queue length
-    __syncthreads();
+    wave_sync();
 
     float en32 = 0.0f; // FP32 form: twice this item's energy, per lane
 
@@ -659,7 +668,7 @@ realspace_item(int home, int chunk, int cell0, const double4 *__restrict__ sorte
             }
         }
         count = base;
-        __syncthreads();
+        wave_sync();
     };
 
     // the accepting lanes (ok) queue the pair (neighbour j, owner | shift)
@@ -679,7 +688,7 @@ realspace_item(int home, int chunk, int cell0, const double4 *__restrict__ sorte
     // evaluate full rounds of 64 queued pairs
     auto flush = [&]() {
         if (count >= kWave) {
-            __syncthreads();
+            wave_sync();
             do
                 drain(kWave);
             while (count >= kWave);
@@ -763,7 +772,7 @@ realspace_item(int home, int chunk, int cell0, const double4 *__restrict__ sorte
             }
         }
     }
-    __syncthreads();
+    wave_sync();
     if (count > 0)
         drain(count);
     if (FP32)
@@ -776,7 +785,7 @@ realspace_item(int home, int chunk, int cell0, const double4 *__restrict__ sorte
         if constexpr (VJP)
             atomicAdd(&dq[p], sh.facc[3][lane]);
     }
-    __syncthreads();
+    wave_sync();
 }
 
 // Persistent grid of the full shell (launched for boxes of fewer than
@@ -909,7 +918,8 @@ template <bool FP32> struct RsHalfShared {
     halfx4 win_a[kWave];         // (-2 n, 1) in FP16, n = n' / side, n' relative to the home cell centre
     float win_n2[kWave];         // |n'|^2; 1e30 in empty slots
     unsigned int win_js[kWave];  // sorted index | shift index << 27
-    int4 cells[kWave];           // the half shell's neighbour cells: range, first item, offsets
+    int4 cells[kWave];           // the half shell's neighbour cells: range, first item, offsets and shift
+    int before[kWave];           // particles of the listed cells before each
     // FP32 form: (n', q as FP32 bits), n' the fixed-point position of the
     // window particle's image relative to the home cell centre
     int4 win_q[FP32 ? kWave : 1];
@@ -980,7 +990,7 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
     int w = 0;            // filled window slots
     bool selfwin = false; // the window holds the item's own chunk
     float en32 = 0.0f;
-    __syncthreads();
+    wave_sync();
 
     // FP32 form: the pair difference d = h - n' is the exact integer
     // difference of the home particle h and the window particle's image n',
@@ -1164,7 +1174,7 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
     // candidate search of the window against the home particles, then all
     // queued pairs, then the reactions to fs; the window is emptied
     auto process_window = [&]() {
-        __syncthreads();
+        wave_sync();
         if (tiles) {
             // two issues at a time (G is even), so that their product chains overlap
             auto issues = [&](auto self_tag) {
@@ -1228,7 +1238,7 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
                 o = (o + 1 == nh) ? 0 : o + 1;
             }
         }
-        __syncthreads();
+        wave_sync();
         flush();
         if (count >= kWave)
             drain(kWave);
@@ -1247,7 +1257,7 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
         sh.win_n2[lane] = 1e30f;
         w = 0;
         selfwin = false;
-        __syncthreads();
+        wave_sync();
     };
 
     const int hitem = istart[cell0 + home] + chunk;
@@ -1260,7 +1270,7 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
     // the half shell's neighbour cells, one per lane (63 for reach 2, 14 for
     // reach 1; the own cell first): offsets, image flags, particle range and
     // first item read by one vector load each, cells that are empty or beyond
-    // rcut from the item's box dropped; the loop then walks the live ones
+    // rcut from the item's box dropped
     bool live = false;
     int cjb = 0, cje = 0, citem = 0;
     unsigned int cinfo = 0;
@@ -1277,112 +1287,146 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
         const float gz = gap(hlo.z, hhi.z, (float)((hz + c) * side), (float)((hz + c + 1) * side));
         if (gx * gx + gy * gy + gz * gz <= rskip2) {
             const int cell = cell0 + (cx * nc + cy) * nc + cz;
-            cjb = start[cell];
+            cjb = lane == 0 ? i0 : start[cell]; // the own cell from the own chunk on
             cje = start[cell + 1];
             citem = istart[cell];
             live = cjb < cje;
         }
-        cinfo = (unsigned)((a + 2) | (b + 2) << 3 | (c + 2) << 6 | (wx + 1) << 9 | (wy + 1) << 11 |
-                           (wz + 1) << 13);
+        cinfo = abc | shift_index(wx, wy, wz) << 9;
     }
-    // kept in LDS for the walk (read back uniformly), not in registers
-    sh.cells[lane] = make_int4(cjb, cje, citem, (int)cinfo);
     unsigned long long cells = __ballot(live);
     if (split_bits > 0) {
         // this unit's share of the live cells, dealt out in turn
         const int rank = (int)__builtin_amdgcn_mbcnt_hi((unsigned int)(cells >> 32),
                                                         __builtin_amdgcn_mbcnt_lo((unsigned int)cells, 0u));
-        cells = __ballot(live && (rank & ((1 << split_bits) - 1)) == part);
+        live = live && (rank & ((1 << split_bits) - 1)) == part;
+        cells = __ballot(live);
         if (cells == 0) {
-            __syncthreads();
+            wave_sync();
             return;
         }
     }
-    while (cells) {
-        const int k = __builtin_ctzll(cells);
-        cells &= cells - 1;
-        {
-            {
-                const int4 ck = sh.cells[k];
-                const int jb = __builtin_amdgcn_readfirstlane(ck.x);
-                const int je = __builtin_amdgcn_readfirstlane(ck.y);
-                const int item0 = __builtin_amdgcn_readfirstlane(ck.z);
-                const unsigned int info = (unsigned)__builtin_amdgcn_readfirstlane(ck.w);
-                const int a = (int)(info & 7u) - 2, b = (int)((info >> 3) & 7u) - 2,
-                          c = (int)((info >> 6) & 7u) - 2;
-                const int wx = (int)((info >> 9) & 3u) - 1, wy = (int)((info >> 11) & 3u) - 1,
-                          wz = (int)((info >> 13) & 3u) - 1;
-                const unsigned int sidx = shift_index(wx, wy, wz) << 27;
-                const float fsx = (float)(wx * L), fsy = (float)(wy * L), fsz = (float)(wz * L);
-                // FP32 form: the neighbour cell's centre relative to the home
-                // cell's is (a, b, c) sides, exactly 2^fb quanta each
-                // (the image shift w L is the whole-mesh part of it), so a
-                // window particle's fixed-point position in the home frame is
-                // its own-cell one plus that integer offset
-                const int fox = a * (1 << fb), foy = b * (1 << fb), foz = c * (1 << fb);
-                const double inv_quantum = ldexp(1.0, fb) / side;
-                const float q_scale = (float)(inv_quantum * inv_quantum);
-                // window rows: A' = (-2 (n + o), 1), o the cell centre relative to the home's
-                const float ox2 = (float)(2.0 * a * side), oy2 = (float)(2.0 * b * side),
-                            oz2 = (float)(2.0 * c * side);
-                const bool own = a == 0 && b == 0 && c == 0;
-                for (int cb = own ? i0 : jb; cb < je; cb += kWave) {
-                    const int cnt = min(kWave, je - cb);
-                    const int nitem = item0 + (cb - jb) / kWave;
-                    float4 nlo = bbox[2 * nitem], nhi = bbox[2 * nitem + 1];
-                    nlo.x += fsx; nlo.y += fsy; nlo.z += fsz;
-                    nhi.x += fsx; nhi.y += fsy; nhi.z += fsz;
-                    if (box_dist2(hlo, hhi, nlo, nhi) > rskip2)
-                        continue;
-                    if (own && cb == i0)
-                        selfwin = true; // the first chunk staged: w == 0 here
-                    // the chunk's particles within rcut of the item's box (all of
-                    // the own chunk), compacted into the window
-                    bool keep_l = false;
-                    halfx4 arow = {(_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f, (_Float16)1.0f};
-                    float n2 = 0.0f;
-                    int4 nq = make_int4(0, 0, 0, 0);
-                    if (lane < cnt) {
-                        const float4 v = sorted32[cb + lane];
-                        if constexpr (FP32) {
-                            const int4 q0 = sortedq[cb + lane];
-                            nq = make_int4(q0.x + fox, q0.y + foy, q0.z + foz,
-                                           __float_as_int(__int_as_float(q0.w) * q_scale));
-                        }
-                        const float ax = v.x - ox2, ay = v.y - oy2, az = v.z - oz2;
-                        const float nx = -0.5f * ax, ny = -0.5f * ay, nz = -0.5f * az;
-                        const float gxx = gap(hlo_r.x, hhi_r.x, nx, nx), gyy = gap(hlo_r.y, hhi_r.y, ny, ny),
-                                    gzz = gap(hlo_r.z, hhi_r.z, nz, nz);
-                        keep_l = gxx * gxx + gyy * gyy + gzz * gzz <= rskip2;
-                        // the matrix row in side units, rounded to FP16, and |n|^2
-                        // of the rounded row
-                        arow = halfx4{(_Float16)(ax * inv_side), (_Float16)(ay * inv_side),
-                                      (_Float16)(az * inv_side), (_Float16)1.0f};
-                        const float rx = -0.5f * (float)arow.x, ry = -0.5f * (float)arow.y,
-                                    rz = -0.5f * (float)arow.z;
-                        n2 = rx * rx + ry * ry + rz * rz;
-                    }
-                    unsigned long long mask = __ballot(keep_l);
-                    while (mask) {
-                        const int take = min(kWave - w, __popcll(mask));
-                        const int rank = (int)__builtin_amdgcn_mbcnt_hi(
-                            (unsigned int)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)mask, 0u));
-                        if (keep_l && rank < take) {
-                            sh.win_a[w + rank] = arow;
-                            sh.win_n2[w + rank] = n2;
-                            sh.win_js[w + rank] = (unsigned)(cb + lane) | sidx;
-                            if constexpr (FP32)
-                                sh.win_q[w + rank] = nq;
-                        }
-                        w += take;
-                        keep_l = keep_l && rank >= take;
-                        mask = __ballot(keep_l);
-                        if (w == kWave)
-                            process_window();
-                    }
-                }
+    // Cells of one chunk (at most 64 particles), and the own cell, are read
+    // as one list: 64 particles of it a step, whatever cells they are in, a
+    // lane finding its particle's cell in the cells' prefix sums.  (A step
+    // per cell leaves most lanes idle in a sparse system: 250,000 particles
+    // at 6 per cell took 875 us.)  Denser cells follow chunk by chunk, so that
+    // chunks beyond rcut are skipped by their boxes.
+    const bool listed = live && (lane == 0 || cje - cjb <= kWave);
+    int upto = listed ? cje - cjb : 0;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int v = __shfl_up(upto, off, kWave);
+        upto += lane >= off ? v : 0;
+    }
+    const int before = upto - (listed ? cje - cjb : 0);
+    const int total = __builtin_amdgcn_readlane(upto, kWave - 1);
+    sh.before[lane] = before;
+    sh.cells[lane] = make_int4(listed ? cjb - before : cjb, cje, citem, (int)cinfo);
+    selfwin = __builtin_amdgcn_readfirstlane((int)listed) != 0; // its own chunk is the list's first nh entries
+    // FP32 form: a neighbour cell's centre relative to the home cell's is
+    // (a, b, c) sides, exactly 2^fb quanta each (the image shift w L is the
+    // whole-mesh part of it), so a window particle's fixed-point position in
+    // the home frame is its own-cell one plus that integer offset
+    const float q_scale = (float)((ldexp(1.0, fb) / side) * (ldexp(1.0, fb) / side));
+    const float side2 = (float)(2.0 * side);
+    // the particles j (valid lanes) of cells with offsets and shift `info`
+    // that are within rcut of the item's box, compacted into the window
+    auto stage = [&](int j, bool valid, unsigned int info) {
+        bool keep_l = false;
+        halfx4 arow = {(_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f, (_Float16)1.0f};
+        float n2 = 0.0f;
+        int4 nq = make_int4(0, 0, 0, 0);
+        if (valid) {
+            const int a = (int)(info & 7u) - 2, b = (int)((info >> 3) & 7u) - 2, c = (int)((info >> 6) & 7u) - 2;
+            const float4 v = sorted32[j];
+            if constexpr (FP32) {
+                const int4 q0 = sortedq[j];
+                nq = make_int4(q0.x + (a << fb), q0.y + (b << fb), q0.z + (c << fb),
+                               __float_as_int(__int_as_float(q0.w) * q_scale));
             }
+            // window rows: A' = (-2 (n + o), 1), o the cell centre relative to the home's
+            const float ax = v.x - a * side2, ay = v.y - b * side2, az = v.z - c * side2;
+            const float nx = -0.5f * ax, ny = -0.5f * ay, nz = -0.5f * az;
+            const float gxx = gap(hlo_r.x, hhi_r.x, nx, nx), gyy = gap(hlo_r.y, hhi_r.y, ny, ny),
+                        gzz = gap(hlo_r.z, hhi_r.z, nz, nz);
+            keep_l = gxx * gxx + gyy * gyy + gzz * gzz <= rskip2;
+            // the matrix row in side units, rounded to FP16, and |n|^2
+            // of the rounded row
+            arow = halfx4{(_Float16)(ax * inv_side), (_Float16)(ay * inv_side), (_Float16)(az * inv_side),
+                          (_Float16)1.0f};
+            const float rx = -0.5f * (float)arow.x, ry = -0.5f * (float)arow.y, rz = -0.5f * (float)arow.z;
+            n2 = rx * rx + ry * ry + rz * rz;
         }
+        unsigned long long mask = __ballot(keep_l);
+        while (mask) {
+            const int take = min(kWave - w, __popcll(mask));
+            const int rank = (int)__builtin_amdgcn_mbcnt_hi(
+                (unsigned int)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)mask, 0u));
+            if (keep_l && rank < take) {
+                sh.win_a[w + rank] = arow;
+                sh.win_n2[w + rank] = n2;
+                sh.win_js[w + rank] = (unsigned)j | (info >> 9) << 27;
+                if constexpr (FP32)
+                    sh.win_q[w + rank] = nq;
+            }
+            w += take;
+            keep_l = keep_l && rank >= take;
+            mask = __ballot(keep_l);
+            if (w == kWave)
+                process_window();
+        }
+    };
+    wave_sync();
+    // one call of stage (its code holds a window's whole evaluation) for
+    // both kinds of cells
+    unsigned long long dense = __ballot(live && !listed);
+    int base = 0, cb = 0, ce = 0, citem0 = 0;
+    unsigned int dinfo = 0;
+    float fsx = 0.0f, fsy = 0.0f, fsz = 0.0f;
+    for (;;) {
+        int j;
+        bool valid;
+        unsigned int info;
+        if (base < total) {
+            const int e = base + lane;
+            int k = 0;
+#pragma unroll
+            for (int step = kWave / 2; step > 0; step >>= 1)
+                k += sh.before[k + step] <= e ? step : 0;
+            const int4 ck = sh.cells[k];
+            j = ck.x + e;
+            info = (unsigned)ck.w;
+            valid = e < total;
+            base += kWave;
+        } else {
+            if (cb >= ce) {
+                if (!dense)
+                    break;
+                const int k = __builtin_ctzll(dense);
+                dense &= dense - 1;
+                const int4 ck = sh.cells[k];
+                cb = __builtin_amdgcn_readfirstlane(ck.x);
+                ce = __builtin_amdgcn_readfirstlane(ck.y);
+                citem0 = __builtin_amdgcn_readfirstlane(ck.z);
+                dinfo = (unsigned)__builtin_amdgcn_readfirstlane(ck.w);
+                const unsigned int sidx = dinfo >> 9;
+                fsx = (float)(((int)(sidx / 9u) - 1) * L);
+                fsy = (float)(((int)((sidx / 3u) % 3u) - 1) * L);
+                fsz = (float)(((int)(sidx % 3u) - 1) * L);
+            }
+            float4 nlo = bbox[2 * citem0], nhi = bbox[2 * citem0 + 1];
+            nlo.x += fsx; nlo.y += fsy; nlo.z += fsz;
+            nhi.x += fsx; nhi.y += fsy; nhi.z += fsz;
+            j = cb + lane;
+            valid = j < ce;
+            info = dinfo;
+            citem0++;
+            cb += kWave;
+            if (box_dist2(hlo, hhi, nlo, nhi) > rskip2)
+                continue;
+        }
+        stage(j, valid, info);
     }
     if (w > 0)
         process_window();
@@ -1399,7 +1443,7 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
         atomicAdd(&fs[stride + i], f1);
         atomicAdd(&fs[2 * stride + i], f2);
     }
-    __syncthreads();
+    wave_sync();
 }
 
 // Persistent grid as k_realspace over the half shell; fs (3 n, sorted order)
@@ -1422,7 +1466,7 @@ k_realspace_half(const double4 *__restrict__ sorted, const float4 *__restrict__ 
         for (int k = threadIdx.x; k < kErfcxTab; k += blockDim.x)
             sh.tab[k] = (&p3m::kErfcxDoubleCoef[0][0])[k];
     }
-    __syncthreads();
+    wave_sync();
     const int sb = split_bits_of(total);
     Claims claims = first_claim(total << sb);
     for (;;) {
@@ -1769,7 +1813,7 @@ k_brealspace_half(const BSys *__restrict__ sys, const int *__restrict__ cell0s, 
         for (int k = threadIdx.x; k < kErfcxTab; k += blockDim.x)
             sh.tab[k] = (&p3m::kErfcxDoubleCoef[0][0])[k];
     }
-    __syncthreads();
+    wave_sync();
     const int sb = split_bits_of(total);
     Claims claims = first_claim(total << sb);
     for (;;) {
