@@ -101,28 +101,28 @@ inline int zero_count_cursor(int *count, int *cursor, size_t m, p3mk_queue *qu) 
     return p3mk_fill_zero(cursor, sizeof(int) * m, qu);
 }
 
-// Below this mean number of particles per cell of side rcut / 2, the cell
-// list takes cells of side rcut instead.  In a sparse system a cell of side
-// rcut / 2 holds one or two particles, and each work item's walk over its 63
-// neighbour cells then outweighs its pairs.  Measured with 200k uniform
-// particles at rcut 3, FP64 forces: 2 per cell take 1.24 ms with small cells
-// against 0.39 with large ones, 8 per cell 0.81 against 0.55, 16 per cell
-// 0.85 against 0.85 and 32 per cell 1.24 against 1.38.  The mean misjudges
-// clustered systems: a Gaussian of 1M particles in a box of side 100 has 8
-// per cell on average but about 90 in the typical particle's cell, and takes
-// 11.0 ms with small cells against 12.0 with large ones.
-constexpr double kSmallCellMinOccupancy = 6.0;
+// Below this number of particles in a typical particle's cell of side
+// rcut / 2 the cell list takes cells of side rcut instead: an item of a few
+// home particles spends more on its walk than on its pairs.  Measured, steps
+// with cells of side rcut against rcut / 2: 250,007 uniform particles FP64 at
+// 6.4 per cell 482 against 757 us, 100,000 mixed at 3.4 157 against 441 us;
+// at 16 per cell the two were equal and at 32 the small cells 10% faster.  A
+// Gaussian of a million particles, 8 per cell on average and 90 in the
+// typical particle's, takes 6.05 ms with small cells, 6.9 with large ones:
+// so the mean is weighted with the clustering seen by a typical particle
+// (1 = uniform), estimated where positions are at hand when the list is made.
+constexpr double kSmallCellMinOccupancy = 12.0;
 constexpr int kMaxCellsPerSide = 512;
 
 // Cell grid of a real-space cell list for n particles: nc cells per side of
 // side >= rcut / reach, with a margin so that rounding of x nc / L never puts
 // a pair inside the cutoff more than `reach` cells apart.  Boxes of fewer than
 // 2 reach + 1 cells per side are left to the nearest-image search.
-inline void cell_geometry(long n, double L, double rcut, int &nc, int &reach) {
+inline void cell_geometry(long n, double L, double rcut, double clustering, int &nc, int &reach) {
     const double margin = 1.0 - 1e-12;
     const int nc2 = (int)std::min<double>(kMaxCellsPerSide, std::floor(L * 2.0 / rcut * margin));
     const int nc1 = (int)std::min<double>(kMaxCellsPerSide, std::floor(L / rcut * margin));
-    const bool sparse = nc1 >= 3 && (double)n < kSmallCellMinOccupancy * nc2 * (double)nc2 * nc2;
+    const bool sparse = nc1 >= 3 && (double)n * clustering < kSmallCellMinOccupancy * nc2 * (double)nc2 * nc2;
     if (nc2 < 5 || sparse) {
         reach = 1;
         nc = nc1;

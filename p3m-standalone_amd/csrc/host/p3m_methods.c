@@ -71,6 +71,7 @@ typedef struct {
     p3mk_cells *cells;
     p3mk_psort *psort;
     double cells_L, cells_rc;
+    double clustering; /* of the positions given to Init */
     int have_G;
     int have_ks_events;
     int have_rs_events;
@@ -130,6 +131,35 @@ static int check_params(int id, const system_t *s, const parameters_t *p) {
     if (!(s->length > 0.0) || !isfinite(s->length))
         return p3mh_fail(P3M_HIP_EINVAL, "box length must be positive");
     return P3M_HIP_OK;
+}
+
+/* Density a typical particle sees over the mean density: pairs of sampled
+ * particles that share a cell of a 16^3 grid, over the number a uniform
+ * system has.  1 without positions.  Only the real-space cell size depends
+ * on it, never a result. */
+#define CLUSTER_GRID 16
+#define CLUSTER_SAMPLE 16384
+static double clustering_of(const system_t *s) {
+    int count[CLUSTER_GRID * CLUSTER_GRID * CLUSTER_GRID] = {0};
+    const int cells = CLUSTER_GRID * CLUSTER_GRID * CLUSTER_GRID;
+    int i, step, k;
+    double m = 0.0, pairs = 0.0, ratio;
+    if (s->p == NULL || s->p->x == NULL || s->p->y == NULL || s->p->z == NULL || s->nparticles < 2)
+        return 1.0;
+    step = (s->nparticles + CLUSTER_SAMPLE - 1) / CLUSTER_SAMPLE;
+    for (i = 0; i < s->nparticles; i += step) {
+        const double r[3] = {s->p->x[i] / s->length, s->p->y[i] / s->length, s->p->z[i] / s->length};
+        int cell = 0;
+        for (k = 0; k < 3; k++) {
+            const double u = r[k] - floor(r[k]);
+            const int c = u >= 0.0 && u < 1.0 ? (int)(u * CLUSTER_GRID) : 0; /* NaN: 0 */
+            cell = cell * CLUSTER_GRID + c;
+        }
+        pairs += 2.0 * count[cell]++;
+        m += 1.0;
+    }
+    ratio = pairs * cells / (m * (m - 1.0));
+    return ratio > 1.0 ? ratio : 1.0;
 }
 
 static int ctx_alloc(p3m_ctx *c) {
@@ -240,6 +270,7 @@ int p3m_hip_init(int method_id, system_t *s, parameters_t *p, int precision, dat
     c->geom.interlaced = is_interlaced(method_id);
     c->geom.fp32 = precision == P3M_HIP_MIXED;
     c->geom.L = s->length;
+    c->clustering = clustering_of(s);
     if (has_self_force(method_id)) {
         d->self_force_corrections = (double *)calloc(81, sizeof(double));
         if (d->self_force_corrections == NULL) {
@@ -507,7 +538,7 @@ static int ensure_cells(p3m_ctx *c, int n, double L, double rcut) {
         return P3M_HIP_OK;
     p3mk_cells_destroy(c->cells);
     c->cells = NULL;
-    TRYK(p3mk_cells_create(&c->cells, n, L, rcut), "cell list");
+    TRYK(p3mk_cells_create(&c->cells, n, L, rcut, c->clustering), "cell list");
     c->cells_L = L;
     c->cells_rc = rcut;
     return P3M_HIP_OK;
@@ -669,7 +700,7 @@ int p3m_hip_realteil(system_t *s, parameters_t *p, forces_t *f) {
         if (r_ != P3MK_OK)                  \
             rc = p3mh_kfail(r_, what);           \
     }
-    CHK(p3mk_cells_create(&cells, (int)n, s->length, p->rcut), "cell list");
+    CHK(p3mk_cells_create(&cells, (int)n, s->length, p->rcut, clustering_of(s)), "cell list");
     CHK(p3mk_alloc((void **)&pos, sizeof(double) * 4 * n), "positions");
     CHK(p3mk_alloc((void **)&fr, sizeof(double) * 3 * n), "forces");
     CHK(p3mk_alloc((void **)&en, sizeof(double)), "energy");
@@ -742,7 +773,7 @@ int p3m_hip_realteil_vjp(system_t *s, parameters_t *p, const vector_array_t *dF,
         if (r_ != P3MK_OK)                  \
             rc = p3mh_kfail(r_, what);      \
     }
-    CHK(p3mk_cells_create(&cells, (int)n, s->length, p->rcut), "cell list");
+    CHK(p3mk_cells_create(&cells, (int)n, s->length, p->rcut, clustering_of(s)), "cell list");
     CHK(p3mk_alloc((void **)&pos, sizeof(double) * 4 * n), "positions");
     CHK(p3mk_alloc((void **)&g, sizeof(double) * 3 * n), "cotangent");
     CHK(p3mk_alloc((void **)&out, sizeof(double) * 4 * n), "adjoint");

@@ -229,7 +229,7 @@ extern "C" int p3mk_batch_create(p3mk_batch **out, int r2c, int interlaced, int 
         mesh_off += align256(p3mk_mesh_bytes(&g64));
         int nc = 1, reach = 1;
         if (I.rcut > 0.0)
-            cell_geometry(I.n, I.L, I.rcut, nc, reach);
+            cell_geometry(I.n, I.L, I.rcut, 1.0, nc, reach);
         S.nc = nc;
         S.reach = reach;
         S.small = (2 * reach + 1 > nc) ? 1 : 0;

@@ -6,9 +6,9 @@
 // and 0.5 q_i q_j erfc(alpha r)/r to the energy.
 //
 // Layout: particles are folded into [0, L) and counting-sorted into cells of
-// side >= rcut/R (R = 2, or R = 1 when cells of side rcut/2 would hold fewer
-// than 6 particles on average or the box has fewer than 5 of them per side;
-// cell_geometry), and inside a cell by octant, so that 64 consecutive particles of a cell are spatially
+// side >= rcut/R (R = 2, or R = 1 when a typical particle's cell of side
+// rcut/2 would hold fewer than 12 particles or the box has fewer than 5 of
+// them per side; cell_geometry), and inside a cell by octant, so that 64 consecutive particles of a cell are spatially
 // compact.  A work item is (home cell, chunk of 64 home particles); a
 // persistent grid of single-wavefront workgroups claims items from an
 // atomic counter, so the dense cells of a clustered system are spread over
@@ -1587,7 +1587,8 @@ extern "C" void p3mk_cells_destroy(p3mk_cells *c) {
     delete c;
 }
 
-extern "C" int p3mk_cells_create(p3mk_cells **out, int n, double L, double rcut) {
+extern "C" int p3mk_cells_create(p3mk_cells **out, int n, double L, double rcut,
+                                  double clustering) {
     *out = nullptr;
     if (!(rcut > 0.0) || !(L > 0.0) || rcut > 0.5 * L)
         return p3mk_fail(P3MK_EINVAL, "real space needs 0 < rcut <= L/2", 0);
@@ -1598,7 +1599,7 @@ extern "C" int p3mk_cells_create(p3mk_cells **out, int n, double L, double rcut)
         return p3mk_fail(P3MK_ENOMEM, "cell list", 0);
     c->nmax = n;
     int nc, reach;
-    p3m::cell_geometry(n, L, rcut, nc, reach);
+    p3m::cell_geometry(n, L, rcut, clustering, nc, reach);
     c->nc = nc;
     c->reach = reach;
     c->ncell = (long)nc * nc * nc;

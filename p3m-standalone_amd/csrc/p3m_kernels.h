@@ -175,7 +175,9 @@ int p3mk_kspace_error_sum(int method, int M, int cao, double L, double alpha, in
 
 /* ---- real space ---------------------------------------------------------- */
 typedef struct p3mk_cells p3mk_cells; /* cell-list workspace */
-int p3mk_cells_create(p3mk_cells **c, int n, double L, double rcut);
+/* clustering: particles in a typical particle's neighbourhood over the mean
+ * (1 for a uniform system); decides the cell size only */
+int p3mk_cells_create(p3mk_cells **c, int n, double L, double rcut, double clustering);
 void p3mk_cells_destroy(p3mk_cells *c);
 /* fr += real-space force of every pair i != j with minimum-image distance
  * <= rcut; *energy (device, may be NULL) += energy.  fp32 selects the

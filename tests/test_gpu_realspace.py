@@ -265,3 +265,37 @@ def test_items_dealt_to_several_wavefronts(pkg, orc, cells, per_cell, prec_name)
     print("cells %d n %d %s rel err %.2e" % (cells, n, prec_name, err))
     assert err < (1e-13 if prec_name == "FP64" else 1e-6)
     solver.close()
+
+
+@pytest.mark.parametrize("prec_name", ["FP64", "MIXED"])
+@pytest.mark.parametrize("layout", ["dense", "clustered", "sparse"])
+def test_cell_size_follows_the_clustering(pkg, orc, layout, prec_name):
+    """Cells of side rcut / 2 for a dense uniform system (18 per such cell)
+    and for one that is sparse on average but clustered (its mean per cell is
+    below the sparse one's), cells of side rcut for the sparse one: all
+    against the oracle (FP64 1e-13; mixed 1e-6 with closest pairs above 0.05)."""
+    import torch
+
+    rcut, alpha = 3.0, 1.0
+    rng = np.random.default_rng(11)
+    L, side = {"dense": (12.0, 19), "clustered": (30.0, 14), "sparse": (18.0, 14)}[layout]
+    lattice = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    box = 6.0 if layout == "clustered" else L
+    p = (lattice + 0.5 + 0.6 * (rng.uniform(size=lattice.shape) - 0.5)) * (box / side)
+    if layout == "clustered":
+        p = np.mod(p - 2.0, L)  # across the box corner
+    n = len(p)
+    s = {"x": p[:, 0].copy(), "y": p[:, 1].copy(), "z": p[:, 2].copy(),
+         "q": np.where(np.arange(n) % 2 == 0, 1.0, -1.0), "L": L}
+    fr_ref, _ = orc.realteil(s, rcut, alpha, cells=True)
+    solver = pkg.Solver(0, pkg.HostSystem.from_dict(s), pkg.parameters(16, 3, alpha, rcut),
+                        getattr(pkg, prec_name))
+    dev = {k: torch.tensor(s[k], dtype=torch.float64, device="cuda") for k in "xyzq"}
+    fr = torch.zeros(3 * n, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    solver.realteil_device(n, L, *[dev[k].data_ptr() for k in "xyzq"], rcut, alpha, fr.data_ptr(), None)
+    solver.synchronize()
+    err = rel_err(fr.cpu().numpy().reshape(3, n), fr_ref)
+    print("%s %s rel err %.2e" % (layout, prec_name, err))
+    assert err < (1e-13 if prec_name == "FP64" else 1e-6)
+    solver.close()
