@@ -158,5 +158,9 @@ int brs_forces(const BForm &f, const BSys *sys, const int *psys, const int *cell
                long ncell, int ntot, const double *x, const double *y, const double *z,
                const double *q, CellArrays &a, int grid, bool any_small, bool any_cells,
                bool time_pairs, double *fr, double *energy, p3mk_queue *qu);
+// buffers brs_forces expects zero-filled (at most 2; returns their number);
+// with any_small also fr.  The cell-grid systems' forces are left in sorted
+// order (a.fsorted by a.key).
+int brs_ranges(CellArrays &a, int ntot, bool any_cells, p3mk_range r[2]);
 
 }  // namespace p3m

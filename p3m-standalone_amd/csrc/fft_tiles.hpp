@@ -34,6 +34,11 @@ struct LineMap {
     long nlines; // number of lines
 };
 
+// up to three meshes transformed by one launch (blockIdx.y picks one)
+template <typename P> struct Three {
+    P p[3];
+};
+
 __device__ __forceinline__ long line_start(const LineMap &m, long L) {
     const long a = L / m.C;
     return a * m.sa + (L - a * m.C);

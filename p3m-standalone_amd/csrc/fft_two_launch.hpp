@@ -14,12 +14,14 @@ namespace fft {
 
 // ---- one mesh (defined in k_fft_two_f32 / _f64) -----------------------------
 template <typename T>
-int two_pass(const TwoPlan &p, c2_t<T> *data, const LineMap &m, const double2 *tw, int inv, bool contig,
-             hipStream_t st);
+int two_pass(const TwoPlan &p, Three<c2_t<T> *> data, int k, const LineMap &m, const double2 *tw, int inv,
+             bool contig, hipStream_t st);
 template <typename T>
-int two_r2c(const TwoPlan &p, const T *in, c2_t<T> *out, long nlines, const double2 *tw, hipStream_t st);
+int two_r2c(const TwoPlan &p, Three<const T *> in, Three<c2_t<T> *> out, int k, long nlines, const double2 *tw,
+            hipStream_t st);
 template <typename T>
-int two_c2r(const TwoPlan &p, const c2_t<T> *in, T *out, long nlines, const double2 *tw, hipStream_t st);
+int two_c2r(const TwoPlan &p, Three<const c2_t<T> *> in, Three<T *> out, int k, long nlines, const double2 *tw,
+            hipStream_t st);
 template <typename T>
 int two_convolve(const TwoPlan &p, const c2_t<T> *in, c2_t<T> *const out[3], int nout, long nl, int W,
                  const double2 *tw, const double *G, const double *Dn, double twopi_L, hipStream_t st);
@@ -81,25 +83,25 @@ template <typename T> size_t two_lds(const TwoPlan &p, int lg) {
 
 template <typename T, bool CONTIG>
 __global__ void __launch_bounds__(kThreads)
-k_two_pass(c2_t<T> *data, LineMap m, TwoPlan p, const double2 *__restrict__ tw, int inv, int lg) {
+k_two_pass(Three<c2_t<T> *> data, LineMap m, TwoPlan p, const double2 *__restrict__ tw, int inv, int lg) {
     extern __shared__ __align__(16) unsigned char smem[];
-    two_pass_tile<T, CONTIG>(data, m, p, tw, inv, lg, (long)blockIdx.x << lg, smem);
+    two_pass_tile<T, CONTIG>(data.p[blockIdx.y], m, p, tw, inv, lg, (long)blockIdx.x << lg, smem);
 }
 
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
-k_two_r2c(const T *__restrict__ in, c2_t<T> *__restrict__ out, long nlines, TwoPlan p,
+k_two_r2c(Three<const T *> in, Three<c2_t<T> *> out, long nlines, TwoPlan p,
           const double2 *__restrict__ tw, int lg) {
     extern __shared__ __align__(16) unsigned char smem[];
-    two_r2c_tile<T>(in, out, nlines, p, tw, lg, (long)blockIdx.x << lg, smem);
+    two_r2c_tile<T>(in.p[blockIdx.y], out.p[blockIdx.y], nlines, p, tw, lg, (long)blockIdx.x << lg, smem);
 }
 
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
-k_two_c2r(const c2_t<T> *__restrict__ in, T *__restrict__ out, long nlines, TwoPlan p,
+k_two_c2r(Three<const c2_t<T> *> in, Three<T *> out, long nlines, TwoPlan p,
           const double2 *__restrict__ tw, int lg) {
     extern __shared__ __align__(16) unsigned char smem[];
-    two_c2r_tile<T>(in, out, nlines, p, tw, lg, (long)blockIdx.x << lg, smem);
+    two_c2r_tile<T>(in.p[blockIdx.y], out.p[blockIdx.y], nlines, p, tw, lg, (long)blockIdx.x << lg, smem);
 }
 
 template <int NOUT, typename T>
@@ -124,10 +126,10 @@ k_two_divergence(const c2_t<T> *in0, const c2_t<T> *in1, const c2_t<T> *in2, c2_
 }  // namespace
 
 template <typename T>
-int two_pass(const TwoPlan &p, c2_t<T> *data, const LineMap &m, const double2 *tw, int inv, bool contig,
-             hipStream_t st) {
-    const int lg = two_lg(m.nlines);
-    const dim3 grid(two_blocks(m.nlines, lg)), block(two_block(p, lg));
+int two_pass(const TwoPlan &p, Three<c2_t<T> *> data, int k, const LineMap &m, const double2 *tw, int inv,
+             bool contig, hipStream_t st) {
+    const int lg = two_lg(k * m.nlines);
+    const dim3 grid(two_blocks(m.nlines, lg), (unsigned)k), block(two_block(p, lg));
     if (contig)
         hipLaunchKernelGGL((k_two_pass<T, true>), grid, block, two_lds<T>(p, lg), st, data, m, p, tw, inv, lg);
     else
@@ -136,17 +138,19 @@ int two_pass(const TwoPlan &p, c2_t<T> *data, const LineMap &m, const double2 *t
 }
 
 template <typename T>
-int two_r2c(const TwoPlan &p, const T *in, c2_t<T> *out, long nlines, const double2 *tw, hipStream_t st) {
-    const int lg = two_lg(nlines);
-    hipLaunchKernelGGL(k_two_r2c<T>, dim3(two_blocks(nlines, lg)), dim3(two_block(p, lg)), two_lds<T>(p, lg), st,
+int two_r2c(const TwoPlan &p, Three<const T *> in, Three<c2_t<T> *> out, int k, long nlines, const double2 *tw,
+            hipStream_t st) {
+    const int lg = two_lg(k * nlines);
+    hipLaunchKernelGGL(k_two_r2c<T>, dim3(two_blocks(nlines, lg), (unsigned)k), dim3(two_block(p, lg)), two_lds<T>(p, lg), st,
                        in, out, nlines, p, tw, lg);
     return p3mk_launch_check("fft r2c");
 }
 
 template <typename T>
-int two_c2r(const TwoPlan &p, const c2_t<T> *in, T *out, long nlines, const double2 *tw, hipStream_t st) {
-    const int lg = two_lg(nlines);
-    hipLaunchKernelGGL(k_two_c2r<T>, dim3(two_blocks(nlines, lg)), dim3(two_block(p, lg)), two_lds<T>(p, lg), st,
+int two_c2r(const TwoPlan &p, Three<const c2_t<T> *> in, Three<T *> out, int k, long nlines, const double2 *tw,
+            hipStream_t st) {
+    const int lg = two_lg(k * nlines);
+    hipLaunchKernelGGL(k_two_c2r<T>, dim3(two_blocks(nlines, lg), (unsigned)k), dim3(two_block(p, lg)), two_lds<T>(p, lg), st,
                        in, out, nlines, p, tw, lg);
     return p3mk_launch_check("fft c2r");
 }
@@ -175,10 +179,12 @@ int two_divergence(const TwoPlan &p, const c2_t<T> *const in[3], c2_t<T> *out, l
 }
 
 #define P3M_INST(T)                                                                                        \
-    template int two_pass<T>(const TwoPlan &, c2_t<T> *, const LineMap &, const double2 *, int, bool,      \
+    template int two_pass<T>(const TwoPlan &, Three<c2_t<T> *>, int, const LineMap &, const double2 *, int, bool, \
                              hipStream_t);                                                                 \
-    template int two_r2c<T>(const TwoPlan &, const T *, c2_t<T> *, long, const double2 *, hipStream_t);    \
-    template int two_c2r<T>(const TwoPlan &, const c2_t<T> *, T *, long, const double2 *, hipStream_t);    \
+    template int two_r2c<T>(const TwoPlan &, Three<const T *>, Three<c2_t<T> *>, int, long, const double2 *, \
+                            hipStream_t);                                                                  \
+    template int two_c2r<T>(const TwoPlan &, Three<const c2_t<T> *>, Three<T *>, int, long, const double2 *, \
+                            hipStream_t);                                                                  \
     template int two_convolve<T>(const TwoPlan &, const c2_t<T> *, c2_t<T> *const[3], int, long, int,      \
                                  const double2 *, const double *, const double *, double, hipStream_t);    \
     template int two_divergence<T>(const TwoPlan &, const c2_t<T> *const[3], c2_t<T> *, long, int,         \

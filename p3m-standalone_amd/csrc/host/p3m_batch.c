@@ -187,21 +187,11 @@ int p3m_hip_batch_kspace_force_device(p3m_hip_batch *b, const double *x, const d
 static int batch_forces_enqueue(p3m_hip_batch *b, const double *x, const double *y, const double *z,
                                 const double *q, double *f, double *fk, double *fr,
                                 double *energy) {
-    const size_t n3 = 3 * (size_t)b->ntot;
     int s, any_rs = 0;
-    /* common.c:274-278 */
-    TRYK(p3mk_fill_zero(f, sizeof(double) * n3, b->q), "zero");
-    TRYK(p3mk_fill_zero(fk, sizeof(double) * n3, b->q), "zero");
-    TRYK(p3mk_fill_zero(fr, sizeof(double) * n3, b->q), "zero");
-    if (energy != NULL)
-        TRYK(p3mk_fill_zero(energy, sizeof(double) * (size_t)b->nsys, b->q), "zero");
     for (s = 0; s < b->nsys; s++)
         any_rs |= b->sys[s].rcut > 0.0;
-    if (any_rs)
-        TRYK(p3mk_batch_realspace(b->kb, x, y, z, q, fr, energy, b->q), "batched real space");
-    TRYK(p3mk_batch_kspace(b->kb, x, y, z, q, fk, f, b->q), "batched k-space force");
-    /* common.c:315-319 */
-    TRYK(p3mk_sum_parts(n3, fk, fr, f, b->q), "sum");
+    /* common.c:274-319 */
+    TRYK(p3mk_batch_forces(b->kb, any_rs, x, y, z, q, f, fk, fr, energy, b->q), "batched forces");
     return P3M_HIP_OK;
 }
 

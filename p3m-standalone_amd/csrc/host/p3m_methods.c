@@ -318,15 +318,19 @@ int p3m_hip_set_precision(data_t *d, int precision) {
 
 /* Assignment, forward FFT, influence-function multiply (ik: and gradient),
  * backward FFT: leaves the field meshes c->F[0..2] (ik) or the potential
- * mesh c->mesh (ad).  Records events 1 and 2. */
+ * mesh c->mesh (ad).  Records events 1 and 2.  filled: the ranges of
+ * p3mk_assign_ranges are zero already. */
 static int field_enqueue(p3m_ctx *c, int n, const double *x, const double *y, const double *z,
-                         const double *q) {
+                         const double *q, int filled) {
     p3mk_fft *fft = ctx_fft(c);
     const p3mk_geom *g = &c->geom;
     void *spec = is_r2c(c->method) ? c->spec[0] : c->mesh;
     void *outs[3];
     int k;
-    TRYK(p3mk_assign(g, n, x, y, z, q, c->psort, c->mesh, c->q), "charge assignment");
+    if (filled)
+        TRYK(p3mk_assign_filled(g, n, x, y, z, q, c->psort, c->mesh, c->q), "charge assignment");
+    else
+        TRYK(p3mk_assign(g, n, x, y, z, q, c->psort, c->mesh, c->q), "charge assignment");
     TRYK(p3mk_record(c->q, 1), "event");
     TRYK(p3mk_fft_forward_zy(fft, c->mesh, spec, c->q), "forward FFT");
     if (!is_ad(c->method)) {
@@ -335,8 +339,7 @@ static int field_enqueue(p3m_ctx *c, int n, const double *x, const double *y, co
         for (k = 0; k < 3; k++)
             outs[k] = is_r2c(c->method) ? c->spec[k] : c->F[k];
         TRYK(p3mk_convolve(fft, 3, c->G, c->Dn, spec, outs, c->q), "convolution");
-        for (k = 0; k < 3; k++)
-            TRYK(p3mk_fft_backward_yz(fft, outs[k], c->F[k], c->q), "backward FFT");
+        TRYK(p3mk_fft_backward_yz_many(fft, 3, outs, c->F, c->q), "backward FFT");
     } else {
         /* ad: phi = FFT^-1[G Q^] (p3m-ad.c:182-196, p3m-ad-i.c:176-190,
          * p3m-ad-real.c:90-104) */
@@ -357,10 +360,10 @@ static double interp_prefactor(const p3m_ctx *c) {
 }
 
 static int kspace_enqueue(p3m_ctx *c, int n, const double *x, const double *y, const double *z,
-                          const double *q, double *fk, double *f) {
+                          const double *q, int filled, double *fk, double *f) {
     const p3mk_geom *g = &c->geom;
     TRYK(p3mk_record(c->q, 0), "event");
-    TRY(field_enqueue(c, n, x, y, z, q));
+    TRY(field_enqueue(c, n, x, y, z, q, filled));
     if (!is_ad(c->method)) {
         TRYK(p3mk_interp_ik(g, n, c->psort, c->F, interp_prefactor(c), fk, c->q),
              "back-interpolation");
@@ -397,12 +400,7 @@ static int collect_stage_times(p3m_ctx *c) {
     return P3M_HIP_OK;
 }
 
-int p3m_hip_kspace_force_device(data_t *d, int n, double length, const double *x,
-                                const double *y, const double *z, const double *q, double *fk,
-                                double *f) {
-    p3m_ctx *c = ctx_of(d);
-    if (c == NULL)
-        return p3mh_fail(P3M_HIP_EINVAL, "data_t was not made by p3m_hip_init");
+static int check_kspace(const p3m_ctx *c, int n, double length, const double *f) {
     if (n != c->n)
         return p3mh_fail(P3M_HIP_EINVAL, "particle count %d differs from Init's %d", n, c->n);
     if (length != c->geom.L)
@@ -411,7 +409,17 @@ int p3m_hip_kspace_force_device(data_t *d, int n, double length, const double *x
         return p3mh_fail(P3M_HIP_EINVAL, "influence function not computed");
     if (has_self_force(c->method) && f == NULL)
         return p3mh_fail(P3M_HIP_EINVAL, "method %d needs the total-force array f", c->method);
-    return kspace_enqueue(c, n, x, y, z, q, fk, f);
+    return P3M_HIP_OK;
+}
+
+int p3m_hip_kspace_force_device(data_t *d, int n, double length, const double *x,
+                                const double *y, const double *z, const double *q, double *fk,
+                                double *f) {
+    p3m_ctx *c = ctx_of(d);
+    if (c == NULL)
+        return p3mh_fail(P3M_HIP_EINVAL, "data_t was not made by p3m_hip_init");
+    TRY(check_kspace(c, n, length, f));
+    return kspace_enqueue(c, n, x, y, z, q, 0, fk, f);
 }
 
 int p3m_hip_synchronize(data_t *d) {
@@ -466,10 +474,11 @@ int p3m_hip_kspace_force(system_t *s, parameters_t *p, data_t *d, forces_t *f) {
     if (n == 0)
         return P3M_HIP_OK;
     TRY(upload_positions(c, s));
-    TRYK(p3mk_fill_zero(c->force, sizeof(double) * 6 * n, c->q), "zero");
-    TRY(kspace_enqueue(c, (int)n, c->pos, c->pos + n, c->pos + 2 * n, c->pos + 3 * n, c->force,
+    TRYK(p3mk_fill_zero(c->force, sizeof(double) * (has_self_force(c->method) ? 6 : 3) * n, c->q), "zero");
+    TRY(kspace_enqueue(c, (int)n, c->pos, c->pos + n, c->pos + 2 * n, c->pos + 3 * n, 0, c->force,
                        c->force + 3 * n));
-    TRYK(p3mk_copy_d2h(c->hforce, c->force, sizeof(double) * 6 * n, c->q), "download");
+    TRYK(p3mk_copy_d2h(c->hforce, c->force, sizeof(double) * (has_self_force(c->method) ? 6 : 3) * n, c->q),
+         "download");
     TRYK(p3mk_queue_sync(c->q), "sync");
     TRY(collect_stage_times(c));
     for (dim = 0; dim < 3; dim++) {
@@ -544,23 +553,73 @@ static int ensure_cells(p3m_ctx *c, int n, double L, double rcut) {
     return P3M_HIP_OK;
 }
 
+static int prepare_realspace(p3m_ctx *c, int n, double length, double rcut) {
+    if (n > c->n)
+        return p3mh_fail(P3M_HIP_EINVAL, "more particles than Init's %d", c->n);
+    if (!(rcut > 0.0) || rcut > 0.5 * length)
+        return p3mh_fail(P3M_HIP_EINVAL, "real space needs 0 < rcut <= L/2");
+    return ensure_cells(c, c->n, length, rcut);
+}
+
 int p3m_hip_realteil_device(data_t *d, int n, double length, const double *x, const double *y,
                             const double *z, const double *q, double rcut, double alpha,
                             double *fr, double *energy) {
     p3m_ctx *c = ctx_of(d);
     if (c == NULL)
         return p3mh_fail(P3M_HIP_EINVAL, "data_t was not made by p3m_hip_init");
-    if (n > c->n)
-        return p3mh_fail(P3M_HIP_EINVAL, "more particles than Init's %d", c->n);
-    if (!(rcut > 0.0) || rcut > 0.5 * length)
-        return p3mh_fail(P3M_HIP_EINVAL, "real space needs 0 < rcut <= L/2");
-    TRY(ensure_cells(c, c->n, length, rcut));
+    TRY(prepare_realspace(c, n, length, rcut));
     TRYK(p3mk_record(c->q, 4), "event");
     TRYK(p3mk_realspace(c->cells, n, length, x, y, z, q, rcut, alpha, c->geom.fp32, fr, energy,
                         c->q),
          "real space");
     TRYK(p3mk_record(c->q, 5), "event");
     c->have_rs_events = 1;
+    return P3M_HIP_OK;
+}
+
+/* Calculate_forces (common.c:268-327) of device arrays, checked and with the
+ * cell list made: every buffer that starts from zero is cleared by one
+ * launch, and the last launch brings the real-space forces to the caller's
+ * order and sums, writing fr and (without a self force) f. */
+static int forces_enqueue(p3m_ctx *c, int n, double length, const double *x, const double *y,
+                          const double *z, const double *q, double rcut, double alpha, double *f,
+                          double *fk, double *fr, double *energy) {
+    p3mk_range r[P3MK_MAX_RANGES];
+    const int *pos = NULL;
+    const double *fs = NULL;
+    const size_t n3 = sizeof(double) * 3 * (size_t)n;
+    int k = 0, add_fr = 0;
+    r[k].p = fk;
+    r[k++].bytes = n3;
+    if (has_self_force(c->method)) {
+        r[k].p = f;
+        r[k++].bytes = n3;
+    }
+    if (energy != NULL) {
+        r[k].p = energy;
+        r[k++].bytes = sizeof(double);
+    }
+    if (rcut != 0.0) { /* common.c:290-294 */
+        k += p3mk_realspace_ranges(c->cells, n, r + k);
+        if (!p3mk_realspace_sorted(c->cells)) {
+            add_fr = 1;
+            r[k].p = fr;
+            r[k++].bytes = n3;
+        }
+    }
+    k += p3mk_assign_ranges(&c->geom, c->psort, c->mesh, r + k);
+    TRYK(p3mk_fill_zero_many(k, r, c->q), "zero");
+    if (rcut != 0.0) {
+        TRYK(p3mk_record(c->q, 4), "event");
+        TRYK(p3mk_realspace_filled(c->cells, n, length, x, y, z, q, rcut, alpha, c->geom.fp32, fr, energy,
+                                   &pos, &fs, c->q),
+             "real space");
+        TRYK(p3mk_record(c->q, 5), "event");
+        c->have_rs_events = 1;
+    }
+    TRY(kspace_enqueue(c, n, x, y, z, q, 1, fk, f));
+    /* common.c:315-319: f += f_k + f_r */
+    TRYK(p3mk_finish_forces(n, pos, fs, add_fr, has_self_force(c->method), fk, fr, f, c->q), "sum");
     return P3M_HIP_OK;
 }
 
@@ -575,17 +634,10 @@ int p3m_hip_calculate_forces_device(data_t *d, int n, double length, const doubl
         return p3mh_fail(P3M_HIP_EINVAL, "force arrays must not be NULL");
     if (n != c->n)
         return p3mh_fail(P3M_HIP_EINVAL, "particle count %d differs from Init's %d", n, c->n);
-    /* common.c:274-278 */
-    TRYK(p3mk_fill_zero(f, sizeof(double) * 3 * (size_t)n, c->q), "zero");
-    TRYK(p3mk_fill_zero(fk, sizeof(double) * 3 * (size_t)n, c->q), "zero");
-    TRYK(p3mk_fill_zero(fr, sizeof(double) * 3 * (size_t)n, c->q), "zero");
-    if (energy != NULL)
-        TRYK(p3mk_fill_zero(energy, sizeof(double), c->q), "zero");
-    if (rcut != 0.0) /* common.c:290-294 */
-        TRY(p3m_hip_realteil_device(d, n, length, x, y, z, q, rcut, alpha, fr, energy));
-    TRY(p3m_hip_kspace_force_device(d, n, length, x, y, z, q, fk, f));
-    /* common.c:315-319: f += f_k + f_r */
-    TRYK(p3mk_sum_parts(3 * (size_t)n, fk, fr, f, c->q), "sum");
+    if (rcut != 0.0)
+        TRY(prepare_realspace(c, n, length, rcut));
+    TRY(check_kspace(c, n, length, f));
+    TRY(forces_enqueue(c, n, length, x, y, z, q, rcut, alpha, f, fk, fr, energy));
     if (c->ring_rs != NULL) {
         int k = p3mk_ring_filled(c->q);
         if (k < c->ring_sets)
@@ -834,13 +886,10 @@ int p3m_hip_calculate_forces(const method_t *m, system_t *s, parameters_t *p, da
     if (s->length != c->geom.L)
         return p3mh_fail(P3M_HIP_EINVAL, "box length differs from the influence function's");
     TRY(upload_positions(c, s));
-    TRYK(p3mk_fill_zero(c->force, sizeof(double) * 9 * n, c->q), "zero");
-    TRYK(p3mk_fill_zero(c->energy, sizeof(double), c->q), "zero");
     if (p->rcut != 0.0) /* common.c:275-279 */
-        TRY(p3m_hip_realteil_device(d, (int)n, s->length, c->pos, c->pos + n, c->pos + 2 * n,
-                                    c->pos + 3 * n, p->rcut, p->alpha, c->force + 6 * n, c->energy));
-    TRY(kspace_enqueue(c, (int)n, c->pos, c->pos + n, c->pos + 2 * n, c->pos + 3 * n, c->force,
-                       c->force + 3 * n));
+        TRY(prepare_realspace(c, (int)n, s->length, p->rcut));
+    TRY(forces_enqueue(c, (int)n, s->length, c->pos, c->pos + n, c->pos + 2 * n, c->pos + 3 * n, p->rcut,
+                       p->alpha, c->force + 3 * n, c->force, c->force + 6 * n, c->energy));
     TRYK(p3mk_copy_d2h(c->hforce, c->force, sizeof(double) * 9 * n, c->q), "download");
     TRYK(p3mk_copy_d2h(&energy, c->energy, sizeof(double), c->q), "download");
     TRYK(p3mk_queue_sync(c->q), "sync");
@@ -851,7 +900,7 @@ int p3m_hip_calculate_forces(const method_t *m, system_t *s, parameters_t *p, da
         for (i = 0; i < n; i++) {
             fk[i] = hk[i];
             fr[i] = hr[i];
-            ft[i] = hs[i] + (fk[i] + fr[i]); /* common.c:315-319 */
+            ft[i] = hs[i];
         }
     }
     s->energy += energy;
@@ -1021,15 +1070,15 @@ int p3m_hip_kspace_force_vjp_device(data_t *d, int n, double length, const doubl
     fft = ctx_fft(c);
     g = &c->geom;
     TRYK(p3mk_record(c->q, 0), "event");
-    TRY(field_enqueue(c, n, x, y, z, q));
+    TRY(field_enqueue(c, n, x, y, z, q, 0));
     if (!is_ad(c->method)) {
         /* psi_d = sum_i q_i g_{i,d} W_i; lambda = sum_d K_d^T psi_d */
         for (k = 0; k < 3; k++) {
             in[k] = is_r2c(c->method) ? c->spec[k] : c->adj[k];
             TRYK(p3mk_assign_weighted(g, n, c->psort, 1, gF + (size_t)k * n, c->adj[k], c->q),
                  "cotangent assignment");
-            TRYK(p3mk_fft_forward_zy(fft, c->adj[k], in[k], c->q), "forward FFT");
         }
+        TRYK(p3mk_fft_forward_zy_many(fft, 3, c->adj, in, c->q), "forward FFT");
         TRYK(p3mk_divergence(fft, c->G, c->Dn, in, in[0], c->q), "adjoint multiply");
         TRYK(p3mk_fft_backward_yz(fft, in[0], c->adj[0], c->q), "backward FFT");
         TRYK(p3mk_adjoint_gather(g, 0, n, c->psort, q, gF, c->F, c->adj[0], interp_prefactor(c),

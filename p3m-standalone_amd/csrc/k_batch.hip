@@ -49,6 +49,7 @@ struct p3mk_batch {
     // the row-parallel assignment (region + staging)
     size_t lds_z = 0, lds_y = 0, lds_x = 0, lds_assign = 0, lds_rows = 0;
     long ntiles = 0, max_items = 0, ncell = 0;
+    bool use_self = false; // self-force correction of ad / ad-r
     int tile_side = 8; // requested assignment tile side (autotuned)
     int rs_grid = 0;   // persistent real-space grid (autotuned)
     bool time_pairs = false; // events around the half-shell kernel (eager calls only)
@@ -357,6 +358,7 @@ extern "C" int p3mk_batch_configure(p3mk_batch *b, int fp32, int use_self_force,
     if (tile_side != 4 && tile_side != 8)
         return p3mk_fail(P3MK_EINVAL, "assignment tile side must be 4 or 8", 0);
     b->form.fp32 = fp32 != 0;
+    b->use_self = use_self_force != 0;
     b->tile_side = tile_side;
     if (rs_grid > 0)
         b->rs_grid = rs_grid;
@@ -393,12 +395,11 @@ extern "C" int p3mk_batch_info(const p3mk_batch *b, int *ntot, long *ntiles, lon
 }
 
 // k-space force of every system: fk += (3 blocks of ntot), ftot -= self force
-// (methods with the correction)
-extern "C" int p3mk_batch_kspace(p3mk_batch *b, const double *x, const double *y, const double *z,
-                                 const double *q, double *fk, double *ftot, p3mk_queue *qu) {
+// (methods with the correction); the meshes are zero
+static int batch_kspace(p3mk_batch *b, const double *x, const double *y, const double *z, const double *q,
+                        double *fk, double *ftot, p3mk_queue *qu) {
     const BForm &f = b->form;
     const int ns = b->nsys;
-    P3MK_TRY(p3mk_fill_zero(b->mesh_arena, b->mesh_region, qu));
     P3MK_TRY(bpart_sort(f, b->dsys, b->psys, b->tile0s, ns, b->ntiles, b->ntot, x, y, z, q, b->key,
                         b->count, b->start, b->cursor, b->perm, b->chunks, b->cstart, b->imap,
                         b->scan, b->sorted, qu));
@@ -437,13 +438,39 @@ extern "C" int p3mk_batch_kspace(p3mk_batch *b, const double *x, const double *y
                         b->imap, b->sorted, b->perm, b->ntot, fk, ftot, qu);
 }
 
-// real-space force of every system with rcut > 0: fr += (3 blocks of ntot);
-// energy[s] += system s's real-space energy (energy may be NULL)
-extern "C" int p3mk_batch_realspace(p3mk_batch *b, const double *x, const double *y,
-                                    const double *z, const double *q, double *fr, double *energy,
-                                    p3mk_queue *qu) {
-    return brs_forces(b->form, b->dsys, b->psys, b->cell0s, b->nsys, b->ncell, b->ntot, x, y, z, q,
-                      b->cells, b->rs_grid, b->rs_small, b->rs_cells, b->time_pairs, fr, energy, qu);
+extern "C" int p3mk_batch_kspace(p3mk_batch *b, const double *x, const double *y, const double *z,
+                                 const double *q, double *fk, double *ftot, p3mk_queue *qu) {
+    P3MK_TRY(p3mk_fill_zero(b->mesh_arena, b->mesh_region, qu));
+    return batch_kspace(b, x, y, z, q, fk, ftot, qu);
+}
+
+// Calculate_forces of every system: real space (the cell-grid systems' forces
+// stay in sorted order until the end), k space, then one pass that
+// brings the real-space forces to the caller's order and sums both.
+extern "C" int p3mk_batch_forces(p3mk_batch *b, int real, const double *x, const double *y, const double *z,
+                                 const double *q, double *f, double *fk, double *fr, double *energy,
+                                 p3mk_queue *qu) {
+    const size_t n3 = sizeof(double) * 3 * (size_t)b->ntot;
+    const bool small = real && b->rs_small, cells = real && b->rs_cells;
+    p3mk_range r[7];
+    int k = 0;
+    r[k++] = {b->mesh_arena, b->mesh_region};
+    r[k++] = {fk, n3};
+    if (b->use_self)
+        r[k++] = {f, n3};
+    if (energy != nullptr)
+        r[k++] = {energy, sizeof(double) * (size_t)b->nsys};
+    if (small)
+        r[k++] = {fr, n3};
+    if (real)
+        k += brs_ranges(b->cells, b->ntot, cells, r + k);
+    P3MK_TRY(p3mk_fill_zero_many(k, r, qu));
+    if (real)
+        P3MK_TRY(brs_forces(b->form, b->dsys, b->psys, b->cell0s, b->nsys, b->ncell, b->ntot, x, y, z, q,
+                            b->cells, b->rs_grid, b->rs_small, b->rs_cells, b->time_pairs, fr, energy, qu));
+    P3MK_TRY(batch_kspace(b, x, y, z, q, fk, f, qu));
+    return p3mk_finish_forces(b->ntot, cells ? b->cells.key : nullptr, cells ? b->cells.fsorted : nullptr,
+                              small ? 1 : 0, b->use_self ? 1 : 0, fk, fr, f, qu);
 }
 
 extern "C" int p3mk_batch_time_pairs(p3mk_batch *b, int on) {

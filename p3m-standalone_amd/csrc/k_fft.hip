@@ -42,8 +42,9 @@ k_fft_pass(c2_t<T> *data, LineMap m, Radices rp, const c2_t<T> *__restrict__ tw,
 // neighbouring lines.
 template <int N, typename T, bool CONTIG>
 __global__ void __launch_bounds__(kThreads)
-k_fft_p2(c2_t<T> *data, LineMap m, const double2 *__restrict__ tw, int inv) {
+k_fft_p2(Three<c2_t<T> *> set, LineMap m, const double2 *__restrict__ tw, int inv) {
     using V = c2_t<T>;
+    V *data = set.p[blockIdx.y];
     constexpr int TPL = N / 8, LPW = kThreads / TPL, PITCH = N + 1;
     __shared__ V buf[LPW * PITCH];
     const int tid = threadIdx.x;
@@ -267,85 +268,99 @@ template <typename T> int launch_lines(int n, int nbuf, long nlines) {
 }
 
 template <int N, typename T>
-int pass_p2(p3mk_fft *f, c2_t<T> *data, const LineMap &m, int inv, bool contig, p3mk_queue *q) {
+int pass_p2(p3mk_fft *f, Three<c2_t<T> *> data, int k, const LineMap &m, int inv, bool contig, p3mk_queue *q) {
     constexpr int LPW = kThreads / (N / 8);
     const long blocks = (m.nlines + LPW - 1) / LPW;
     const double2 *tw = f->tw64;
     if (contig)
-        hipLaunchKernelGGL((k_fft_p2<N, T, true>), dim3((unsigned)blocks), dim3(kThreads), 0,
+        hipLaunchKernelGGL((k_fft_p2<N, T, true>), dim3((unsigned)blocks, (unsigned)k), dim3(kThreads), 0,
                            p3mk_stream(q), data, m, tw, inv);
     else
-        hipLaunchKernelGGL((k_fft_p2<N, T, false>), dim3((unsigned)blocks), dim3(kThreads), 0,
+        hipLaunchKernelGGL((k_fft_p2<N, T, false>), dim3((unsigned)blocks, (unsigned)k), dim3(kThreads), 0,
                            p3mk_stream(q), data, m, tw, inv);
     return p3mk_launch_check("fft pass");
 }
 
+// one pass over k <= 3 meshes
 template <typename T>
-int pass(p3mk_fft *f, c2_t<T> *data, const LineMap &m, int inv, bool contig, p3mk_queue *q) {
+int pass(p3mk_fft *f, Three<c2_t<T> *> data, int k, const LineMap &m, int inv, bool contig, p3mk_queue *q) {
     switch (m.n) {
-    case 16: return pass_p2<16, T>(f, data, m, inv, contig, q);
-    case 32: return pass_p2<32, T>(f, data, m, inv, contig, q);
-    case 64: return pass_p2<64, T>(f, data, m, inv, contig, q);
-    case 128: return pass_p2<128, T>(f, data, m, inv, contig, q);
-    case 256: return pass_p2<256, T>(f, data, m, inv, contig, q);
+    case 16: return pass_p2<16, T>(f, data, k, m, inv, contig, q);
+    case 32: return pass_p2<32, T>(f, data, k, m, inv, contig, q);
+    case 64: return pass_p2<64, T>(f, data, k, m, inv, contig, q);
+    case 128: return pass_p2<128, T>(f, data, k, m, inv, contig, q);
+    case 256: return pass_p2<256, T>(f, data, k, m, inv, contig, q);
     default: break;
     }
     const c2_t<T> *tw = sizeof(T) == 8 ? (const c2_t<T> *)f->tw64 : (const c2_t<T> *)f->tw32;
     if (f->two.r1 > 0)
-        return two_pass<T>(f->two, data, m, f->tw64, inv, contig, p3mk_stream(q));
+        return two_pass<T>(f->two, data, k, m, f->tw64, inv, contig, p3mk_stream(q));
     const int lt = launch_lines<T>(m.n, 2, m.nlines);
     const size_t lds = 2 * (size_t)lt * (m.n + 1) * sizeof(c2_t<T>);
     const long blocks = (m.nlines + lt - 1) / lt;
-    hipLaunchKernelGGL(k_fft_pass<T>, dim3((unsigned)blocks), dim3(kThreads), lds, p3mk_stream(q),
-                       data, m, f->rp, tw, inv, lt, contig ? 1 : 0);
+    for (int j = 0; j < k; j++)
+        hipLaunchKernelGGL(k_fft_pass<T>, dim3((unsigned)blocks), dim3(kThreads), lds, p3mk_stream(q),
+                           data.p[j], m, f->rp, tw, inv, lt, contig ? 1 : 0);
     return p3mk_launch_check("fft pass");
 }
 
-template <typename T> int forward_zy(p3mk_fft *f, void *mesh, void *spec, p3mk_queue *q) {
+template <typename P> Three<P> three(int k, void *const p[3]) {
+    Three<P> r = {};
+    for (int j = 0; j < k; j++)
+        r.p[j] = (P)p[j];
+    return r;
+}
+
+template <typename T>
+int forward_zy(p3mk_fft *f, int k, void *const mesh[3], void *const spec[3], p3mk_queue *q) {
     using V = c2_t<T>;
     const int M = f->M, H = f->H;
-    const c2_t<T> *tw = sizeof(T) == 8 ? (const V *)f->tw64 : (const V *)f->tw32;
     if (!f->g.r2c) {
-        V *d = (V *)mesh;
+        const Three<V *> d = three<V *>(k, mesh);
         LineMap z = {M, 1, 1, M, (long)M * M};
-        P3MK_TRY(pass<T>(f, d, z, 0, true, q));
+        P3MK_TRY(pass<T>(f, d, k, z, 0, true, q));
         LineMap y = {M, M, M, (long)M * M, (long)M * M};
-        return pass<T>(f, d, y, 0, false, q);
+        return pass<T>(f, d, k, y, 0, false, q);
     }
     const long nl = (long)M * M;
+    const Three<V *> s = three<V *>(k, spec);
     if (f->two.r1 > 0) {
-        P3MK_TRY(two_r2c<T>(f->two, (const T *)mesh, (V *)spec, nl, f->tw64, p3mk_stream(q)));
+        P3MK_TRY(two_r2c<T>(f->two, three<const T *>(k, mesh), s, k, nl, f->tw64, p3mk_stream(q)));
     } else {
+        const c2_t<T> *tw = sizeof(T) == 8 ? (const V *)f->tw64 : (const V *)f->tw32;
         const int lt = launch_lines<T>(M, 2, nl);
         const size_t lds = 2 * (size_t)lt * (M + 1) * sizeof(V);
-        hipLaunchKernelGGL(k_fft_r2c_z<T>, dim3((unsigned)((nl + lt - 1) / lt)), dim3(kThreads), lds,
-                           p3mk_stream(q), (const T *)mesh, (V *)spec, nl, M, f->rp, tw, lt);
+        for (int j = 0; j < k; j++)
+            hipLaunchKernelGGL(k_fft_r2c_z<T>, dim3((unsigned)((nl + lt - 1) / lt)), dim3(kThreads), lds,
+                               p3mk_stream(q), (const T *)mesh[j], s.p[j], nl, M, f->rp, tw, lt);
         P3MK_TRY(p3mk_launch_check("fft r2c"));
     }
     LineMap y = {M, H, H, (long)M * H, (long)M * H};
-    return pass<T>(f, (V *)spec, y, 0, false, q);
+    return pass<T>(f, s, k, y, 0, false, q);
 }
 
-template <typename T> int backward_yz(p3mk_fft *f, void *spec, void *mesh, p3mk_queue *q) {
+template <typename T>
+int backward_yz(p3mk_fft *f, int k, void *const spec[3], void *const mesh[3], p3mk_queue *q) {
     using V = c2_t<T>;
     const int M = f->M, H = f->H;
-    const c2_t<T> *tw = sizeof(T) == 8 ? (const V *)f->tw64 : (const V *)f->tw32;
+    const Three<V *> s = three<V *>(k, spec);
     if (!f->g.r2c) {
-        V *d = (V *)spec;
         LineMap y = {M, M, M, (long)M * M, (long)M * M};
-        P3MK_TRY(pass<T>(f, d, y, 1, false, q));
+        P3MK_TRY(pass<T>(f, s, k, y, 1, false, q));
         LineMap z = {M, 1, 1, M, (long)M * M};
-        return pass<T>(f, d, z, 1, true, q);
+        return pass<T>(f, s, k, z, 1, true, q);
     }
     LineMap y = {M, H, H, (long)M * H, (long)M * H};
-    P3MK_TRY(pass<T>(f, (V *)spec, y, 1, false, q));
+    P3MK_TRY(pass<T>(f, s, k, y, 1, false, q));
     const long nl = (long)M * M;
     if (f->two.r1 > 0)
-        return two_c2r<T>(f->two, (const V *)spec, (T *)mesh, nl, f->tw64, p3mk_stream(q));
+        return two_c2r<T>(f->two, three<const V *>(k, spec), three<T *>(k, mesh), k, nl, f->tw64, p3mk_stream(q));
+    const c2_t<T> *tw = sizeof(T) == 8 ? (const V *)f->tw64 : (const V *)f->tw32;
     const int lt = launch_lines<T>(M, 2, nl);
     const size_t lds = 2 * (size_t)lt * (M + 1) * sizeof(V);
-    hipLaunchKernelGGL(k_fft_c2r_z<T>, dim3((unsigned)((nl + lt - 1) / lt)), dim3(kThreads), lds,
-                       p3mk_stream(q), (const V *)spec, (T *)mesh, nl, M, f->rp, tw, lt);
+    for (int j = 0; j < k; j++)
+        hipLaunchKernelGGL(k_fft_c2r_z<T>, dim3((unsigned)((nl + lt - 1) / lt)), dim3(kThreads), lds,
+                           p3mk_stream(q), (const V *)spec[j], (T *)mesh[j], nl, M, f->rp, tw, lt);
     return p3mk_launch_check("fft c2r");
 }
 
@@ -479,12 +494,24 @@ int bfft_convolve_x(const BForm &f, const BSys *sys, const long *blk, int nsys, 
 
 }  // namespace p3m
 
+extern "C" int p3mk_fft_forward_zy_many(p3mk_fft *f, int k, void *const mesh[3], void *const spec[3],
+                                        p3mk_queue *q) {
+    return f->g.fp32 ? forward_zy<float>(f, k, mesh, spec, q) : forward_zy<double>(f, k, mesh, spec, q);
+}
+
+extern "C" int p3mk_fft_backward_yz_many(p3mk_fft *f, int k, void *const spec[3], void *const mesh[3],
+                                         p3mk_queue *q) {
+    return f->g.fp32 ? backward_yz<float>(f, k, spec, mesh, q) : backward_yz<double>(f, k, spec, mesh, q);
+}
+
 extern "C" int p3mk_fft_forward_zy(p3mk_fft *f, void *mesh, void *spec, p3mk_queue *q) {
-    return f->g.fp32 ? forward_zy<float>(f, mesh, spec, q) : forward_zy<double>(f, mesh, spec, q);
+    void *const m[3] = {mesh, nullptr, nullptr}, *const s[3] = {spec, nullptr, nullptr};
+    return p3mk_fft_forward_zy_many(f, 1, m, s, q);
 }
 
 extern "C" int p3mk_fft_backward_yz(p3mk_fft *f, void *spec, void *mesh, p3mk_queue *q) {
-    return f->g.fp32 ? backward_yz<float>(f, spec, mesh, q) : backward_yz<double>(f, spec, mesh, q);
+    void *const m[3] = {mesh, nullptr, nullptr}, *const s[3] = {spec, nullptr, nullptr};
+    return p3mk_fft_backward_yz_many(f, 1, s, m, q);
 }
 
 extern "C" int p3mk_convolve(p3mk_fft *f, int nout, const double *G, const double *Dn, void *spec,
@@ -505,13 +532,13 @@ template <typename T> static int fft3d(p3mk_fft *f, void *data, int sign, p3mk_q
     using V = c2_t<T>;
     const int M = f->M;
     const int inv = sign > 0;
-    V *d = (V *)data;
+    const Three<V *> d = {{(V *)data, nullptr, nullptr}};
     LineMap z = {M, 1, 1, M, (long)M * M};
     LineMap y = {M, M, M, (long)M * M, (long)M * M};
     LineMap x = {M, (long)M * M, (long)M * M, 0, (long)M * M};
-    P3MK_TRY(pass<T>(f, d, z, inv, true, q));
-    P3MK_TRY(pass<T>(f, d, y, inv, false, q));
-    return pass<T>(f, d, x, inv, false, q);
+    P3MK_TRY(pass<T>(f, d, 1, z, inv, true, q));
+    P3MK_TRY(pass<T>(f, d, 1, y, inv, false, q));
+    return pass<T>(f, d, 1, x, inv, false, q);
 }
 
 extern "C" int p3mk_fft3d(p3mk_fft *f, void *data, int sign, p3mk_queue *q) {

@@ -206,6 +206,56 @@ __global__ void k_item_map(const int *__restrict__ cstart, long ntiles, int2 *__
         imap[c] = make_int2((int)t, c - b);
 }
 
+// Tile starts, chunk prefix sums and the item map in one workgroup, for up to
+// kSmallTiles tiles (k_tile_ranges, a scan and k_item_map: three launches of
+// 4 us each): thread t takes its run of consecutive tiles.
+constexpr int kTileItemThreads = 1024;
+constexpr long kSmallTiles = 4096;
+
+__global__ void __launch_bounds__(kTileItemThreads)
+k_tile_items(const int *__restrict__ fstart, int ntiles, int T3, int *__restrict__ start,
+             int *__restrict__ cstart, int2 *__restrict__ imap) {
+    __shared__ int wsum[kTileItemThreads / 64];
+    constexpr int kRun = (int)(kSmallTiles / kTileItemThreads);
+    const int run = (ntiles + kTileItemThreads - 1) / kTileItemThreads;
+    const int t0 = (int)threadIdx.x * run, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int chunks[kRun];
+    int sum = 0;
+#pragma unroll
+    for (int k = 0; k < kRun; k++) {
+        chunks[k] = 0;
+        if (k < run && t0 + k < ntiles) {
+            const int s = fstart[(t0 + k) * T3], e = fstart[(t0 + k + 1) * T3];
+            start[t0 + k] = s;
+            chunks[k] = (e - s + kChunk - 1) / kChunk;
+            sum += chunks[k];
+        }
+    }
+    int x = sum;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(x, off, 64);
+        x += lane >= off ? y : 0;
+    }
+    if (lane == 63)
+        wsum[wave] = x;
+    __syncthreads();
+    int before = x - sum;
+    for (int w = 0; w < wave; w++)
+        before += wsum[w];
+#pragma unroll
+    for (int k = 0; k < kRun; k++)
+        if (k < run && t0 + k < ntiles) {
+            cstart[t0 + k] = before;
+            for (int c = 0; c < chunks[k]; c++)
+                imap[before + c] = make_int2(t0 + k, c);
+            before += chunks[k];
+        }
+    if (threadIdx.x == kTileItemThreads - 1) {
+        start[ntiles] = fstart[ntiles * T3];
+        cstart[ntiles] = before;
+    }
+}
+
 // the batched form: (global tile, chunk, system)
 __global__ void k_bitem_map(const int *__restrict__ cstart, long ntiles, const long *__restrict__ tile0s,
                             int nsys, int4 *__restrict__ imap) {
@@ -686,7 +736,8 @@ int launch_interp_ik(const p3mk_geom *g, int n, const p3mk_psort *s, void *const
 
 template <typename T, bool R2C>
 int launch_interp_ad(const p3mk_geom *g, int n, const p3mk_psort *s, const void *phi,
-                     double prefac, const double *selfb, double *fk, double *f, p3mk_queue *qu) {
+                     double prefac, const double *selfb, double *fk, double *f,
+                     p3mk_queue *qu) {
     const double Hi = (double)g->M / g->L;
     const double h = g->L / g->M;
     const T *ph = (const T *)phi;
@@ -705,11 +756,11 @@ int launch_interp_ad(const p3mk_geom *g, int n, const p3mk_psort *s, const void 
         if (il)                                                                                    \
             P3MK_TRY(launch_lds(k_interp_ad_tile<P, T, R2C, true>, grid, lds, st, \
                                s->sorted, s->perm, s->start, s->cstart, s->imap, s->ntiles, s->nt, s->T,    \
-                               g->M, Hi, 1.0 / g->L, ph, prefac, selfb, h, fk, f, (long)n));        \
+                               g->M, Hi, 1.0 / g->L, ph, prefac, selfb, h, fk, f, (long)n));   \
         else                                                                                       \
             P3MK_TRY(launch_lds(k_interp_ad_tile<P, T, R2C, false>, grid, lds,    \
                                st, s->sorted, s->perm, s->start, s->cstart, s->imap, s->ntiles, s->nt, s->T, \
-                               g->M, Hi, 1.0 / g->L, ph, prefac, selfb, h, fk, f, (long)n));        \
+                               g->M, Hi, 1.0 / g->L, ph, prefac, selfb, h, fk, f, (long)n));   \
         break;
         CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7)
 #undef CASE
@@ -782,14 +833,32 @@ int launch_adjoint(const p3mk_geom *g, int ad, int n, const p3mk_psort *s, const
 
 }  // namespace
 
+extern "C" int p3mk_assign_ranges(const p3mk_geom *g, p3mk_psort *s, void *mesh, p3mk_range r[2]) {
+    r[0] = {mesh, p3mk_mesh_bytes(g)};
+    if (s->nf == 0)
+        return 1;
+    r[1] = {s->fcount, sizeof(int) * ((size_t)s->nf + 1)};
+    return 2;
+}
+
 extern "C" int p3mk_assign(const p3mk_geom *g, int n, const double *x, const double *y,
                            const double *z, const double *q, p3mk_psort *s, void *mesh,
                            p3mk_queue *qu) {
     if (n > s->nmax || g->M != s->M)
         return p3mk_fail(P3MK_EINVAL, "particle sort was made for another size", 0);
+    p3mk_range r[2];
+    const int k = p3mk_assign_ranges(g, s, mesh, r);
+    P3MK_TRY(p3mk_fill_zero_many(n > 0 ? k : 1, r, qu));
+    return p3mk_assign_filled(g, n, x, y, z, q, s, mesh, qu);
+}
+
+extern "C" int p3mk_assign_filled(const p3mk_geom *g, int n, const double *x, const double *y,
+                                  const double *z, const double *q, p3mk_psort *s, void *mesh,
+                                  p3mk_queue *qu) {
+    if (n > s->nmax || g->M != s->M)
+        return p3mk_fail(P3MK_EINVAL, "particle sort was made for another size", 0);
     hipStream_t st = p3mk_stream(qu);
     s->n = n;
-    P3MK_TRY(p3mk_fill_zero(mesh, p3mk_mesh_bytes(g), qu));
     if (n <= 0)
         return P3MK_OK;
     const double Hi = (double)g->M / g->L;
@@ -797,7 +866,6 @@ extern "C" int p3mk_assign(const p3mk_geom *g, int n, const double *x, const dou
     const size_t nt1 = (size_t)s->ntiles + 1;
     if (s->nf > 0) {
         const int T3 = s->T * s->T * s->T;
-        P3MK_TRY(p3mk_fill_zero(s->fcount, sizeof(int) * ((size_t)s->nf + 1), qu));
         hipLaunchKernelGGL(k_fine_count, dim3(nb), dim3(256), 0, st, n, x, y, z, Hi, g->cao, g->M, s->T,
                            s->nt, s->key, s->rank, s->fcount);
         P3MK_TRY(p3mk_launch_check("base count"));
@@ -805,6 +873,12 @@ extern "C" int p3mk_assign(const p3mk_geom *g, int n, const double *x, const dou
         hipLaunchKernelGGL(k_fine_scatter, dim3(nb), dim3(256), 0, st, n, x, y, z, q, s->key, s->rank,
                            s->fstart, s->perm, s->sorted);
         P3MK_TRY(p3mk_launch_check("base scatter"));
+        if (s->ntiles <= kSmallTiles) {
+            hipLaunchKernelGGL(k_tile_items, dim3(1), dim3(kTileItemThreads), 0, st, s->fstart, (int)s->ntiles,
+                               T3, s->start, s->cstart, s->imap);
+            P3MK_TRY(p3mk_launch_check("tile items"));
+            return assign_mode(g, n, s, mesh, kCharge, nullptr, qu);
+        }
         hipLaunchKernelGGL(k_tile_ranges, dim3((unsigned)((s->ntiles + 256) / 256)), dim3(256), 0, st,
                            s->fstart, s->ntiles, T3, s->start, s->count, s->chunks);
         P3MK_TRY(p3mk_launch_check("tile ranges"));

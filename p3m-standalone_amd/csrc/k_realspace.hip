@@ -189,6 +189,52 @@ __global__ void k_cell_start_items(const int *__restrict__ fstart, long ncell, i
         items[c] = (fstart[8 * (c + 1)] - fstart[8 * c] + 63) / 64;
 }
 
+// the same with the items' prefix sums, in one workgroup for up to
+// kSmallCells cells (two launches otherwise): thread t takes its run of cells
+constexpr int kCellItemThreads = 1024;
+constexpr long kSmallCells = 4096;
+
+__global__ void __launch_bounds__(kCellItemThreads)
+k_cell_items_small(const int *__restrict__ fstart, int ncell, int *__restrict__ start, int *__restrict__ istart) {
+    __shared__ int wsum[kCellItemThreads / 64];
+    constexpr int kRun = (int)(kSmallCells / kCellItemThreads);
+    const int run = (ncell + kCellItemThreads - 1) / kCellItemThreads;
+    const int c0 = (int)threadIdx.x * run, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int items[kRun];
+    int sum = 0;
+#pragma unroll
+    for (int k = 0; k < kRun; k++) {
+        items[k] = 0;
+        if (k < run && c0 + k < ncell) {
+            const int s = fstart[8 * (c0 + k)], e = fstart[8 * (c0 + k + 1)];
+            start[c0 + k] = s;
+            items[k] = (e - s + 63) / 64;
+            sum += items[k];
+        }
+    }
+    int x = sum;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(x, off, 64);
+        x += lane >= off ? y : 0;
+    }
+    if (lane == 63)
+        wsum[wave] = x;
+    __syncthreads();
+    int before = x - sum;
+    for (int w = 0; w < wave; w++)
+        before += wsum[w];
+#pragma unroll
+    for (int k = 0; k < kRun; k++)
+        if (k < run && c0 + k < ncell) {
+            istart[c0 + k] = before;
+            before += items[k];
+        }
+    if (threadIdx.x == kCellItemThreads - 1) {
+        start[ncell] = fstart[8 * ncell];
+        istart[ncell] = before;
+    }
+}
+
 // last index k with prefix[k] <= v
 __device__ __forceinline__ long prefix_find(const int *__restrict__ prefix, long count, int v) {
     long lo = 0, hi = count;
@@ -1557,11 +1603,10 @@ int cells_alloc(CellArrays &a, long n, long ncell) {
     return rc;
 }
 
-// zero the octant counts and the work-item counters (one allocation) before
+// the octant counts and the work-item counters (one allocation), zero before
 // the keys are counted
-static int cells_begin(CellArrays &a, long ncell, p3mk_queue *qu) {
-    (void)ncell;
-    return p3mk_fill_zero(a.fcount, sizeof(int) * (size_t)(a.counter + kCounters - a.fcount), qu);
+static p3mk_range cells_counts(CellArrays &a) {
+    return {a.fcount, sizeof(int) * (size_t)(a.counter + kCounters - a.fcount)};
 }
 
 // octant starts after the count (before the scatter)
@@ -1569,9 +1614,17 @@ static int cells_scan(CellArrays &a, long ncell, p3mk_queue *qu) {
     return p3mk_exclusive_scan(a.fcount, 8 * ncell, a.fstart, a.scan, qu);
 }
 
-// after the scatter: cell starts, work items, item boxes, counter reset
+// after the scatter: cell starts, work items, item boxes
 static int cells_end(CellArrays &a, long ncell, p3mk_queue *qu) {
     hipStream_t s = p3mk_stream(qu);
+    if (ncell <= kSmallCells) {
+        hipLaunchKernelGGL(k_cell_items_small, dim3(1), dim3(kCellItemThreads), 0, s, a.fstart, (int)ncell,
+                           a.start, a.istart);
+        P3MK_TRY(p3mk_launch_check("cell items"));
+        hipLaunchKernelGGL(k_item_bbox, dim3((unsigned)((a.max_items * kBoxLanes + 255) / 256)), dim3(256), 0, s,
+                           a.start, a.istart, ncell, a.max_items, a.sorted, a.bbox);
+        return p3mk_launch_check("item boxes");
+    }
     hipLaunchKernelGGL(k_cell_start_items, dim3((unsigned)((ncell + 1 + 255) / 256)), dim3(256), 0, s,
                        a.fstart, ncell, a.start, a.items);
     P3MK_TRY(p3mk_launch_check("cell starts"));
@@ -1634,7 +1687,7 @@ extern "C" int p3mk_cells_create(p3mk_cells **out, int n, double L, double rcut,
     return P3MK_OK;
 }
 
-// sort the particles into the cell list (with g: also the cotangent)
+// sort the particles into the cell list, its counts zero (with g: also the cotangent)
 static int build_cells(p3mk_cells *c, int n, double L, const double *x, const double *y,
                        const double *z, const double *q, double rcut, const double *g,
                        p3mk_queue *qu) {
@@ -1643,7 +1696,6 @@ static int build_cells(p3mk_cells *c, int n, double L, const double *x, const do
     CellArrays &a = c->a;
     hipStream_t s = p3mk_stream(qu);
     const int nb = (n + 255) / 256, nbp = (n + kPad + 255) / 256;
-    P3MK_TRY(p3m::cells_begin(a, c->ncell, qu));
     hipLaunchKernelGGL(k_cell_count, dim3(nb), dim3(256), 0, s, n, x, y, z, L, c->inv_side, c->nc,
                        a.key, a.rank, a.fcount);
     P3MK_TRY(p3mk_launch_check("cell count"));
@@ -1663,6 +1715,8 @@ extern "C" int p3mk_realspace_vjp(p3mk_cells *c, int n, double L, const double *
     CellArrays &a = c->a;
     if (a.gsorted == nullptr)
         P3MK_TRY(p3mk_alloc((void **)&a.gsorted, sizeof(double4) * ((size_t)c->nmax + kPad)));
+    const p3mk_range counts = p3m::cells_counts(a);
+    P3MK_TRY(p3mk_fill_zero_many(1, &counts, qu));
     P3MK_TRY(build_cells(c, n, L, x, y, z, q, rcut, g, qu));
     const bool all_cells = (2 * c->reach + 1 > c->nc);
     const dim3 grid((unsigned)std::min<long>(c->grid, a.max_items));
@@ -1678,9 +1732,42 @@ extern "C" int p3mk_realspace_vjp(p3mk_cells *c, int n, double L, const double *
     return p3mk_launch_check("real-space adjoint");
 }
 
+extern "C" int p3mk_realspace_sorted(const p3mk_cells *c) { return 2 * c->reach + 1 <= c->nc; }
+
+extern "C" int p3mk_realspace_ranges(p3mk_cells *c, int n, p3mk_range r[2]) {
+    r[0] = p3m::cells_counts(c->a);
+    if (!p3mk_realspace_sorted(c) || n <= 0)
+        return 1;
+    r[1] = {c->a.fsorted, sizeof(double) * 3 * (size_t)n};
+    return 2;
+}
+
 extern "C" int p3mk_realspace(p3mk_cells *c, int n, double L, const double *x, const double *y,
                               const double *z, const double *q, double rcut, double alpha,
                               int fp32, double *fr, double *energy, p3mk_queue *qu) {
+    if (n <= 0)
+        return P3MK_OK;
+    if (n > c->nmax)
+        return p3mk_fail(P3MK_EINVAL, "cell list was built for another system size, box or cutoff", 0);
+    p3mk_range r[2];
+    P3MK_TRY(p3mk_fill_zero_many(p3mk_realspace_ranges(c, n, r), r, qu));
+    const int *pos = nullptr;
+    const double *fs = nullptr;
+    P3MK_TRY(p3mk_realspace_filled(c, n, L, x, y, z, q, rcut, alpha, fp32, fr, energy, &pos, &fs, qu));
+    if (fs != nullptr) {
+        hipLaunchKernelGGL(k_unsort_add, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, p3mk_stream(qu), n, pos,
+                           fs, (long)n, fr);
+        return p3mk_launch_check("realspace forces to caller order");
+    }
+    return P3MK_OK;
+}
+
+extern "C" int p3mk_realspace_filled(p3mk_cells *c, int n, double L, const double *x, const double *y,
+                                     const double *z, const double *q, double rcut, double alpha, int fp32,
+                                     double *fr, double *energy, const int **pos, const double **fs,
+                                     p3mk_queue *qu) {
+    *pos = nullptr;
+    *fs = nullptr;
     if (n <= 0)
         return P3MK_OK;
     CellArrays &a = c->a;
@@ -1690,9 +1777,8 @@ extern "C" int p3mk_realspace(p3mk_cells *c, int n, double L, const double *x, c
     const long units = all_cells ? a.max_items : a.max_items << kMaxSplitBits;
     const dim3 grid((unsigned)std::min<long>(c->grid, units));
     if (!all_cells) {
-        // half shell: forces summed in sorted order, then added by perm
+        // half shell: forces summed in sorted order
         P3MK_TRY(build_cells(c, n, L, x, y, z, q, rcut, nullptr, qu));
-        P3MK_TRY(p3mk_fill_zero(a.fsorted, sizeof(double) * 3 * (size_t)n, qu));
         // the pair kernel alone between two events
         P3MK_TRY(p3mk_record(qu, P3MK_EV_PAIRS));
         if (fp32)
@@ -1704,10 +1790,9 @@ extern "C" int p3mk_realspace(p3mk_cells *c, int n, double L, const double *x, c
                                a.sortedq, a.start, a.istart, a.bbox, c->ncell, c->nc, c->reach, L,
                                rcut, alpha, a.counter, (long)n, a.fsorted, energy);
         P3MK_TRY(p3mk_launch_check("realspace (half shell)"));
-        P3MK_TRY(p3mk_record(qu, P3MK_EV_PAIRS + 1));
-        hipLaunchKernelGGL(k_unsort_add, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, a.key,
-                           a.fsorted, (long)n, fr);
-        return p3mk_launch_check("realspace forces to caller order");
+        *pos = a.key;
+        *fs = a.fsorted;
+        return p3mk_record(qu, P3MK_EV_PAIRS + 1);
     }
     P3MK_TRY(build_cells(c, n, L, x, y, z, q, rcut, nullptr, qu));
 #define LAUNCH(F32, SB)                                                                            \
@@ -1856,6 +1941,14 @@ k_brealspace_half(const BSys *__restrict__ sys, const int *__restrict__ cell0s, 
 
 namespace p3m {
 
+int brs_ranges(CellArrays &a, int ntot, bool any_cells, p3mk_range r[2]) {
+    r[0] = cells_counts(a);
+    if (!any_cells)
+        return 1;
+    r[1] = {a.fsorted, sizeof(double) * 3 * (size_t)ntot};
+    return 2;
+}
+
 int brs_forces(const BForm &f, const BSys *sys, const int *psys, const int *cell0s, int nsys,
                long ncell, int ntot, const double *x, const double *y, const double *z,
                const double *q, CellArrays &a, int grid, bool any_small, bool any_cells,
@@ -1864,7 +1957,6 @@ int brs_forces(const BForm &f, const BSys *sys, const int *psys, const int *cell
         return P3MK_OK;
     hipStream_t s = p3mk_stream(qu);
     const int nb = (ntot + 255) / 256;
-    P3MK_TRY(cells_begin(a, ncell, qu));
     hipLaunchKernelGGL(k_bcell_count, dim3(nb), dim3(256), 0, s, ntot, sys, psys, x, y, z, a.key,
                        a.rank, a.fcount);
     P3MK_TRY(p3mk_launch_check("batched cell count"));
@@ -1887,8 +1979,7 @@ int brs_forces(const BForm &f, const BSys *sys, const int *psys, const int *cell
         P3MK_TRY(p3mk_launch_check("batched real space (nearest images)"));
     }
     if (any_cells) {
-        // cell-grid systems: half shell in sorted order, then added by perm
-        P3MK_TRY(p3mk_fill_zero(a.fsorted, sizeof(double) * 3 * (size_t)ntot, qu));
+        // cell-grid systems: half shell in sorted order
         // the half-shell kernel alone between two events, on request (not
         // in captured graphs)
         if (time_pairs)
@@ -1904,9 +1995,6 @@ int brs_forces(const BForm &f, const BSys *sys, const int *psys, const int *cell
         P3MK_TRY(p3mk_launch_check("batched real space (half shell)"));
         if (time_pairs)
             P3MK_TRY(p3mk_record(qu, P3MK_EV_PAIRS + 1));
-        hipLaunchKernelGGL(k_unsort_add, dim3((unsigned)((ntot + 255) / 256)), dim3(256), 0, s, ntot,
-                           a.key, a.fsorted, (long)ntot, fr);
-        P3MK_TRY(p3mk_launch_check("batched real-space forces to caller order"));
     }
     return P3MK_OK;
 }

@@ -274,24 +274,93 @@ extern "C" int p3mk_axpy(size_t n, double a, const double *x, double *y, p3mk_qu
     return p3mk_launch_check("axpy");
 }
 
-// f[i] += fk[i] + fr[i]: the sum of Calculate_forces in its order
-// (common.c:315-319), so the total force rounds as the reference's does.
-__global__ void k_sum_parts(size_t n, const double *__restrict__ fk, const double *__restrict__ fr,
-                            double *__restrict__ f) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride)
-        f[i] += fk[i] + fr[i];
+struct FillRanges {
+    unsigned char *p[P3MK_MAX_RANGES];
+    unsigned long long bytes[P3MK_MAX_RANGES], first[P3MK_MAX_RANGES + 1]; // first 16-byte unit of each
+};
+
+__global__ void k_fill_many(FillRanges r, int k) {
+    const unsigned long long stride = (unsigned long long)gridDim.x * blockDim.x;
+    const uint4 z = make_uint4(0u, 0u, 0u, 0u);
+    for (unsigned long long u = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x; u < r.first[k];
+         u += stride) {
+        int s = 0;
+#pragma unroll
+        for (int j = 1; j < P3MK_MAX_RANGES; j++)
+            s += (j < k && u >= r.first[j]) ? 1 : 0;
+        unsigned char *base = r.p[0];
+        unsigned long long bytes = r.bytes[0], first = r.first[0];
+#pragma unroll
+        for (int j = 1; j < P3MK_MAX_RANGES; j++)
+            if (s == j) {
+                base = r.p[j];
+                bytes = r.bytes[j];
+                first = r.first[j];
+            }
+        const unsigned long long at = (u - first) * 16;
+        if (at + 16 <= bytes) {
+            *reinterpret_cast<uint4 *>(base + at) = z;
+        } else {
+            for (unsigned long long b = at; b + 4 <= bytes; b += 4)
+                *reinterpret_cast<unsigned int *>(base + b) = 0u;
+        }
+    }
 }
 
-extern "C" int p3mk_sum_parts(size_t n, const double *fk, const double *fr, double *f, p3mk_queue *q) {
+// One launch for all the buffers a force evaluation starts from zero (a
+// launch each, and one more for a size that is no multiple of 16 bytes, were
+// a third of a small system's launches).
+extern "C" int p3mk_fill_zero_many(int k, const p3mk_range *ranges, p3mk_queue *q) {
+    FillRanges r = {};
+    int n = 0;
+    unsigned long long units = 0;
+    for (int j = 0; j < k; j++) {
+        if (ranges[j].bytes == 0)
+            continue;
+        if (n == P3MK_MAX_RANGES || ranges[j].bytes % 4 != 0)
+            return p3mk_fail(P3MK_EINVAL, "zero fill: too many ranges or an odd size", 0);
+        r.p[n] = (unsigned char *)ranges[j].p;
+        r.bytes[n] = ranges[j].bytes;
+        r.first[n] = units;
+        units += (ranges[j].bytes + 15) / 16;
+        n++;
+    }
     if (n == 0)
         return P3MK_OK;
-    size_t blocks = (n + 255) / 256;
-    if (blocks > 8192)
-        blocks = 8192;
-    hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)blocks), dim3(256), 0, q->stream, n, fk, fr, f);
-    return p3mk_launch_check("sum_parts");
+    for (int j = n; j <= P3MK_MAX_RANGES; j++)
+        r.first[j] = units;
+    const unsigned blocks = (unsigned)(units > 8192ull * 256 ? 8192 : (units + 255) / 256);
+    hipLaunchKernelGGL(k_fill_many, dim3(blocks), dim3(256), 0, q->stream, r, n);
+    return p3mk_launch_check("fill_zero");
+}
+
+// The reference's sum (common.c:315-319): f_k + f_r rounded, then added to f.
+__global__ void k_finish_forces(int n, const int *__restrict__ pos, const double *__restrict__ fs, int add_fr,
+                                int add_f, const double *__restrict__ fk, double *__restrict__ fr,
+                                double *__restrict__ f) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n)
+        return;
+    const long p = fs != nullptr ? pos[i] : 0;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const long j = (long)d * n + i;
+        double r = add_fr ? fr[j] : 0.0;
+        if (fs != nullptr)
+            r += fs[(long)d * n + p];
+        fr[j] = r;
+        const double s = fk[j] + r;
+        f[j] = add_f ? f[j] + s : s;
+    }
+}
+
+extern "C" int p3mk_finish_forces(int n, const int *pos, const double *fs, int add_fr, int add_f,
+                                  const double *fk, double *fr, double *f, p3mk_queue *q) {
+    if (n <= 0)
+        return P3MK_OK;
+    hipLaunchKernelGGL(k_finish_forces, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, q->stream, n, pos, fs,
+                       add_fr, add_f, fk, fr, f);
+    return p3mk_launch_check("finish forces");
 }
 
 __global__ void k_check_positions(int n, double lo, double hi, const double *__restrict__ x,

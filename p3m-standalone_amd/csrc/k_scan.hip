@@ -1,9 +1,9 @@
 // Exclusive prefix sum of int counts, used by the counting sorts of the
 // particle <-> mesh and real-space kernels.  Up to 4096 counts: one launch
 // of one workgroup (runs of up to four counts per thread; longer serial runs
-// lose to the three launches below).  Beyond: three launches, per-block
-// scans of 1024 elements, a scan of the block sums, and the block offsets
-// added.
+// lose to the launches below).  Beyond: two launches, per-block scans of 1024
+// elements, and the sums of the blocks before added (each block adds them up
+// itself: a launch less than a scan of the sums, 4 us of a system's step).
 #include <hip/hip_runtime.h>
 
 #include "k_internal.hpp"
@@ -52,33 +52,28 @@ __global__ void __launch_bounds__(kBlock) k_scan_blocks(const int *__restrict__ 
         sums[blockIdx.x] = total;
 }
 
-// single block: exclusive scan of nb block sums (nb <= 1024 * 1024 handled by
-// a serial carry over 1024-chunks), total written to sums[nb]
-__global__ void __launch_bounds__(kBlock) k_scan_sums(int *__restrict__ sums, int nb) {
-    __shared__ int sh[128];
-    int carry = 0;
-    for (int base = 0; base < nb; base += kBlock) {
-        const int i = base + threadIdx.x;
-        const int v = (i < nb) ? sums[i] : 0;
-        int total;
-        const int e = block_exclusive_scan(v, sh, total);
-        __syncthreads();
-        if (i < nb)
-            sums[i] = carry + e;
-        carry += total;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-        sums[nb] = carry;
-}
-
+// adds to each block's elements the sums of the blocks before it, which the
+// block adds up itself (at most a few thousand, one or two per thread)
 __global__ void __launch_bounds__(kBlock) k_scan_add(int *__restrict__ out, int m,
                                                      const int *__restrict__ sums, int nb) {
+    __shared__ int sh[kBlock / 64];
+    int part = 0;
+    for (int b = threadIdx.x; b < (int)blockIdx.x; b += kBlock)
+        part += sums[b];
+    for (int off = 32; off > 0; off >>= 1)
+        part += __shfl_xor(part, off, 64);
+    if ((threadIdx.x & 63) == 0)
+        sh[threadIdx.x >> 6] = part;
+    __syncthreads();
+    int before = 0;
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; w++)
+        before += sh[w];
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i < m)
-        out[i] += sums[blockIdx.x];
-    if (i == 0)
-        out[m] = sums[nb];
+        out[i] += before;
+    if ((int)blockIdx.x == nb - 1 && threadIdx.x == 0)
+        out[m] = before + sums[nb - 1];
 }
 
 // one workgroup: thread t sums its run of ceil(m / 1024) consecutive counts,
@@ -120,8 +115,6 @@ int p3mk_exclusive_scan(const int *count, long m, int *start, int *scratch, p3mk
     }
     hipLaunchKernelGGL(k_scan_blocks, dim3(nb), dim3(kBlock), 0, s, count, (int)m, start, scratch);
     P3MK_TRY(p3mk_launch_check("scan blocks"));
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kBlock), 0, s, scratch, nb);
-    P3MK_TRY(p3mk_launch_check("scan sums"));
     hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(kBlock), 0, s, start, (int)m, scratch, nb);
     return p3mk_launch_check("scan add");
 }

@@ -54,10 +54,21 @@ int p3mk_copy_d2h(void *dst, const void *src, size_t bytes, p3mk_queue *q);
 int p3mk_copy_d2d(void *dst, const void *src, size_t bytes, p3mk_queue *q);
 /* zero fill by a kernel (safe inside captured graphs) */
 int p3mk_fill_zero(void *p, size_t bytes, p3mk_queue *q);
+/* the same over up to P3MK_MAX_RANGES ranges (sizes multiples of 4 bytes) in
+ * one launch */
+typedef struct {
+    void *p;
+    size_t bytes;
+} p3mk_range;
+#define P3MK_MAX_RANGES 8
+int p3mk_fill_zero_many(int k, const p3mk_range *r, p3mk_queue *q);
 /* y[i] += a * x[i] for i < n (FP64) */
 int p3mk_axpy(size_t n, double a, const double *x, double *y, p3mk_queue *q);
-/* f[i] += fk[i] + fr[i] for i < n (FP64; Calculate_forces' order) */
-int p3mk_sum_parts(size_t n, const double *fk, const double *fr, double *f, p3mk_queue *q);
+/* last step of Calculate_forces over n particles (3 blocks of n):
+ * fr = (add_fr ? fr : 0) + (fs ? fs[pos[i]] : 0), f = (add_f ? f : 0) + (fk + fr)
+ * (FP64, the reference's order); fs: forces in the sorted order of pos */
+int p3mk_finish_forces(int n, const int *pos, const double *fs, int add_fr, int add_f, const double *fk,
+                       double *fr, double *f, p3mk_queue *q);
 /* positions inside [lo, hi) (not NaN)?  *bad receives the count of others */
 int p3mk_check_positions(int n, double lo, double hi, const double *x, const double *y,
                          const double *z, int *bad, int *scratch, p3mk_queue *q);
@@ -97,6 +108,11 @@ int p3mk_divergence(p3mk_fft *f, const double *G, const double *Dn, void *const 
 /* backward transform along y and z: c2c in place (mesh == spec);
  * r2c spec -> real mesh */
 int p3mk_fft_backward_yz(p3mk_fft *f, void *spec, void *mesh, p3mk_queue *q);
+/* the same for k <= 3 meshes, one launch per pass */
+int p3mk_fft_forward_zy_many(p3mk_fft *f, int k, void *const mesh[3], void *const spec[3],
+                             p3mk_queue *q);
+int p3mk_fft_backward_yz_many(p3mk_fft *f, int k, void *const spec[3], void *const mesh[3],
+                              p3mk_queue *q);
 /* plain 3D transforms of a complex M^3 (c2c geometry) array, for tests:
  * sign -1 forward, +1 backward, unnormalised, in place */
 int p3mk_fft3d(p3mk_fft *f, void *data, int sign, p3mk_queue *q);
@@ -111,7 +127,11 @@ void p3mk_psort_destroy(p3mk_psort *s);
  * every mesh point is written, no prior zeroing needed */
 int p3mk_assign(const p3mk_geom *g, int n, const double *x, const double *y, const double *z,
                 const double *q, p3mk_psort *s, void *mesh, p3mk_queue *qu);
-/* ik back-interpolation: fk[d*n + i] += -prefac * sum W F_d (meshes F[0..2]) */
+/* p3mk_assign in two parts, for a caller that zero-fills the ranges of the
+ * first (at most 2; returns their number) in a launch of its own */
+int p3mk_assign_ranges(const p3mk_geom *g, p3mk_psort *s, void *mesh, p3mk_range r[2]);
+int p3mk_assign_filled(const p3mk_geom *g, int n, const double *x, const double *y, const double *z,
+                       const double *q, p3mk_psort *s, void *mesh, p3mk_queue *qu);
 /* assignment with the sort of the last p3mk_assign (same particles, n):
  * mode 1: particle i deposits q_i gv[i] W_i; mode 2: q_i sum_d gv[d n + i]
  * W^(d)_i, W^(d) = W with axis d's weight replaced by its derivative in mesh
@@ -126,6 +146,7 @@ int p3mk_assign_weighted(const p3mk_geom *g, int n, p3mk_psort *s, int mode, con
 int p3mk_adjoint_gather(const p3mk_geom *g, int ad, int n, const p3mk_psort *s, const double *q,
                         const double *gv, void *const F[3], const void *lam, double prefac,
                         const double *selfb, double *dpos, double *dq, p3mk_queue *q_);
+/* ik back-interpolation: fk[d*n + i] += -prefac * sum W F_d (meshes F[0..2]) */
 int p3mk_interp_ik(const p3mk_geom *g, int n, const p3mk_psort *s, void *const F[3],
                    double prefac, double *fk, p3mk_queue *qu);
 /* ad back-interpolation: fk -= prefac * sum phi dQ; with selfb (81 FP64 on
@@ -185,6 +206,16 @@ void p3mk_cells_destroy(p3mk_cells *c);
 int p3mk_realspace(p3mk_cells *c, int n, double L, const double *x, const double *y,
                    const double *z, const double *q, double rcut, double alpha, int fp32,
                    double *fr, double *energy, p3mk_queue *qu);
+/* p3mk_realspace in three parts, for Calculate_forces: ranges to zero-fill
+ * first (at most 2; returns their number), the pairs, and where the forces
+ * then are: in sorted order (*pos, *fs for p3mk_finish_forces) when
+ * p3mk_realspace_sorted, else added to fr (zero-filled by the caller) */
+int p3mk_realspace_sorted(const p3mk_cells *c);
+int p3mk_realspace_ranges(p3mk_cells *c, int n, p3mk_range r[2]);
+int p3mk_realspace_filled(p3mk_cells *c, int n, double L, const double *x, const double *y,
+                          const double *z, const double *q, double rcut, double alpha, int fp32,
+                          double *fr, double *energy, const int **pos, const double **fs,
+                          p3mk_queue *qu);
 /* adjoint over the same pairs (FP64): for the cotangent g (3n) of the
  * real-space force, dpos (3n) += d/d pos and dq (n) += d/d q of sum g . f_r */
 int p3mk_realspace_vjp(p3mk_cells *c, int n, double L, const double *x, const double *y,
@@ -216,9 +247,11 @@ int p3mk_batch_info(const p3mk_batch *b, int *ntot, long *ntiles, long *ncell, i
 /* fk (3 blocks of ntot) += k-space force; ftot -= self force when enabled */
 int p3mk_batch_kspace(p3mk_batch *b, const double *x, const double *y, const double *z,
                       const double *q, double *fk, double *ftot, p3mk_queue *q_);
-/* fr (3 blocks of ntot) += real-space force; energy[s] += system energy */
-int p3mk_batch_realspace(p3mk_batch *b, const double *x, const double *y, const double *z,
-                         const double *q, double *fr, double *energy, p3mk_queue *q_);
+/* Calculate_forces of every system: f, fk, fr (3 blocks of ntot) and energy
+ * (nsys, may be NULL) are written; real: any system has a real-space part */
+int p3mk_batch_forces(p3mk_batch *b, int real, const double *x, const double *y, const double *z,
+                      const double *q, double *f, double *fk, double *fr, double *energy,
+                      p3mk_queue *q_);
 /* record events P3MK_EV_PAIRS, +1 around the batched half-shell kernel in
  * the following calls (on != 0); not for calls captured into a graph */
 int p3mk_batch_time_pairs(p3mk_batch *b, int on);

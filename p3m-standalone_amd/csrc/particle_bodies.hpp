@@ -35,6 +35,38 @@ __device__ __forceinline__ long item_tile(const int *__restrict__ cstart, long n
     return lo;
 }
 
+// f(lx, ly, lz, g) for every point of a tile's halo region of side R <= 16 at
+// (t0x, t0y, t0z), g its mesh index (periodic wrap): 16 lanes along z, the
+// workgroup's rows of 16 lanes over the region's rows, with no division (the
+// index arithmetic of a flat loop over R^3 points, six divisions by run-time
+// values a point, cost more than a sparse tile's stencils).
+template <typename F>
+__device__ __forceinline__ void for_region(int R, int M, int t0x, int t0y, int t0z, F &&f) {
+    const int lz = threadIdx.x & 15, step = (int)blockDim.x >> 4;
+    int gz = t0z + lz;
+    while (gz >= M)
+        gz -= M;
+    int lx = 0, ly = (int)threadIdx.x >> 4;
+    while (ly >= R) {
+        ly -= R;
+        lx++;
+    }
+    while (lx < R) {
+        int gx = t0x + lx, gy = t0y + ly;
+        while (gx >= M)
+            gx -= M;
+        while (gy >= M)
+            gy -= M;
+        if (lz < R)
+            f(lx, ly, lz, (long)(gx * M + gy) * M + gz);
+        ly += step;
+        while (ly >= R) {
+            ly -= R;
+            lx++;
+        }
+    }
+}
+
 // What a particle deposits (MODE): kCharge q W; kWeighted q g_i W with a
 // per-particle factor g (the adjoint's q g_d); kDipole
 // q sum_d g_{i,d} W^(d), W^(d) = W with the d-axis weight replaced by its
@@ -217,19 +249,15 @@ assign_rows_item(const double4 *__restrict__ sorted, int pb, int pe, long tl, in
             __syncthreads();
         }
         // add the region to mesh ii (periodic wrap of the halo)
-        const int R = rg.R;
-        for (int k = threadIdx.x; k < R * R * R; k += blockDim.x) {
-            const int lz = k % R, ly = (k / R) % R, lx = k / (R * R);
+        for_region(rg.R, M, t0x, t0y, t0z, [&](int lx, int ly, int lz, long g) {
             const T v = (T)acc[lx * rg.Sx + ly * rg.Sy + lz];
             if (v != T(0)) {
-                const int gx = (t0x + lx) % M, gy = (t0y + ly) % M, gz = (t0z + lz) % M;
-                const long g = ((long)gx * M + gy) * M + gz;
                 if (R2C)
                     atomicAdd(&mesh[g], v);
                 else
                     atomicAdd(&mesh[2 * g + ii], v);
             }
-        }
+        });
         __syncthreads();
     }
 }
@@ -324,10 +352,8 @@ assign_item(const double4 *__restrict__ sorted, int pb, int pe, long tl, int nt,
     }
     __syncthreads();
     // add the region to the mesh (periodic wrap of the halo)
-    for (int k = threadIdx.x; k < npts; k += blockDim.x) {
-        const int lz = k % R, ly = (k / R) % R, lx = k / (R * R);
-        const int gx = (t0x + lx) % M, gy = (t0y + ly) % M, gz = (t0z + lz) % M;
-        const long g = ((long)gx * M + gy) * M + gz;
+    for_region(R, M, t0x, t0y, t0z, [&](int lx, int ly, int lz, long g) {
+        const int k = (lx * R + ly) * R + lz;
 #pragma unroll
         for (int ii = 0; ii < NM; ii++) {
             const T v = (T)acc[ii * npts + k];
@@ -338,7 +364,7 @@ assign_item(const double4 *__restrict__ sorted, int pb, int pe, long tl, int nt,
                     atomicAdd(&mesh[2 * g + ii], v);
             }
         }
-    }
+    });
 }
 
 // ---- back-interpolation -----------------------------------------------------
@@ -380,10 +406,8 @@ interp_ik_item(const double4 *__restrict__ sorted, const int *__restrict__ perm,
     const double sc = (IL ? 0.5 * prefac : prefac) * stencil_norm<P>;
     for (int d = 0; d < 3; d++) {
         const T *F = d == 0 ? F0 : (d == 1 ? F1 : F2);
-        for (int k = threadIdx.x; k < npts; k += blockDim.x) {
-            const int lz = k % R, ly = (k / R) % R, lx = k / (R * R);
-            const int gx = (t0x + lx) % M, gy = (t0y + ly) % M, gz = (t0z + lz) % M;
-            const long g = ((long)gx * M + gy) * M + gz;
+        for_region(R, M, t0x, t0y, t0z, [&](int lx, int ly, int lz, long g) {
+            const int k = (lx * R + ly) * R + lz;
             if (R2C) {
                 lds[k] = F[g];
             } else {
@@ -391,7 +415,7 @@ interp_ik_item(const double4 *__restrict__ sorted, const int *__restrict__ perm,
                 if (IL)
                     lds[npts + k] = F[2 * g + 1];
             }
-        }
+        });
         __syncthreads();
         for (int p = pb + threadIdx.x; p < pe; p += blockDim.x) {
             const double4 r = sorted[p];
@@ -454,10 +478,8 @@ interp_ad_item(const double4 *__restrict__ sorted, const int *__restrict__ perm,
     const int npts = R * R * R;
     const int tz = (int)(tl % nt), ty = (int)((tl / nt) % nt), tx = (int)(tl / ((long)nt * nt));
     const int t0x = tx * Tt, t0y = ty * Tt, t0z = tz * Tt;
-    for (int k = threadIdx.x; k < npts; k += blockDim.x) {
-        const int lz = k % R, ly = (k / R) % R, lx = k / (R * R);
-        const int gx = (t0x + lx) % M, gy = (t0y + ly) % M, gz = (t0z + lz) % M;
-        const long g = ((long)gx * M + gy) * M + gz;
+    for_region(R, M, t0x, t0y, t0z, [&](int lx, int ly, int lz, long g) {
+        const int k = (lx * R + ly) * R + lz;
         if (R2C) {
             lds[k] = phi[g];
         } else {
@@ -465,7 +487,7 @@ interp_ad_item(const double4 *__restrict__ sorted, const int *__restrict__ perm,
             if (IL)
                 lds[npts + k] = phi[2 * g + 1];
         }
-    }
+    });
     __syncthreads();
     for (int p = pb + threadIdx.x; p < pe; p += blockDim.x) {
         const double4 r = sorted[p];

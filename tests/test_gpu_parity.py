@@ -442,6 +442,42 @@ def test_fft_r2c_zy_vs_numpy(pkg, M, fp32):
         rig.close()
 
 
+@pytest.mark.parametrize("method,n,L,M,cao,rcut", [
+    (2, 333, 8.0, 16, 5, 3.9),    # nearest images (no cell grid), self force, ragged sizes
+    (7, 1001, 30.0, 32, 4, 3.0),  # cell grid, self force, r2c
+    (0, 501, 12.0, 18, 3, 0.0),   # no real space
+    (1, 4097, 60.0, 36, 3, 3.0),  # 8000 cells (items by separate launches)
+    (3, 777, 20.0, 140, 3, 3.0),  # 5832 mesh tiles (items by separate launches)
+])
+def test_calculate_forces_writes_everything(pkg, orc, method, n, L, M, cao, rcut):
+    """Calculate_forces on device arrays that start as NaN: f, f_k, f_r and
+    the energy are written whole, twice in a row, as the oracle has them."""
+    import torch
+
+    alpha = 1.0
+    s = random_system(n, L, seed=n, charges="normal")
+    fk_ref, f_self = orc.kspace_force(method, s, M, cao, alpha)
+    fr_ref, e_ref = orc.realteil(s, rcut, alpha, cells=True) if rcut else (np.zeros((3, n)), 0.0)
+    solver = pkg.Solver(method, pkg.HostSystem.from_dict(s), pkg.parameters(M, cao, alpha, rcut))
+    dev = {k: torch.tensor(s[k], dtype=torch.float64, device="cuda") for k in "xyzq"}
+    f, fk, fr = (torch.full((3 * n,), float("nan"), dtype=torch.float64, device="cuda") for _ in range(3))
+    en = torch.full((1,), float("nan"), dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    for _ in range(2):
+        solver.calculate_forces_device(n, L, *[dev[k].data_ptr() for k in "xyzq"], rcut, alpha,
+                                       f.data_ptr(), fk.data_ptr(), fr.data_ptr(), en.data_ptr())
+    solver.synchronize()
+    got = [t.cpu().numpy().reshape(3, n) for t in (f, fk, fr)]
+    assert rel_err(got[1], fk_ref) < 1e-12
+    assert rel_err(got[0], f_self + (fk_ref + fr_ref)) < 1e-12
+    if rcut:
+        assert rel_err(got[2], fr_ref) < 1e-13
+        assert abs(en.item() - e_ref) <= 1e-12 * abs(e_ref)
+    else:
+        assert not got[2].any() and en.item() == 0.0
+    solver.close()
+
+
 @pytest.mark.parametrize("fp32", [0, 1])
 @pytest.mark.parametrize("M", [4, 6, 10, 14, 26, 32, 50, 90, 104, 112, 120, 150, 156, 160, 162, 220, 256])
 def test_fft_factor_splits(pkg, M, fp32):
