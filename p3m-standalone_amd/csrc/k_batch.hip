@@ -100,7 +100,7 @@ int build_descriptors(p3mk_batch *b) {
         tiles += (long)S.nt * S.nt * S.nt;
         items += (S.n + part::kChunk - 1) / part::kChunk + (long)S.nt * S.nt * S.nt;
         const int R = S.T + S.cao - 1 + (b->form.interlaced ? 1 : 0);
-        lds_a = std::max(lds_a, sizeof(double) * NM * (size_t)R * R * R);
+        lds_a = std::max(lds_a, (b->form.fp32 ? sizeof(float) : sizeof(double)) * NM * (size_t)R * R * R);
         const part::RowRegion rg = part::row_region(S.T, S.cao, b->form.interlaced != 0);
         lds_r = std::max(lds_r, sizeof(double) * (size_t)rg.size +
                                     (size_t)(part::kThreads / 64) *
