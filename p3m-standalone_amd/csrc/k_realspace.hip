@@ -538,8 +538,8 @@ __device__ __forceinline__ int next_item(int *counter, Claims &c) {
     return c.next++;
 }
 
-// Units of the half shell per work item: when the items are fewer than the
-// GPU has wavefront slots, an item's neighbour cells are dealt out to
+// Units per work item: when the items are fewer than the GPU has wavefront
+// slots, an item's neighbour cells are dealt out to
 // 2^split_bits wavefronts (each walks every 2^split_bits-th live cell and
 // adds its share of the forces), so that a small system's chain of windows
 // is shared.  With the first claims by block index, whole steps: 1,000
@@ -649,7 +649,7 @@ realspace_item(int home, int chunk, int cell0, const double4 *__restrict__ sorte
                const float4 *__restrict__ sorted32, const int *__restrict__ perm,
                const int *__restrict__ start, const int *__restrict__ istart,
                const float4 *__restrict__ bbox, int nc, int reach, double L, double rcut,
-               double alpha, long stride, double *__restrict__ fr,
+               double alpha, long stride, int split_bits, int part, double *__restrict__ fr,
                RsShared<FP32, VJP> &sh, double &en_tot, const double4 *__restrict__ gsorted = nullptr,
                double *__restrict__ dq = nullptr) {
     static_assert(!(VJP && FP32), "the adjoint is FP64");
@@ -747,7 +747,7 @@ realspace_item(int home, int chunk, int cell0, const double4 *__restrict__ sorte
         const double Li = 1.0 / L;
         const double rc2 = rcut * rcut * (1.0 + 1e-12);
         const int ncell = nc * nc * nc;
-        for (int cl = 0; cl < ncell; cl++) {
+        for (int cl = part; cl < ncell; cl += 1 << split_bits) {
             const int cell = cell0 + cl;
             const int jb = __builtin_amdgcn_readfirstlane(start[cell]);
             const int je = __builtin_amdgcn_readfirstlane(start[cell + 1]);
@@ -777,6 +777,7 @@ realspace_item(int home, int chunk, int cell0, const double4 *__restrict__ sorte
         // this lane's home particle relative to the home cell centre (inactive
         // lanes far away)
         const float4 hl = active ? sorted32[i] : make_float4(-2e30f, -2e30f, -2e30f, 0.0f);
+        int visit = 0; // cells are dealt to the item's units in turn
         for (int a = -reach; a <= reach; a++) {
             int cx = hx + a, wx = 0;
             if (cx < 0) { cx += nc; wx = -1; } else if (cx >= nc) { cx -= nc; wx = 1; }
@@ -789,6 +790,8 @@ realspace_item(int home, int chunk, int cell0, const double4 *__restrict__ sorte
                 if (gx * gx + gy * gy > rskip2)
                     continue;
                 for (int c = -reach; c <= reach; c++) {
+                    if ((visit++ & ((1 << split_bits) - 1)) != part)
+                        continue;
                     int cz = hz + c, wz = 0;
                     if (cz < 0) { cz += nc; wz = -1; } else if (cz >= nc) { cz -= nc; wz = 1; }
                     const float gz = gap(hlo.z, hhi.z, (float)((hz + c) * side), (float)((hz + c + 1) * side));
@@ -849,14 +852,16 @@ k_realspace(int n, const double4 *__restrict__ sorted, const float4 *__restrict_
     const int total = istart[ncell];
     double en_tot = 0.0;
     load_erfcx_table(sh);
-    Claims claims = first_claim(total);
+    const int sb = split_bits_of(total);
+    Claims claims = first_claim(total << sb);
     for (;;) {
-        const int item = next_item(counter, claims);
-        if (item >= total)
+        const int unit = next_item(counter, claims);
+        if (unit >= claims.total)
             break;
+        const int item = unit >> sb, part = unit & ((1 << sb) - 1);
         const int home = __float_as_int(bbox[2 * item].w), chunk = __float_as_int(bbox[2 * item + 1].w);
         realspace_item<FP32, SMALL_BOX>(home, chunk, 0, sorted, sorted32, perm,
-                                        start, istart, bbox, nc, reach, L, rcut, alpha, n, fr, sh,
+                                        start, istart, bbox, nc, reach, L, rcut, alpha, n, sb, part, fr, sh,
                                         en_tot);
     }
     if (energy != nullptr) {
@@ -882,15 +887,17 @@ k_realspace_vjp(int n, const double4 *__restrict__ sorted, const float4 *__restr
     const int total = istart[ncell];
     double en_unused = 0.0;
     load_erfcx_table(sh);
-    Claims claims = first_claim(total);
+    const int sb = split_bits_of(total);
+    Claims claims = first_claim(total << sb);
     for (;;) {
-        const int item = next_item(counter, claims);
-        if (item >= total)
+        const int unit = next_item(counter, claims);
+        if (unit >= claims.total)
             break;
+        const int item = unit >> sb, part = unit & ((1 << sb) - 1);
         const int home = __float_as_int(bbox[2 * item].w), chunk = __float_as_int(bbox[2 * item + 1].w);
         realspace_item<false, SMALL_BOX, true>(home, chunk, 0, sorted, sorted32,
                                                perm, start, istart, bbox, nc, reach, L, rcut, alpha,
-                                               n, dpos, sh, en_unused, gsorted, dq);
+                                               n, sb, part, dpos, sh, en_unused, gsorted, dq);
     }
 }
 
@@ -1719,7 +1726,7 @@ extern "C" int p3mk_realspace_vjp(p3mk_cells *c, int n, double L, const double *
     P3MK_TRY(p3mk_fill_zero_many(1, &counts, qu));
     P3MK_TRY(build_cells(c, n, L, x, y, z, q, rcut, g, qu));
     const bool all_cells = (2 * c->reach + 1 > c->nc);
-    const dim3 grid((unsigned)std::min<long>(c->grid, a.max_items));
+    const dim3 grid((unsigned)std::min<long>(c->grid, a.max_items << kMaxSplitBits));
     hipStream_t s = p3mk_stream(qu);
     if (all_cells)
         hipLaunchKernelGGL(k_realspace_vjp<true>, grid, dim3(kWave), 0, s, n, a.sorted, a.sorted32,
@@ -1773,8 +1780,8 @@ extern "C" int p3mk_realspace_filled(p3mk_cells *c, int n, double L, const doubl
     CellArrays &a = c->a;
     hipStream_t s = p3mk_stream(qu);
     const bool all_cells = (2 * c->reach + 1 > c->nc);
-    // no more wavefronts than units (half shell) or items can be
-    const long units = all_cells ? a.max_items : a.max_items << kMaxSplitBits;
+    // no more wavefronts than there can be units
+    const long units = a.max_items << kMaxSplitBits;
     const dim3 grid((unsigned)std::min<long>(c->grid, units));
     if (!all_cells) {
         // half shell: forces summed in sorted order
@@ -1869,11 +1876,13 @@ k_brealspace(const BSys *__restrict__ sys, const int *__restrict__ cell0s, int n
     __shared__ RsShared<FP32> sh;
     const int total = istart[ncell];
     load_erfcx_table(sh);
-    Claims claims = first_claim(total);
+    const int sb = split_bits_of(total);
+    Claims claims = first_claim(total << sb);
     for (;;) {
-        const int item = next_item(counter, claims);
-        if (item >= total)
+        const int unit = next_item(counter, claims);
+        if (unit >= claims.total)
             break;
+        const int item = unit >> sb, part = unit & ((1 << sb) - 1);
         const int home = __float_as_int(bbox[2 * item].w), chunk = __float_as_int(bbox[2 * item + 1].w);
         const int s = p3m::fft::prefix_slot(cell0s, nsys, (long)home);
         const BSys &S = sys[s];
@@ -1882,7 +1891,7 @@ k_brealspace(const BSys *__restrict__ sys, const int *__restrict__ cell0s, int n
         double en = 0.0;
         realspace_item<FP32, true>(home - S.cell0, chunk, S.cell0, sorted, sorted32,
                                    perm, start, istart, bbox, S.nc, S.reach, S.L, S.rcut, S.alpha, ntot,
-                                   fr, sh, en);
+                                   sb, part, fr, sh, en);
         if (energy != nullptr) {
             for (int off = 32; off > 0; off >>= 1)
                 en += __shfl_down(en, off, kWave);

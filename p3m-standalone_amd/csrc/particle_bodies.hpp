@@ -453,6 +453,28 @@ interp_ik_item(const double4 *__restrict__ sorted, const int *__restrict__ perm,
     }
 }
 
+// Phases exp(2 pi i m'.u), u = r / h, of the self-force sums over m' in
+// {-1, 0, 1}^3: three sincos and products in place of a sine per m', and half
+// of the m' (b(m') meets sin, odd, so m' and -m' go together).
+struct SelfPhases {
+    double2 p[3];
+    __device__ __forceinline__ SelfPhases(double ux, double uy, double uz) {
+        sincospi(2.0 * ux, &p[0].y, &p[0].x);
+        sincospi(2.0 * uy, &p[1].y, &p[1].x);
+        sincospi(2.0 * uz, &p[2].y, &p[2].x);
+    }
+    __device__ __forceinline__ double2 power(int d, int m) const {
+        return m == 0 ? make_double2(1.0, 0.0) : make_double2(p[d].x, m > 0 ? p[d].y : -p[d].y);
+    }
+    // f(3 index of m', 3 index of -m', phase of m') for the 13 m' > -m'
+    template <typename F> __device__ __forceinline__ void each(F &&f) const {
+        for (int k = 14; k < 27; k++) {
+            const int m0 = k / 9 - 1, m1 = (k / 3) % 3 - 1, m2 = k % 3 - 1;
+            f(3 * k, 3 * (26 - k), cmul(cmul(power(0, m0), power(1, m1)), power(2, m2)));
+        }
+    }
+};
+
 // ---- tile-staged ad back-interpolation ------------------------------------------
 //
 // A work item is a chunk of the particles of one mesh tile (as in assignment).
@@ -535,17 +557,13 @@ interp_ad_item(const double4 *__restrict__ sorted, const int *__restrict__ perm,
             // f -= sum_m' b(m') q^2 sin(2 pi m'.r / h)  (p3m-ad-self-forces.c:122-135)
             const double q2 = r.w * r.w;
             double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-            int ind = 0;
-            for (int m0 = -1; m0 <= 1; m0++)
-                for (int m1 = -1; m1 <= 1; m1++)
-                    for (int m2 = -1; m2 <= 1; m2++) {
-                        const double st = q2 * sin(2 * 3.14159265358979323846 *
-                                                   (m0 * r.x / h + m1 * r.y / h + m2 * r.z / h));
-                        s0 += selfb[ind] * st;
-                        s1 += selfb[ind + 1] * st;
-                        s2 += selfb[ind + 2] * st;
-                        ind += 3;
-                    }
+            SelfPhases ph(r.x / h, r.y / h, r.z / h);
+            ph.each([&](int ind, int neg, double2 e) {
+                const double st = q2 * e.y;
+                s0 += (selfb[ind] - selfb[neg]) * st;
+                s1 += (selfb[ind + 1] - selfb[neg + 1]) * st;
+                s2 += (selfb[ind + 2] - selfb[neg + 2]) * st;
+            });
             f[i] -= s0;
             f[stride + i] -= s1;
             f[2 * stride + i] -= s2;
