@@ -60,8 +60,11 @@ constexpr int kWave = 64;
 // full-shell kernels (nearest images, adjoint): at most 63 pending pairs plus
 // one append of the vector search
 constexpr int kQueue = 2 * kWave;
-// work-item counters of a cell list (one per kernel launched on it)
-constexpr int kCounters = 4;
+// work-item counters of a cell list: kClaimGroups per kernel launched on it
+// (at most two), in cache lines of their own
+constexpr int kClaimGroups = 8, kClaimStride = 32;
+constexpr int kKernelCounters = kClaimGroups * kClaimStride;
+constexpr int kCounters = 2 * kKernelCounters;
 // sorted arrays carry kPad zero-charge entries past the last particle
 constexpr int kPad = 64;
 // home cells of more particles than this use the matrix-core candidate search
@@ -502,12 +505,13 @@ __device__ __forceinline__ void load_erfcx_table(RsShared<FP32, VJP> &sh) {
 
 // Work-item claims of the persistent grids: a claim takes `per` consecutive
 // items.  A wavefront's first claim is its block index (no memory access),
-// the later ones take a device atomic on the shared counter, which counts
-// from the grid's first claims on.  The counter is a serial point (about
-// 18 ns an atomic): with a first claim by atomic, the 8192 wavefronts of the
-// grid took 150 us for that alone, whatever the system.  per = total /
-// (8 grid), at least 1, leaves a wavefront about eight claims, for the
-// balance of clustered systems.
+// the later ones take a device atomic.  One counter is a serial point (about
+// 18 ns an atomic: 8192 first claims, or 8192 last ones that find nothing,
+// take 150 us), so the wavefronts are in kClaimGroups groups by block index,
+// each with a counter in a cache line of its own and every kClaimGroups-th
+// claim of the rest of the items, which are interleaved finely enough for the
+// groups to end together.  per = total / (8 grid), at least 1, leaves a
+// wavefront about eight claims, for the balance of clustered systems.
 struct Claims {
     int next, end, per, total;
 };
@@ -523,16 +527,19 @@ __device__ __forceinline__ Claims first_claim(int total) {
 // this wavefront's next item, total when the items are exhausted
 __device__ __forceinline__ int next_item(int *counter, Claims &c) {
     if (c.next >= c.end) {
-        const int given = (int)gridDim.x * c.per; // by block index
+        const long given = (long)gridDim.x * c.per; // by block index
         if (given >= c.total || c.next >= c.total)
             return c.total;
-        int first = 0;
+        const int groups = (int)gridDim.x >= kClaimGroups ? kClaimGroups : 1;
+        const int group = (int)blockIdx.x % groups;
+        int k = 0;
         if (threadIdx.x == 0)
-            first = atomicAdd(counter, c.per);
-        first = __builtin_amdgcn_readfirstlane(first);
-        if (first >= c.total - given)
+            k = atomicAdd(counter + group * kClaimStride, 1);
+        k = __builtin_amdgcn_readfirstlane(k);
+        const long first = given + ((long)k * groups + group) * c.per;
+        if (first >= c.total)
             return c.total;
-        c.next = given + first;
+        c.next = (int)first;
         c.end = min(c.total, c.next + c.per);
     }
     return c.next++;
@@ -547,7 +554,7 @@ __device__ __forceinline__ int next_item(int *counter, Claims &c) {
 // 240 -> 154 us, a batch of 24 small systems 542 -> 455 us; a million
 // particles 6.26 -> 6.15 ms.
 constexpr int kMaxSplitBits = 4;
-constexpr int kSplitUnits = 4096; // about the resident wavefronts
+constexpr int kSplitUnits = 1024; // a wavefront per SIMD; 4096 took 78 us where 1024 took 57 (32,768 particles FP64)
 __device__ __forceinline__ int split_bits_of(int total) {
     int b = 0;
     while (b < kMaxSplitBits && (total << b) < kSplitUnits)
@@ -1587,8 +1594,8 @@ int cells_alloc(CellArrays &a, long n, long ncell) {
     int rc = P3MK_OK;
     if (rc == P3MK_OK) rc = p3mk_alloc((void **)&a.key, sizeof(int) * nn);
     // fcount and the work-item counters in one allocation, cleared by one
-    // fill: [fcount | counters], fcount a multiple of 16 bytes
-    const size_t nf4 = (nf + 3) & ~(size_t)3;
+    // fill: [fcount | counters], the counters from a cache line on
+    const size_t nf4 = (nf + kClaimStride - 1) / kClaimStride * kClaimStride;
     if (rc == P3MK_OK) rc = p3mk_alloc((void **)&a.fcount, sizeof(int) * (nf4 + kCounters));
     if (rc == P3MK_OK)
         a.counter = a.fcount + nf4;
@@ -1996,11 +2003,11 @@ int brs_forces(const BForm &f, const BSys *sys, const int *psys, const int *cell
         if (f.fp32)
             hipLaunchKernelGGL(k_brealspace_half<true>, dim3((unsigned)grid), dim3(kWave), 0, s, sys,
                                cell0s, nsys, ntot, a.sorted, a.sorted32, a.sortedq, a.start, a.istart, a.bbox, ncell,
-                               a.counter + 1, a.fsorted, energy);
+                               a.counter + kKernelCounters, a.fsorted, energy);
         else
             hipLaunchKernelGGL(k_brealspace_half<false>, dim3((unsigned)grid), dim3(kWave), 0, s, sys,
                                cell0s, nsys, ntot, a.sorted, a.sorted32, a.sortedq, a.start, a.istart, a.bbox, ncell,
-                               a.counter + 1, a.fsorted, energy);
+                               a.counter + kKernelCounters, a.fsorted, energy);
         P3MK_TRY(p3mk_launch_check("batched real space (half shell)"));
         if (time_pairs)
             P3MK_TRY(p3mk_record(qu, P3MK_EV_PAIRS + 1));
