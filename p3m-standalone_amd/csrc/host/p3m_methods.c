@@ -138,7 +138,7 @@ static int check_params(int id, const system_t *s, const parameters_t *p) {
  * system has.  1 without positions.  Only the real-space cell size depends
  * on it, never a result. */
 #define CLUSTER_GRID 16
-#define CLUSTER_SAMPLE 16384
+#define CLUSTER_SAMPLE 4096
 static double clustering_of(const system_t *s) {
     int count[CLUSTER_GRID * CLUSTER_GRID * CLUSTER_GRID] = {0};
     const int cells = CLUSTER_GRID * CLUSTER_GRID * CLUSTER_GRID;
