@@ -1064,12 +1064,9 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
     // test runs on the FP64 positions.  The relative error of d is at most
     // 2 u + sqrt(3) s / r, r >= rcut / 16 (below, u).  The pair
     // arithmetic runs in units of s: D = d / s, the window charge staged as
-    // q 2^(2 fb) (a power of two: a rounded 1 / s^2 scales every force by its
-    // error), alpha and 2 alpha / sqrt(pi) taken times s, so that the sums of
-    // (q_i q_j 2^(2 fb))(erfc(alpha s R) / R + 2 alpha s e^{-alpha^2 s^2 R^2} / sqrt(pi)) D / R^2
-    // are side^2 times the force; they are divided by it in FP64 when a
-    // particle's sum is done, and the energy sum, side 2^fb times the energy,
-    // once per item.
+    // q / s^2, alpha and 2 alpha / sqrt(pi) taken times s, so that
+    // (q_i q_j / s^2)(erfc(alpha s R) / R + 2 alpha s e^{-alpha^2 s^2 R^2} / sqrt(pi)) D / R^2
+    // is the force, and the energy sum, in units of 1 / s, is scaled once.
     const int fb = fix_bits(reach);
     const double quantum = ldexp(side, -fb);
     const double band = 4.0 * (3.4642 * quantum / rcut + 8.0 * 0x1p-24);
@@ -1078,7 +1075,7 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
     // Pairs closer than rcut / 16 (one in 4096 of a uniform system) take
     // their difference from the FP64 positions too: below that distance the
     // quantum's sqrt(3) s / r would exceed FP32's rounding.
-    const double inv_quantum = 1.0 / quantum, inv_side_sq = 1.0 / (side * side);
+    const double inv_quantum = ldexp(1.0, fb) / side;
     const float r2_close = (float)(rq2 * (1.0 / 256.0));
     const double alpha_q = alpha * quantum, two_a_spi_q = two_a_spi * quantum;
     // one queued pair: what a round reads before its arithmetic (FP32: the
@@ -1321,7 +1318,7 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
             for (int d = 0; d < 3; d++) {
                 const double v = sh.facc_nb[d][lane];
                 if (v != 0.0)
-                    atomicAdd(&fs[d * stride + j], FP32 ? -v * inv_side_sq : -v);
+                    atomicAdd(&fs[d * stride + j], -v);
                 sh.facc_nb[d][lane] = 0.0;
             }
         }
@@ -1399,7 +1396,7 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
     // (a, b, c) sides, exactly 2^fb quanta each (the image shift w L is the
     // whole-mesh part of it), so a window particle's fixed-point position in
     // the home frame is its own-cell one plus that integer offset
-    const float q_scale = ldexpf(1.0f, 2 * fb);
+    const float q_scale = (float)(inv_quantum * inv_quantum);
     const float side2 = (float)(2.0 * side);
     // the particles j (valid lanes) of cells with offsets and shift `info`
     // that are within rcut of the item's box, compacted into the window
@@ -1502,7 +1499,7 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
     if (w > 0)
         process_window();
     if (FP32)
-        en_tot += ldexp(1.0, -fb) / side * (double)en32;
+        en_tot += quantum * (double)en32;
     if (active) {
         double f0 = 0.0, f1 = 0.0, f2 = 0.0;
         for (int r = 0; r < orep; r++) {
@@ -1510,10 +1507,9 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
             f1 += sh.facc[1][lane + oslots * r];
             f2 += sh.facc[2][lane + oslots * r];
         }
-        const double unit = FP32 ? inv_side_sq : 1.0;
-        atomicAdd(&fs[i], f0 * unit);
-        atomicAdd(&fs[stride + i], f1 * unit);
-        atomicAdd(&fs[2 * stride + i], f2 * unit);
+        atomicAdd(&fs[i], f0);
+        atomicAdd(&fs[stride + i], f1);
+        atomicAdd(&fs[2 * stride + i], f2);
     }
     wave_sync();
 }
