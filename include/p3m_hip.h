@@ -231,7 +231,9 @@ enum {
 const char *p3m_hip_last_error(void);
 
 /* Init of method `method_id` with the given precision; *out receives the
- * data_t.  Replaces method.Init (p3m-common.c:145-232 + Init_*). */
+ * data_t.  Replaces method.Init (p3m-common.c:145-232 + Init_*).  Of s only
+ * the particle count and the box length are read: s->p and s->q may be NULL
+ * or hold device pointers for a program that keeps to the device calls. */
 int p3m_hip_init(int method_id, system_t *s, parameters_t *p, int precision, data_t **out);
 /* Influence_function with a status (p3m-ik.c:135-173, p3m-ik-i.c:126-166,
  * p3m-ad.c:111-158, p3m-ad-i.c:121-150). */
@@ -262,7 +264,10 @@ int p3m_hip_synchronize(data_t *d);
  * (rcut <= L/2).  f->f_r += forces, s->energy += energy. */
 int p3m_hip_realteil(system_t *s, parameters_t *p, forces_t *f);
 /* Device-resident real-space part: fr (3n) += forces; energy (device
- * double, may be NULL) += energy.  Uses the stream of d. */
+ * double, may be NULL) += energy.  Uses the stream of d.  The first
+ * real-space call for a box length and cutoff makes the cell list: it
+ * allocates, and waits for the stream to see how clustered the positions
+ * are (the cell size follows them, never a result). */
 int p3m_hip_realteil_device(data_t *d, int n, double length, const double *x, const double *y,
                             const double *z, const double *q, double rcut, double alpha,
                             double *fr, double *energy);

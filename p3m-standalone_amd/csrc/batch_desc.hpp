@@ -110,18 +110,27 @@ inline int zero_count_cursor(int *count, int *cursor, size_t m, p3mk_queue *qu) 
 // Gaussian of a million particles, 8 per cell on average and 90 in the
 // typical particle's, takes 6.05 ms with small cells, 6.9 with large ones:
 // so the mean is weighted with the clustering seen by a typical particle
-// (1 = uniform), estimated where positions are at hand when the list is made.
+// (1 = uniform), estimated from the positions the list is made for.
 constexpr double kSmallCellMinOccupancy = 12.0;
 constexpr int kMaxCellsPerSide = 512;
+
+inline int cells_per_side(double L, double side) { // with the margin of cell_geometry
+    return (int)std::min<double>(kMaxCellsPerSide, std::floor(L / side * (1.0 - 1e-12)));
+}
+
+// does a clustering above 1 change the cell size?
+inline bool cells_by_clustering(long n, double L, double rcut) {
+    const int nc2 = cells_per_side(L, 0.5 * rcut);
+    return cells_per_side(L, rcut) >= 3 && nc2 >= 5 &&
+           (double)n < kSmallCellMinOccupancy * nc2 * (double)nc2 * nc2;
+}
 
 // Cell grid of a real-space cell list for n particles: nc cells per side of
 // side >= rcut / reach, with a margin so that rounding of x nc / L never puts
 // a pair inside the cutoff more than `reach` cells apart.  Boxes of fewer than
 // 2 reach + 1 cells per side are left to the nearest-image search.
 inline void cell_geometry(long n, double L, double rcut, double clustering, int &nc, int &reach) {
-    const double margin = 1.0 - 1e-12;
-    const int nc2 = (int)std::min<double>(kMaxCellsPerSide, std::floor(L * 2.0 / rcut * margin));
-    const int nc1 = (int)std::min<double>(kMaxCellsPerSide, std::floor(L / rcut * margin));
+    const int nc2 = cells_per_side(L, 0.5 * rcut), nc1 = cells_per_side(L, rcut);
     const bool sparse = nc1 >= 3 && (double)n * clustering < kSmallCellMinOccupancy * nc2 * (double)nc2 * nc2;
     if (nc2 < 5 || sparse) {
         reach = 1;

@@ -10,6 +10,10 @@ int p3mh_fail(int code, const char *fmt, ...);
 /* p3mh_fail with the kernel layer's message appended */
 int p3mh_kfail(int code, const char *what);
 
+/* the cell list that the real-space calls on d use (NULL before the first) */
+struct p3mk_cells;
+const struct p3mk_cells *p3mh_cells(data_t *d);
+
 #define TRYK(expr, what)                          \
     do {                                          \
         int rc_ = (expr);                         \

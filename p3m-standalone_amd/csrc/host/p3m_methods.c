@@ -66,12 +66,12 @@ typedef struct {
     double *pos;    /* x, y, z, q blocks of n */
     double *force;  /* fk (3n), f (3n), fr (3n) */
     double *hforce; /* pinned staging, 9n */
+    double *hclust; /* pinned, one word: clustering of the positions */
     double *energy; /* device scalar */
     int *iscratch;
     p3mk_cells *cells;
     p3mk_psort *psort;
     double cells_L, cells_rc;
-    double clustering; /* of the positions given to Init */
     int have_G;
     int have_ks_events;
     int have_rs_events;
@@ -108,6 +108,7 @@ static void ctx_free(p3m_ctx *c) {
     p3mk_release(c->energy);
     p3mk_release(c->iscratch);
     p3mk_release_host(c->hforce);
+    p3mk_release_host(c->hclust);
     p3mk_cells_destroy(c->cells);
     p3mk_psort_destroy(c->psort);
     p3mk_queue_destroy(c->q);
@@ -131,35 +132,6 @@ static int check_params(int id, const system_t *s, const parameters_t *p) {
     if (!(s->length > 0.0) || !isfinite(s->length))
         return p3mh_fail(P3M_HIP_EINVAL, "box length must be positive");
     return P3M_HIP_OK;
-}
-
-/* Density a typical particle sees over the mean density: pairs of sampled
- * particles that share a cell of a 16^3 grid, over the number a uniform
- * system has.  1 without positions.  Only the real-space cell size depends
- * on it, never a result. */
-#define CLUSTER_GRID 16
-#define CLUSTER_SAMPLE 4096
-static double clustering_of(const system_t *s) {
-    int count[CLUSTER_GRID * CLUSTER_GRID * CLUSTER_GRID] = {0};
-    const int cells = CLUSTER_GRID * CLUSTER_GRID * CLUSTER_GRID;
-    int i, step, k;
-    double m = 0.0, pairs = 0.0, ratio;
-    if (s->p == NULL || s->p->x == NULL || s->p->y == NULL || s->p->z == NULL || s->nparticles < 2)
-        return 1.0;
-    step = (s->nparticles + CLUSTER_SAMPLE - 1) / CLUSTER_SAMPLE;
-    for (i = 0; i < s->nparticles; i += step) {
-        const double r[3] = {s->p->x[i] / s->length, s->p->y[i] / s->length, s->p->z[i] / s->length};
-        int cell = 0;
-        for (k = 0; k < 3; k++) {
-            const double u = r[k] - floor(r[k]);
-            const int c = u >= 0.0 && u < 1.0 ? (int)(u * CLUSTER_GRID) : 0; /* NaN: 0 */
-            cell = cell * CLUSTER_GRID + c;
-        }
-        pairs += 2.0 * count[cell]++;
-        m += 1.0;
-    }
-    ratio = pairs * cells / (m * (m - 1.0));
-    return ratio > 1.0 ? ratio : 1.0;
 }
 
 static int ctx_alloc(p3m_ctx *c) {
@@ -202,6 +174,7 @@ static int ctx_alloc(p3m_ctx *c) {
     TRYK(p3mk_alloc((void **)&c->energy, sizeof(double)), "energy");
     TRYK(p3mk_alloc((void **)&c->iscratch, sizeof(int) * 16), "int scratch");
     TRYK(p3mk_alloc_host((void **)&c->hforce, sizeof(double) * 9 * n), "pinned staging");
+    TRYK(p3mk_alloc_host((void **)&c->hclust, sizeof(double)), "pinned staging");
     TRYK(p3mk_fill_zero(c->selfb, sizeof(double) * 81, c->q), "zero");
     TRYK(p3mk_fill_zero(c->G, sizeof(double) * M3, c->q), "zero");
     TRYK(p3mk_queue_sync(c->q), "sync");
@@ -270,7 +243,6 @@ int p3m_hip_init(int method_id, system_t *s, parameters_t *p, int precision, dat
     c->geom.interlaced = is_interlaced(method_id);
     c->geom.fp32 = precision == P3M_HIP_MIXED;
     c->geom.L = s->length;
-    c->clustering = clustering_of(s);
     if (has_self_force(method_id)) {
         d->self_force_corrections = (double *)calloc(81, sizeof(double));
         if (d->self_force_corrections == NULL) {
@@ -542,23 +514,47 @@ int p3m_hip_get_self_force_coefficients(data_t *d, double *b) {
 /* Real space and Calculate_forces                                         */
 /* ---------------------------------------------------------------------- */
 
-static int ensure_cells(p3m_ctx *c, int n, double L, double rcut) {
+/* The cell list of a system of n particles; its cell size follows the
+ * clustering of the npos device positions at hand (no host array is read).
+ * Waits for the queue where the size depends on them.  word: pinned. */
+static int make_cells(p3mk_cells **cells, int n, double L, double rcut, int npos, const double *x,
+                      const double *y, const double *z, double *word, p3mk_queue *q) {
+    double clustering = 1.0;
+    if (p3mk_cells_by_clustering(n, L, rcut)) {
+        int rc = p3mk_clustering(npos, L, x, y, z, word, q);
+        if (rc == P3MK_OK)
+            rc = p3mk_queue_sync(q);
+        if (rc != P3MK_OK)
+            return rc;
+        clustering = *word;
+    }
+    return p3mk_cells_create(cells, n, L, rcut, clustering);
+}
+
+static int ensure_cells(p3m_ctx *c, double L, double rcut, int n, const double *x, const double *y,
+                        const double *z) {
     if (c->cells != NULL && c->cells_L == L && c->cells_rc == rcut)
         return P3M_HIP_OK;
     p3mk_cells_destroy(c->cells);
     c->cells = NULL;
-    TRYK(p3mk_cells_create(&c->cells, n, L, rcut, c->clustering), "cell list");
+    TRYK(make_cells(&c->cells, c->n, L, rcut, n, x, y, z, c->hclust, c->q), "cell list");
     c->cells_L = L;
     c->cells_rc = rcut;
     return P3M_HIP_OK;
 }
 
-static int prepare_realspace(p3m_ctx *c, int n, double length, double rcut) {
+const p3mk_cells *p3mh_cells(data_t *d) {
+    const p3m_ctx *c = ctx_of(d);
+    return c ? c->cells : NULL;
+}
+
+static int prepare_realspace(p3m_ctx *c, int n, double length, double rcut, const double *x,
+                             const double *y, const double *z) {
     if (n > c->n)
         return p3mh_fail(P3M_HIP_EINVAL, "more particles than Init's %d", c->n);
     if (!(rcut > 0.0) || rcut > 0.5 * length)
         return p3mh_fail(P3M_HIP_EINVAL, "real space needs 0 < rcut <= L/2");
-    return ensure_cells(c, c->n, length, rcut);
+    return ensure_cells(c, length, rcut, n, x, y, z);
 }
 
 int p3m_hip_realteil_device(data_t *d, int n, double length, const double *x, const double *y,
@@ -567,7 +563,7 @@ int p3m_hip_realteil_device(data_t *d, int n, double length, const double *x, co
     p3m_ctx *c = ctx_of(d);
     if (c == NULL)
         return p3mh_fail(P3M_HIP_EINVAL, "data_t was not made by p3m_hip_init");
-    TRY(prepare_realspace(c, n, length, rcut));
+    TRY(prepare_realspace(c, n, length, rcut, x, y, z));
     TRYK(p3mk_record(c->q, 4), "event");
     TRYK(p3mk_realspace(c->cells, n, length, x, y, z, q, rcut, alpha, c->geom.fp32, fr, energy,
                         c->q),
@@ -634,9 +630,9 @@ int p3m_hip_calculate_forces_device(data_t *d, int n, double length, const doubl
         return p3mh_fail(P3M_HIP_EINVAL, "force arrays must not be NULL");
     if (n != c->n)
         return p3mh_fail(P3M_HIP_EINVAL, "particle count %d differs from Init's %d", n, c->n);
-    if (rcut != 0.0)
-        TRY(prepare_realspace(c, n, length, rcut));
     TRY(check_kspace(c, n, length, f));
+    if (rcut != 0.0)
+        TRY(prepare_realspace(c, n, length, rcut, x, y, z));
     TRY(forces_enqueue(c, n, length, x, y, z, q, rcut, alpha, f, fk, fr, energy));
     if (c->ring_rs != NULL) {
         int k = p3mk_ring_filled(c->q);
@@ -752,7 +748,6 @@ int p3m_hip_realteil(system_t *s, parameters_t *p, forces_t *f) {
         if (r_ != P3MK_OK)                  \
             rc = p3mh_kfail(r_, what);           \
     }
-    CHK(p3mk_cells_create(&cells, (int)n, s->length, p->rcut, clustering_of(s)), "cell list");
     CHK(p3mk_alloc((void **)&pos, sizeof(double) * 4 * n), "positions");
     CHK(p3mk_alloc((void **)&fr, sizeof(double) * 3 * n), "forces");
     CHK(p3mk_alloc((void **)&en, sizeof(double)), "energy");
@@ -761,6 +756,7 @@ int p3m_hip_realteil(system_t *s, parameters_t *p, forces_t *f) {
     CHK(p3mk_copy_h2d(pos + n, s->p->y, sizeof(double) * n, q), "upload");
     CHK(p3mk_copy_h2d(pos + 2 * n, s->p->z, sizeof(double) * n, q), "upload");
     CHK(p3mk_copy_h2d(pos + 3 * n, s->q, sizeof(double) * n, q), "upload");
+    CHK(make_cells(&cells, (int)n, s->length, p->rcut, (int)n, pos, pos + n, pos + 2 * n, h, q), "cell list");
     CHK(p3mk_fill_zero(fr, sizeof(double) * 3 * n, q), "zero");
     CHK(p3mk_fill_zero(en, sizeof(double), q), "zero");
     CHK(p3mk_realspace(cells, (int)n, s->length, pos, pos + n, pos + 2 * n, pos + 3 * n, p->rcut,
@@ -792,11 +788,7 @@ int p3m_hip_realteil_vjp_device(data_t *d, int n, double length, const double *x
         return p3mh_fail(P3M_HIP_EINVAL, "data_t was not made by p3m_hip_init");
     if (gF == NULL || dpos == NULL || dq == NULL)
         return p3mh_fail(P3M_HIP_EINVAL, "cotangent and result arrays must not be NULL");
-    if (n > c->n)
-        return p3mh_fail(P3M_HIP_EINVAL, "more particles than Init's %d", c->n);
-    if (!(rcut > 0.0) || rcut > 0.5 * length)
-        return p3mh_fail(P3M_HIP_EINVAL, "real space needs 0 < rcut <= L/2");
-    TRY(ensure_cells(c, c->n, length, rcut));
+    TRY(prepare_realspace(c, n, length, rcut, x, y, z));
     TRYK(p3mk_realspace_vjp(c->cells, n, length, x, y, z, q, rcut, alpha, gF, dpos, dq, c->q),
          "real-space adjoint");
     return P3M_HIP_OK;
@@ -825,7 +817,6 @@ int p3m_hip_realteil_vjp(system_t *s, parameters_t *p, const vector_array_t *dF,
         if (r_ != P3MK_OK)                  \
             rc = p3mh_kfail(r_, what);      \
     }
-    CHK(p3mk_cells_create(&cells, (int)n, s->length, p->rcut, clustering_of(s)), "cell list");
     CHK(p3mk_alloc((void **)&pos, sizeof(double) * 4 * n), "positions");
     CHK(p3mk_alloc((void **)&g, sizeof(double) * 3 * n), "cotangent");
     CHK(p3mk_alloc((void **)&out, sizeof(double) * 4 * n), "adjoint");
@@ -834,6 +825,7 @@ int p3m_hip_realteil_vjp(system_t *s, parameters_t *p, const vector_array_t *dF,
     CHK(p3mk_copy_h2d(pos + n, s->p->y, sizeof(double) * n, q), "upload");
     CHK(p3mk_copy_h2d(pos + 2 * n, s->p->z, sizeof(double) * n, q), "upload");
     CHK(p3mk_copy_h2d(pos + 3 * n, s->q, sizeof(double) * n, q), "upload");
+    CHK(make_cells(&cells, (int)n, s->length, p->rcut, (int)n, pos, pos + n, pos + 2 * n, h, q), "cell list");
     for (dim = 0; dim < 3; dim++)
         CHK(p3mk_copy_h2d(g + dim * n, field((vector_array_t *)dF, dim), sizeof(double) * n, q),
             "upload");
@@ -887,7 +879,7 @@ int p3m_hip_calculate_forces(const method_t *m, system_t *s, parameters_t *p, da
         return p3mh_fail(P3M_HIP_EINVAL, "box length differs from the influence function's");
     TRY(upload_positions(c, s));
     if (p->rcut != 0.0) /* common.c:275-279 */
-        TRY(prepare_realspace(c, (int)n, s->length, p->rcut));
+        TRY(prepare_realspace(c, (int)n, s->length, p->rcut, c->pos, c->pos + n, c->pos + 2 * n));
     TRY(forces_enqueue(c, (int)n, s->length, c->pos, c->pos + n, c->pos + 2 * n, c->pos + 3 * n, p->rcut,
                        p->alpha, c->force + 3 * n, c->force, c->force + 6 * n, c->energy));
     TRYK(p3mk_copy_d2h(c->hforce, c->force, sizeof(double) * 9 * n, c->q), "download");

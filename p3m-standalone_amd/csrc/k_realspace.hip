@@ -1655,6 +1655,68 @@ struct p3mk_cells {
     int grid;
 };
 
+namespace {
+
+// Density a typical particle sees over the mean density: pairs of sampled
+// particles that share a cell of a 16^3 grid, over the number a uniform
+// system has.  One workgroup: 4096 reads of each coordinate, 5 us beside the
+// launch, when a cell list is made.
+constexpr int kClusterGrid = 16, kClusterCells = kClusterGrid * kClusterGrid * kClusterGrid;
+constexpr int kClusterSample = 4096, kClusterThreads = 1024;
+
+__global__ void __launch_bounds__(kClusterThreads)
+k_clustering(int n, double Li, const double *__restrict__ x, const double *__restrict__ y,
+             const double *__restrict__ z, double *out) {
+    __shared__ int count[kClusterCells];
+    __shared__ int part[kClusterThreads / 64];
+    for (int c = threadIdx.x; c < kClusterCells; c += kClusterThreads)
+        count[c] = 0;
+    __syncthreads();
+    const int step = (n - 1) / kClusterSample + 1, m = (n - 1) / step + 1;
+    int pairs = 0; // below 4096^2 / 2 in all
+    for (int k = threadIdx.x; k < m; k += kClusterThreads) {
+        const int i = k * step;
+        const double r[3] = {x[i] * Li, y[i] * Li, z[i] * Li};
+        int cell = 0;
+        for (int d = 0; d < 3; d++) {
+            const double u = r[d] - floor(r[d]);
+            cell = cell * kClusterGrid + (u >= 0.0 && u < 1.0 ? (int)(u * kClusterGrid) : 0); // NaN: 0
+        }
+        pairs += atomicAdd(&count[cell], 1);
+    }
+    for (int off = 32; off > 0; off >>= 1)
+        pairs += __shfl_down(pairs, off, 64);
+    if ((threadIdx.x & 63) == 0)
+        part[threadIdx.x >> 6] = pairs;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double sum = 0.0;
+        for (int w = 0; w < kClusterThreads / 64; w++)
+            sum += part[w];
+        *out = fmax(1.0, 2.0 * sum * kClusterCells / ((double)m * (m - 1.0)));
+    }
+}
+
+}  // namespace
+
+extern "C" int p3mk_clustering(int n, double L, const double *x, const double *y, const double *z, double *out,
+                               p3mk_queue *qu) {
+    *out = 1.0;
+    if (n < 2)
+        return P3MK_OK;
+    hipLaunchKernelGGL(k_clustering, dim3(1), dim3(kClusterThreads), 0, p3mk_stream(qu), n, 1.0 / L, x, y, z, out);
+    return p3mk_launch_check("clustering");
+}
+
+extern "C" int p3mk_cells_by_clustering(int n, double L, double rcut) {
+    return p3m::cells_by_clustering(n, L, rcut);
+}
+
+extern "C" void p3mk_cells_geometry(const p3mk_cells *c, int *nc, int *reach) {
+    *nc = c->nc;
+    *reach = c->reach;
+}
+
 extern "C" void p3mk_cells_destroy(p3mk_cells *c) {
     if (!c)
         return;

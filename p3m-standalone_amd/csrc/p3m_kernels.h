@@ -199,6 +199,14 @@ typedef struct p3mk_cells p3mk_cells; /* cell-list workspace */
 /* clustering: particles in a typical particle's neighbourhood over the mean
  * (1 for a uniform system); decides the cell size only */
 int p3mk_cells_create(p3mk_cells **c, int n, double L, double rcut, double clustering);
+/* does the cell size of a list for n particles depend on the clustering? */
+int p3mk_cells_by_clustering(int n, double L, double rcut);
+/* cells per side and their side in units of 1 / rcut (1 or 2) */
+void p3mk_cells_geometry(const p3mk_cells *c, int *nc, int *reach);
+/* clustering of n device positions to *out, host memory the device writes
+ * (p3mk_alloc_host); valid after p3mk_queue_sync */
+int p3mk_clustering(int n, double L, const double *x, const double *y, const double *z, double *out,
+                    p3mk_queue *qu);
 void p3mk_cells_destroy(p3mk_cells *c);
 /* fr += real-space force of every pair i != j with minimum-image distance
  * <= rcut; *energy (device, may be NULL) += energy.  fp32 selects the

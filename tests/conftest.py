@@ -1,3 +1,4 @@
+import ctypes
 import os
 import sys
 
@@ -77,6 +78,19 @@ def cell_geometry(n, L, rcut):
     if nc2 < 5 or (nc1 >= 3 and n < 6.0 * nc2 ** 3):
         return max(nc1, 1), 1
     return nc2, 2
+
+
+def cells_of(pkg, solver):
+    """(cells per side, reach) of the cell list the solver's real space uses."""
+    L = pkg.lib()
+    L.p3mh_cells.restype, L.p3mh_cells.argtypes = ctypes.c_void_p, [ctypes.c_void_p]
+    L.p3mk_cells_geometry.restype = None
+    L.p3mk_cells_geometry.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)]
+    cells = L.p3mh_cells(solver.d)
+    assert cells, "no real-space call yet"
+    nc, reach = ctypes.c_int(), ctypes.c_int()
+    L.p3mk_cells_geometry(cells, ctypes.byref(nc), ctypes.byref(reach))
+    return nc.value, reach.value
 
 
 def mixed_realspace_bound(s, rcut):

@@ -4,12 +4,13 @@ the reaction added to the partner) against the oracle's Realteil
 sparse ones, clusters that wrap across the periodic boundary, both cell
 sizes (side rcut / 2, and side rcut for sparse systems), the device entry
 point accumulating into the caller's arrays, and the mixed form."""
+import ctypes
 import math
 
 import numpy as np
 import pytest
 
-from conftest import cell_geometry, rel_err
+from conftest import cell_geometry, cells_of, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -298,4 +299,67 @@ def test_cell_size_follows_the_clustering(pkg, orc, layout, prec_name):
     err = rel_err(fr.cpu().numpy().reshape(3, n), fr_ref)
     print("%s %s rel err %.2e" % (layout, prec_name, err))
     assert err < (1e-13 if prec_name == "FP64" else 1e-6)
+    solver.close()
+
+
+def lattice(side, L, seed):
+    """side^3 particles in site order, jittered: no two closer than 0.4 sites."""
+    rng = np.random.default_rng(seed)
+    site = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    p = (site + 0.5 + 0.6 * (rng.uniform(size=site.shape) - 0.5)) * (L / side)
+    q = np.where(np.arange(len(p)) % 2 == 0, 1.0, -1.0)
+    return {"x": p[:, 0].copy(), "y": p[:, 1].copy(), "z": p[:, 2].copy(), "q": q, "L": float(L)}
+
+
+class DeviceRealteil:
+    """realteil_device of `solver` on device copies of a system."""
+
+    def __init__(self, solver, s, rcut, alpha):
+        import torch
+
+        self.solver, self.rcut, self.alpha = solver, rcut, alpha
+        self.n, self.L = len(s["q"]), s["L"]
+        self.dev = {k: torch.empty(self.n, dtype=torch.float64, device="cuda") for k in "xyzq"}
+        self.fr = torch.zeros(3 * self.n, dtype=torch.float64, device="cuda")
+        self.put(s)
+
+    def put(self, s):
+        import torch
+
+        self.solver.synchronize()
+        for k in "xyzq":
+            self.dev[k].copy_(torch.tensor(s[k]))
+        torch.cuda.synchronize()
+
+    def run(self, calls=1):
+        import torch
+
+        for _ in range(calls):
+            self.solver.realteil_device(self.n, self.L, *[self.dev[k].data_ptr() for k in "xyzq"], self.rcut,
+                                        self.alpha, self.fr.data_ptr(), None)
+        self.solver.synchronize()
+        out = self.fr.cpu().numpy().reshape(3, self.n).copy()
+        self.fr.zero_()
+        torch.cuda.synchronize()
+        return out
+
+
+@pytest.mark.parametrize("held", ["nothing", "unreadable", "zeros"])
+def test_init_reads_sizes_only(pkg, orc, held):
+    """Init takes the particle count and the box length of a system whose
+    arrays are absent, not readable by the host, or placeholders; the cell
+    size follows the positions of the first real-space call (uniform and
+    sparse here: side rcut)."""
+    rcut, alpha = 3.0, 1.0
+    s = lattice(12, 18.0, seed=3)
+    system = pkg.HostSystem.from_dict(dict(s, **{k: np.zeros_like(s[k]) for k in "xyz"}))
+    if held == "nothing":
+        system.c.p, system.c.q = None, None
+    elif held == "unreadable":
+        nowhere = ctypes.cast(ctypes.c_void_p(8), ctypes.POINTER(ctypes.c_double))
+        system.c.p.contents.x = system.c.p.contents.y = system.c.p.contents.z = system.c.q = nowhere
+    solver = pkg.Solver(7, system, pkg.parameters(16, 3, alpha, rcut))
+    fr = DeviceRealteil(solver, s, rcut, alpha).run()
+    assert cells_of(pkg, solver)[1] == 1
+    assert rel_err(fr, orc.realteil(s, rcut, alpha, cells=True)[0]) < 1e-13
     solver.close()
