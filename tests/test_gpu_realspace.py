@@ -363,3 +363,16 @@ def test_init_reads_sizes_only(pkg, orc, held):
     assert cells_of(pkg, solver)[1] == 1
     assert rel_err(fr, orc.realteil(s, rcut, alpha, cells=True)[0]) < 1e-13
     solver.close()
+
+
+@pytest.mark.parametrize("side", [32, 63, 64])
+def test_lattice_order_is_not_clustered(pkg, side):
+    """Particles in the site order of a lattice (the usual start of a
+    simulation), whose rows the sample's runs of side^3 / 4096 particles
+    divide or nearly divide: uniform, so cells of side rcut at 3.4 particles
+    per cell of side rcut / 2."""
+    s = lattice(side, float(side), seed=4)
+    solver = pkg.Solver(0, pkg.HostSystem.from_dict(s), pkg.parameters(16, 3, 1.0, 3.0))
+    DeviceRealteil(solver, s, 3.0, 1.0).run()
+    assert cells_of(pkg, solver)[1] == 1
+    solver.close()
