@@ -103,15 +103,18 @@ inline int zero_count_cursor(int *count, int *cursor, size_t m, p3mk_queue *qu) 
 
 // Below this number of particles in a typical particle's cell of side
 // rcut / 2 the cell list takes cells of side rcut instead: an item of a few
-// home particles spends more on its walk than on its pairs.  Measured, steps
-// with cells of side rcut against rcut / 2: 250,007 uniform particles FP64 at
-// 6.4 per cell 482 against 757 us, 100,000 mixed at 3.4 157 against 441 us;
-// at 16 per cell the two were equal and at 32 the small cells 10% faster.  A
-// Gaussian of a million particles, 8 per cell on average and 90 in the
-// typical particle's, takes 6.05 ms with small cells, 6.9 with large ones:
-// so the mean is weighted with the clustering seen by a typical particle
-// (1 = uniform), estimated from the positions the list is made for.
-constexpr double kSmallCellMinOccupancy = 12.0;
+// home particles spends more on its walk than on its pairs.  Measured, real
+// space of 200,000 uniform particles at rcut 3, cells of side rcut / 2 against
+// rcut, us: FP64 338 / 257 at 3.4 per cell, 376 / 386 at 6.4, 404 / 453 at 8,
+// 497 / 591 at 12; mixed 320 / 197, 297 / 259, 300 / 309 and 349 / 379.  The
+// batch crosses at the same place (32 systems of 8,000, step, FP64: 541 / 463
+// at 4, 581 / 595 at 6.4, 626 / 697 at 8).  In a clustered system the mean says
+// little (Gaussian particles, sigma an eighth of the box, real space FP64:
+// 428 / 396 at a mean of 0.3, 441 / 577 at 0.6), so it is weighted with the
+// clustering seen by a typical particle (1 = uniform; about 11.5 there),
+// estimated from the positions the list is made for.  A batch has no positions
+// when its list is made and goes by the mean.
+constexpr double kSmallCellMinOccupancy = 7.0;
 constexpr int kMaxCellsPerSide = 512;
 
 inline int cells_per_side(double L, double side) { // with the margin of cell_geometry

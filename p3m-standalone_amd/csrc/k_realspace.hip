@@ -7,9 +7,9 @@
 //
 // Layout: particles are folded into [0, L) and counting-sorted into cells of
 // side >= rcut/R (R = 2, or R = 1 when a typical particle's cell of side
-// rcut/2 would hold fewer than 12 particles or the box has fewer than 5 of
-// them per side; cell_geometry), and inside a cell by octant, so that 64 consecutive particles of a cell are spatially
-// compact.  A work item is (home cell, chunk of 64 home particles); a
+// rcut/2 would hold fewer than 7 particles or the box has fewer than 5 of
+// them per side; cell_geometry), and inside a cell by octant, so that 64
+// consecutive particles of a cell are spatially compact.  A work item is (home cell, chunk of 64 home particles); a
 // persistent grid of single-wavefront workgroups claims items from an
 // atomic counter, so the dense cells of a clustered system are spread over
 // the whole GPU.  Every item has a bounding box (computed after the sort),

@@ -69,13 +69,13 @@ def fold(s):
 
 
 def cell_geometry(n, L, rcut):
-    """The library's real-space cell grid: (cells per side, reach).  Cells
-    of side >= rcut / 2 (reach 2) unless those would hold fewer than 6
-    particles on average, or the box has fewer than 5 of them per side; then
+    """The library's real-space cell grid for a uniform system: (cells per
+    side, reach).  Cells of side >= rcut / 2 (reach 2) unless those would hold
+    fewer than 7 particles, or the box has fewer than 5 of them per side; then
     side >= rcut (reach 1)."""
     nc2 = min(512, int(np.floor(L * 2 / rcut * (1 - 1e-12))))
     nc1 = min(512, int(np.floor(L / rcut * (1 - 1e-12))))
-    if nc2 < 5 or (nc1 >= 3 and n < 6.0 * nc2 ** 3):
+    if nc2 < 5 or (nc1 >= 3 and n < 7.0 * nc2 ** 3):
         return max(nc1, 1), 1
     return nc2, 2
 

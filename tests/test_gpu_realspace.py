@@ -31,12 +31,76 @@ def corner_cluster(n_cluster, n_background, L, sigma, seed, centre=(0.0, 0.0, 0.
     return {"x": p[:, 0].copy(), "y": p[:, 1].copy(), "z": p[:, 2].copy(), "q": q, "L": float(L)}
 
 
-def cell_counts(s, rcut):
-    """Particles per cell of the library's grid."""
+def lattice(side, L, seed):
+    """side^3 particles in site order, jittered: no two closer than 0.4 sites."""
+    rng = np.random.default_rng(seed)
+    site = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    p = (site + 0.5 + 0.6 * (rng.uniform(size=site.shape) - 0.5)) * (L / side)
+    q = np.where(np.arange(len(p)) % 2 == 0, 1.0, -1.0)
+    return {"x": p[:, 0].copy(), "y": p[:, 1].copy(), "z": p[:, 2].copy(), "q": q, "L": float(L)}
+
+
+class DeviceRealteil:
+    """realteil_device of `solver` on device copies of a system."""
+
+    def __init__(self, solver, s, rcut, alpha):
+        import torch
+
+        self.solver, self.rcut, self.alpha = solver, rcut, alpha
+        self.n, self.L = len(s["q"]), s["L"]
+        self.dev = {k: torch.empty(self.n, dtype=torch.float64, device="cuda") for k in "xyzq"}
+        self.fr = torch.zeros(3 * self.n, dtype=torch.float64, device="cuda")
+        self.en = torch.zeros(1, dtype=torch.float64, device="cuda")
+        self.put(s)
+
+    def put(self, s):
+        import torch
+
+        self.solver.synchronize()
+        for k in "xyzq":
+            self.dev[k].copy_(torch.tensor(s[k]))
+        torch.cuda.synchronize()
+
+    def run(self, calls=1):
+        """Forces (3, n) and energy, summed over `calls` calls."""
+        import torch
+
+        for _ in range(calls):
+            self.solver.realteil_device(self.n, self.L, *[self.dev[k].data_ptr() for k in "xyzq"], self.rcut,
+                                        self.alpha, self.fr.data_ptr(), self.en.data_ptr())
+        self.solver.synchronize()
+        out = self.fr.cpu().numpy().reshape(3, self.n).copy(), float(self.en.item())
+        self.fr.zero_()
+        self.en.zero_()
+        torch.cuda.synchronize()
+        return out
+
+
+def on_cells(pkg, s, rcut, alpha, reach, prec_name="FP64"):
+    """Real-space forces, energy and cells per side of `s` (below 7
+    particles per cell of side rcut / 2 on average) on a cell list of the given
+    reach: the list is made by a first call, for uniform positions (reach 1)
+    or for a cluster (reach 2), and kept for `s`."""
+    rng = np.random.default_rng(1)
+    n, L = len(s["q"]), s["L"]
+    first = rng.uniform(0.0, L if reach == 1 else L / 16, (3, n))
+    solver = pkg.Solver(0, pkg.HostSystem.from_dict(s), pkg.parameters(16, 3, alpha, rcut),
+                        getattr(pkg, prec_name))
+    dev = DeviceRealteil(solver, dict(s, x=first[0], y=first[1], z=first[2]), rcut, alpha)
+    dev.run()
+    dev.put(s)
+    f, e = dev.run()
+    nc, got = cells_of(pkg, solver)
+    assert got == reach
+    solver.close()
+    return f, e, nc
+
+
+def cell_counts(s, nc):
+    """Particles per cell of a grid of nc cells per side."""
     L = s["L"]
-    nc, reach = cell_geometry(len(s["q"]), L, rcut)
     c = np.minimum((np.stack([s["x"], s["y"], s["z"]], 1) * nc / L).astype(int), nc - 1)
-    return nc, reach, np.bincount((c[:, 0] * nc + c[:, 1]) * nc + c[:, 2], minlength=nc ** 3)
+    return np.bincount((c[:, 0] * nc + c[:, 1]) * nc + c[:, 2], minlength=nc ** 3)
 
 
 @pytest.mark.parametrize("L,n_background,centre,reach", [
@@ -49,39 +113,43 @@ def test_wrapped_dense_cluster(pkg, orc, L, n_background, centre, reach):
     dense cell pairs; with cells of side rcut / 2 and of side rcut."""
     rcut, alpha = 3.0, 1.0
     s = corner_cluster(2500 if reach == 2 else 2000, n_background, L, 0.9, seed=31, centre=centre)
-    nc, got_reach, cnt = cell_counts(s, rcut)
-    assert got_reach == reach
+    f, e, nc = on_cells(pkg, s, rcut, alpha, reach)
+    cnt = cell_counts(s, nc)
     assert nc >= 2 * reach + 1 and cnt.max() > 128 and np.sum((cnt > 0) & (cnt <= 4)) > 50
     system = pkg.HostSystem.from_dict(s)
     forces = pkg.realteil(system, rcut, alpha)
     fr_ref, e_ref = orc.realteil(s, rcut, alpha)
-    err = rel_err(forces.real(), fr_ref)
+    err = max(rel_err(forces.real(), fr_ref), rel_err(f, fr_ref))
     print("reach %d, max cell %d, rel err %.2e, energy %.15e vs %.15e" % (
         reach, cnt.max(), err, system.c.energy, e_ref))
     assert err < 1e-13
     assert abs(system.c.energy - e_ref) <= 1e-12 * abs(e_ref)
+    assert abs(e - e_ref) <= 1e-12 * abs(e_ref)
 
 
-def test_single_dense_cell_of_many_chunks(pkg, orc):
+@pytest.mark.parametrize("reach,nc", [(1, 3), (2, 7)])
+def test_single_dense_cell_of_many_chunks(pkg, orc, reach, nc):
     """One cell of ~600 particles (ten chunks: the item's own chunk, later
     chunks of its cell, earlier ones left to their own items) in an
     otherwise sparse box."""
     L, rcut, alpha = 12.0, 3.0, 1.2
     rng = np.random.default_rng(5)
-    nc, _ = cell_geometry(900, L, rcut)
     side = L / nc
     cell = rng.uniform(1 * side + 1e-3, 2 * side - 1e-3, (600, 3))
     rest = rng.uniform(0.0, L, (300, 3))
     p = np.concatenate([cell, rest])
     q = np.where(np.arange(900) % 2 == 0, 1.0, -1.0)
     s = {"x": p[:, 0].copy(), "y": p[:, 1].copy(), "z": p[:, 2].copy(), "q": q, "L": L}
-    _, _, cnt = cell_counts(s, rcut)
-    assert cnt.max() >= 600
+    assert cell_counts(s, nc).max() >= 600
+    f, e, got_nc = on_cells(pkg, s, rcut, alpha, reach)
+    assert got_nc == nc
     system = pkg.HostSystem.from_dict(s)
     forces = pkg.realteil(system, rcut, alpha)
     fr_ref, e_ref = orc.realteil(s, rcut, alpha)
     assert rel_err(forces.real(), fr_ref) < 1e-13
     assert abs(system.c.energy - e_ref) <= 1e-12 * abs(e_ref)
+    assert rel_err(f, fr_ref) < 1e-13
+    assert abs(e - e_ref) <= 1e-12 * abs(e_ref)
 
 
 def test_newton_third_law(pkg):
@@ -129,7 +197,7 @@ def test_device_form_accumulates_and_mixed_is_close(pkg, orc, prec_name):
         assert abs(e - e_ref) <= 1e-5 * abs(e_ref)
 
 
-@pytest.mark.parametrize("m,reach", [(400, 1), (1100, 2)])
+@pytest.mark.parametrize("m,reach", [(400, 1), (1400, 2)])
 def test_pairs_at_the_cutoff(pkg, orc, m, reach):
     """Pairs placed within 1e-9 of rcut on either side, in all directions and
     across cell and box boundaries: the candidate search (FP16 operands in
@@ -154,7 +222,7 @@ def test_pairs_at_the_cutoff(pkg, orc, m, reach):
     assert abs(system.c.energy - e_ref) <= 1e-12 * abs(e_ref)
 
 
-@pytest.mark.parametrize("m,reach", [(400, 1), (1100, 2)])
+@pytest.mark.parametrize("m,reach", [(400, 1), (1400, 2)])
 def test_pairs_at_the_cutoff_mixed(pkg, orc, m, reach):
     """The mixed form on the pairs of test_pairs_at_the_cutoff: their FP32
     squared distances fall inside the band around rcut^2, where the FP64 test
@@ -302,48 +370,6 @@ def test_cell_size_follows_the_clustering(pkg, orc, layout, prec_name):
     solver.close()
 
 
-def lattice(side, L, seed):
-    """side^3 particles in site order, jittered: no two closer than 0.4 sites."""
-    rng = np.random.default_rng(seed)
-    site = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)
-    p = (site + 0.5 + 0.6 * (rng.uniform(size=site.shape) - 0.5)) * (L / side)
-    q = np.where(np.arange(len(p)) % 2 == 0, 1.0, -1.0)
-    return {"x": p[:, 0].copy(), "y": p[:, 1].copy(), "z": p[:, 2].copy(), "q": q, "L": float(L)}
-
-
-class DeviceRealteil:
-    """realteil_device of `solver` on device copies of a system."""
-
-    def __init__(self, solver, s, rcut, alpha):
-        import torch
-
-        self.solver, self.rcut, self.alpha = solver, rcut, alpha
-        self.n, self.L = len(s["q"]), s["L"]
-        self.dev = {k: torch.empty(self.n, dtype=torch.float64, device="cuda") for k in "xyzq"}
-        self.fr = torch.zeros(3 * self.n, dtype=torch.float64, device="cuda")
-        self.put(s)
-
-    def put(self, s):
-        import torch
-
-        self.solver.synchronize()
-        for k in "xyzq":
-            self.dev[k].copy_(torch.tensor(s[k]))
-        torch.cuda.synchronize()
-
-    def run(self, calls=1):
-        import torch
-
-        for _ in range(calls):
-            self.solver.realteil_device(self.n, self.L, *[self.dev[k].data_ptr() for k in "xyzq"], self.rcut,
-                                        self.alpha, self.fr.data_ptr(), None)
-        self.solver.synchronize()
-        out = self.fr.cpu().numpy().reshape(3, self.n).copy()
-        self.fr.zero_()
-        torch.cuda.synchronize()
-        return out
-
-
 @pytest.mark.parametrize("held", ["nothing", "unreadable", "zeros"])
 def test_init_reads_sizes_only(pkg, orc, held):
     """Init takes the particle count and the box length of a system whose
@@ -359,7 +385,7 @@ def test_init_reads_sizes_only(pkg, orc, held):
         nowhere = ctypes.cast(ctypes.c_void_p(8), ctypes.POINTER(ctypes.c_double))
         system.c.p.contents.x = system.c.p.contents.y = system.c.p.contents.z = system.c.q = nowhere
     solver = pkg.Solver(7, system, pkg.parameters(16, 3, alpha, rcut))
-    fr = DeviceRealteil(solver, s, rcut, alpha).run()
+    fr, _ = DeviceRealteil(solver, s, rcut, alpha).run()
     assert cells_of(pkg, solver)[1] == 1
     assert rel_err(fr, orc.realteil(s, rcut, alpha, cells=True)[0]) < 1e-13
     solver.close()
@@ -376,3 +402,24 @@ def test_lattice_order_is_not_clustered(pkg, side):
     DeviceRealteil(solver, s, 3.0, 1.0).run()
     assert cells_of(pkg, solver)[1] == 1
     solver.close()
+
+
+@pytest.mark.parametrize("per_cell,clustering,reach", [(6, 1.0, 1), (8, 1.0, 2), (11, 1.0, 2), (2, 3.0, 1),
+                                                       (2, 4.0, 2), (0.5, 100.0, 2), (0.5, 1.0, 1)])
+def test_cell_size_rule(pkg, per_cell, clustering, reach):
+    """Cells of side rcut / 2 from 7 particles in a typical particle's cell
+    on; clustering 1 is what the batch assumes."""
+    L, rcut = 30.3, 3.0  # 20 cells of side rcut / 2, 10 of side rcut
+    n = int(per_cell * 8000)
+    lib = pkg.lib()
+    lib.p3mk_cells_create.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_int] + [ctypes.c_double] * 3
+    lib.p3mk_cells_geometry.restype = None
+    lib.p3mk_cells_geometry.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)]
+    lib.p3mk_cells_destroy.restype, lib.p3mk_cells_destroy.argtypes = None, [ctypes.c_void_p]
+    cells, nc, got = ctypes.c_void_p(), ctypes.c_int(), ctypes.c_int()
+    assert lib.p3mk_cells_create(ctypes.byref(cells), n, L, rcut, clustering) == 0
+    lib.p3mk_cells_geometry(cells, ctypes.byref(nc), ctypes.byref(got))
+    lib.p3mk_cells_destroy(cells)
+    assert (nc.value, got.value) == ((10, 1) if reach == 1 else (20, 2))
+    if clustering == 1.0:
+        assert cell_geometry(n, L, rcut) == (nc.value, got.value)
