@@ -267,7 +267,9 @@ int p3m_hip_realteil(system_t *s, parameters_t *p, forces_t *f);
  * double, may be NULL) += energy.  Uses the stream of d.  The first
  * real-space call for a box length and cutoff makes the cell list: it
  * allocates, and waits for the stream to see how clustered the positions
- * are (the cell size follows them, never a result). */
+ * are (the cell size follows them, never a result).  Later calls look again
+ * now and then without waiting; one that finds the clustering much changed
+ * makes the list anew. */
 int p3m_hip_realteil_device(data_t *d, int n, double length, const double *x, const double *y,
                             const double *z, const double *q, double rcut, double alpha,
                             double *fr, double *energy);

@@ -72,6 +72,7 @@ typedef struct {
     p3mk_cells *cells;
     p3mk_psort *psort;
     double cells_L, cells_rc;
+    int clust_calls, clust_asked; /* calls since the last sample; a sample is under way */
     int have_G;
     int have_ks_events;
     int have_rs_events;
@@ -531,15 +532,55 @@ static int make_cells(p3mk_cells **cells, int n, double L, double rcut, int npos
     return p3mk_cells_create(cells, n, L, rcut, clustering);
 }
 
+/* The list of an earlier call meets the positions of now: every
+ * CLUSTER_CALLS calls (a launch of one workgroup, 5 us) their clustering is
+ * sampled again without waiting, and once the sample has arrived the list is
+ * remade if it asks for the other cell size by a quarter more than the line
+ * (so that noise of the sample does not remake it back and forth).  Without
+ * the memory for it the old list stays. */
+#define CLUSTER_CALLS 64
+#define CLUSTER_MARGIN 1.25
+static int follow_clustering(p3m_ctx *c, int n, const double *x, const double *y, const double *z) {
+    int nc, reach;
+    double seen;
+    if (!p3mk_cells_by_clustering(c->n, c->cells_L, c->cells_rc))
+        return P3M_HIP_OK;
+    if (!c->clust_asked) {
+        if (++c->clust_calls < CLUSTER_CALLS)
+            return P3M_HIP_OK;
+        c->clust_calls = 0;
+        c->clust_asked = 1;
+        TRYK(p3mk_clustering(n, c->cells_L, x, y, z, c->hclust, c->q), "clustering");
+        return P3M_HIP_OK;
+    }
+    seen = *(volatile double *)c->hclust;
+    if (!(seen > 0.0))
+        return P3M_HIP_OK;
+    c->clust_asked = 0;
+    p3mk_cells_geometry(c->cells, &nc, &reach);
+    seen = reach == 2 ? seen * CLUSTER_MARGIN : seen / CLUSTER_MARGIN;
+    if (p3mk_cells_reach(c->n, c->cells_L, c->cells_rc, seen) != reach) {
+        p3mk_cells *other = NULL;
+        if (p3mk_cells_create(&other, c->n, c->cells_L, c->cells_rc, seen) == P3MK_OK) {
+            p3mk_cells *old = c->cells;
+            c->cells = other;
+            TRYK(p3mk_queue_sync(c->q), "sync"); /* the old one may be in use */
+            p3mk_cells_destroy(old);
+        }
+    }
+    return P3M_HIP_OK;
+}
+
 static int ensure_cells(p3m_ctx *c, double L, double rcut, int n, const double *x, const double *y,
                         const double *z) {
     if (c->cells != NULL && c->cells_L == L && c->cells_rc == rcut)
-        return P3M_HIP_OK;
+        return follow_clustering(c, n, x, y, z);
     p3mk_cells_destroy(c->cells);
     c->cells = NULL;
     TRYK(make_cells(&c->cells, c->n, L, rcut, n, x, y, z, c->hclust, c->q), "cell list");
     c->cells_L = L;
     c->cells_rc = rcut;
+    c->clust_calls = c->clust_asked = 0;
     return P3M_HIP_OK;
 }
 

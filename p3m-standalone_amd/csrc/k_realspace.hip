@@ -1698,7 +1698,8 @@ k_clustering(int n, double Li, const double *__restrict__ x, const double *__res
         double sum = 0.0;
         for (int w = 0; w < kClusterThreads / 64; w++)
             sum += part[w];
-        *out = fmax(1.0, 2.0 * sum * kClusterCells / ((double)m * (m - 1.0)));
+        __hip_atomic_store(out, fmax(1.0, 2.0 * sum * kClusterCells / ((double)m * (m - 1.0))), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -1706,7 +1707,7 @@ k_clustering(int n, double Li, const double *__restrict__ x, const double *__res
 
 extern "C" int p3mk_clustering(int n, double L, const double *x, const double *y, const double *z, double *out,
                                p3mk_queue *qu) {
-    *out = 1.0;
+    *out = n < 2 ? 1.0 : 0.0;
     if (n < 2)
         return P3MK_OK;
     hipLaunchKernelGGL(k_clustering, dim3(1), dim3(kClusterThreads), 0, p3mk_stream(qu), n, 1.0 / L, x, y, z, out);
@@ -1715,6 +1716,12 @@ extern "C" int p3mk_clustering(int n, double L, const double *x, const double *y
 
 extern "C" int p3mk_cells_by_clustering(int n, double L, double rcut) {
     return p3m::cells_by_clustering(n, L, rcut);
+}
+
+extern "C" int p3mk_cells_reach(int n, double L, double rcut, double clustering) {
+    int nc, reach;
+    p3m::cell_geometry(n, L, rcut, clustering, nc, reach);
+    return reach;
 }
 
 extern "C" void p3mk_cells_geometry(const p3mk_cells *c, int *nc, int *reach) {

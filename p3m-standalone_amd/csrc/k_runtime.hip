@@ -178,6 +178,7 @@ extern "C" int p3mk_alloc(void **p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) {
         *p = nullptr;
+        (void)hipGetLastError(); // reported here, not by the next launch check
         return p3mk_fail(P3MK_ENOMEM, "hipMalloc", (int)e);
     }
     return P3MK_OK;

@@ -201,10 +201,12 @@ typedef struct p3mk_cells p3mk_cells; /* cell-list workspace */
 int p3mk_cells_create(p3mk_cells **c, int n, double L, double rcut, double clustering);
 /* does the cell size of a list for n particles depend on the clustering? */
 int p3mk_cells_by_clustering(int n, double L, double rcut);
+/* reach of the list that p3mk_cells_create makes */
+int p3mk_cells_reach(int n, double L, double rcut, double clustering);
 /* cells per side and their side in units of 1 / rcut (1 or 2) */
 void p3mk_cells_geometry(const p3mk_cells *c, int *nc, int *reach);
-/* clustering of n device positions to *out, host memory the device writes
- * (p3mk_alloc_host); valid after p3mk_queue_sync */
+/* clustering (>= 1) of n device positions to *out, host memory the device
+ * writes (p3mk_alloc_host); 0 until the queue has come to it */
 int p3mk_clustering(int n, double L, const double *x, const double *y, const double *z, double *out,
                     p3mk_queue *qu);
 void p3mk_cells_destroy(p3mk_cells *c);

@@ -423,3 +423,26 @@ def test_cell_size_rule(pkg, per_cell, clustering, reach):
     assert (nc.value, got.value) == ((10, 1) if reach == 1 else (20, 2))
     if clustering == 1.0:
         assert cell_geometry(n, L, rcut) == (nc.value, got.value)
+
+
+def test_cell_size_follows_changed_positions(pkg, orc):
+    """A system that clusters and spreads out again: the list's cell size is
+    the new positions' within 2 x 64 calls, and the forces are the oracle's
+    before, at and after the change."""
+    rcut, alpha = 3.0, 1.0
+    spread = lattice(14, 27.0, seed=6)
+    tight = dict(spread)
+    for k in "xyz":
+        tight[k] = np.mod(spread[k] * 0.25 - 2.0, 27.0)  # spacing 0.48, across the box corner
+    ref = {id(s): orc.realteil(s, rcut, alpha, cells=True)[0] for s in (spread, tight)}
+    solver = pkg.Solver(0, pkg.HostSystem.from_dict(spread), pkg.parameters(16, 3, alpha, rcut))
+    dev = DeviceRealteil(solver, spread, rcut, alpha)
+    for s, before, after in ((spread, 1, 1), (tight, 1, 2), (spread, 2, 1)):
+        dev.put(s)
+        assert rel_err(dev.run()[0], ref[id(s)]) < 1e-13
+        assert cells_of(pkg, solver)[1] == before
+        dev.run(130)
+        dev.run(2)
+        assert cells_of(pkg, solver)[1] == after
+        assert rel_err(dev.run()[0], ref[id(s)]) < 1e-13
+    solver.close()
