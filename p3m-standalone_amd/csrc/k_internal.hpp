@@ -19,4 +19,4 @@ hipStream_t p3mk_stream(p3mk_queue *q);
 // Exclusive prefix sum: start[0..m] (start[m] = total) of count[0..m);
 // scratch holds p3mk_scan_scratch_ints(m) ints.
 size_t p3mk_scan_scratch_ints(long m);
-int p3mk_exclusive_scan(const int *count, long m, int *start, int *scratch, p3mk_queue *q);
+extern "C" int p3mk_exclusive_scan(const int *count, long m, int *start, int *scratch, p3mk_queue *q);

@@ -1,9 +1,10 @@
 // Exclusive prefix sum of int counts, used by the counting sorts of the
 // particle <-> mesh and real-space kernels.  Up to 4096 counts: one launch
 // of one workgroup (runs of up to four counts per thread; longer serial runs
-// lose to the launches below).  Beyond: two launches, per-block scans of 1024
-// elements, and the sums of the blocks before added (each block adds them up
-// itself: a launch less than a scan of the sums, 4 us of a system's step).
+// lose to the launches below).  Beyond: per-block scans of 1024 elements, and
+// the sums of the blocks before added.  Up to kDirectBlocks blocks each block
+// adds those up itself; beyond, where that grows with the square of the
+// blocks, their own prefix sums are made by a launch between the two.
 #include <hip/hip_runtime.h>
 
 #include "k_internal.hpp"
@@ -52,8 +53,41 @@ __global__ void __launch_bounds__(kBlock) k_scan_blocks(const int *__restrict__ 
         sums[blockIdx.x] = total;
 }
 
+// Blocks up to which k_scan_add adds up the sums itself.  Whole scans, that
+// way against a launch for the sums, us: 512 blocks 6.3 / 9.9, 1024 9.3 / 10.5,
+// 2048 15.2 / 15.6, 4096 26.2 / 25.2, 16,384 113 / 85, 262,144 8336 / 1590.
+constexpr int kDirectBlocks = 2048;
+
+// single block: exclusive scan of nb block sums, 1024 a step with a carry
+__global__ void __launch_bounds__(kBlock) k_scan_sums(int *__restrict__ sums, int nb) {
+    __shared__ int sh[128];
+    int carry = 0;
+    for (int base = 0; base < nb; base += kBlock) {
+        const int i = base + threadIdx.x;
+        const int v = (i < nb) ? sums[i] : 0;
+        int total;
+        const int e = block_exclusive_scan(v, sh, total);
+        if (i < nb)
+            sums[i] = carry + e;
+        carry += total;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0)
+        sums[nb] = carry;
+}
+
+// the same from the sums' prefix sums
+__global__ void __launch_bounds__(kBlock) k_scan_add_prefix(int *__restrict__ out, int m,
+                                                            const int *__restrict__ sums, int nb) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < m)
+        out[i] += sums[blockIdx.x];
+    if (i == 0)
+        out[m] = sums[nb];
+}
+
 // adds to each block's elements the sums of the blocks before it, which the
-// block adds up itself (at most a few thousand, one or two per thread)
+// block adds up itself (at most kDirectBlocks, two per thread)
 __global__ void __launch_bounds__(kBlock) k_scan_add(int *__restrict__ out, int m,
                                                      const int *__restrict__ sums, int nb) {
     __shared__ int sh[kBlock / 64];
@@ -115,6 +149,12 @@ int p3mk_exclusive_scan(const int *count, long m, int *start, int *scratch, p3mk
     }
     hipLaunchKernelGGL(k_scan_blocks, dim3(nb), dim3(kBlock), 0, s, count, (int)m, start, scratch);
     P3MK_TRY(p3mk_launch_check("scan blocks"));
+    if (nb > kDirectBlocks) {
+        hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kBlock), 0, s, scratch, nb);
+        P3MK_TRY(p3mk_launch_check("scan sums"));
+        hipLaunchKernelGGL(k_scan_add_prefix, dim3(nb), dim3(kBlock), 0, s, start, (int)m, scratch, nb);
+        return p3mk_launch_check("scan add");
+    }
     hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(kBlock), 0, s, start, (int)m, scratch, nb);
     return p3mk_launch_check("scan add");
 }
