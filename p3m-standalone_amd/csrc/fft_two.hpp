@@ -39,8 +39,6 @@ namespace p3m {
 namespace fft {
 
 constexpr int kMaxTwoRadix = 16;
-// threads of a single-mesh workgroup: lines x R2, rounded up to wavefronts
-constexpr int kTwoThreads = 256;
 
 // N = r1 r2; div1 / div2: u / r = (u div) >> 16 for u < 1024
 struct TwoPlan {

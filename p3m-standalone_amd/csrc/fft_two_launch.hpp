@@ -66,20 +66,23 @@ namespace p3m {
 namespace fft {
 namespace {
 
+template <typename T> size_t two_lds(const TwoPlan &p, int lg) {
+    return sizeof(c2_t<T>) * (size_t)two_lds_points(p, 1 << lg);
+}
+
 // Lines per workgroup over one mesh: 16 (a strided row of 128 bytes in FP32,
 // 256 in FP64), halved down to 4 while the launch would have fewer
-// workgroups than the GPU has CUs.
-inline int two_lg(long nlines) {
+// workgroups than the GPU has CUs, or while its LDS is above kLdsBudget, what
+// a kernel gets without an attribute of its own (FP64 at 256 points: 69,632
+// bytes with 16 lines).
+template <typename T> int two_lg(const TwoPlan &p, long nlines) {
     int lg = 4;
-    while (lg > 2 && ((nlines + (1 << lg) - 1) >> lg) < 256)
+    while (lg > 2 && (((nlines + (1 << lg) - 1) >> lg) < 256 || two_lds<T>(p, lg) > kLdsBudget))
         lg--;
     return lg;
 }
 inline unsigned two_blocks(long nlines, int lg) { return (unsigned)((nlines + (1 << lg) - 1) >> lg); }
 inline unsigned two_block(const TwoPlan &p, int lg) { return (unsigned)((((p.r2 << lg) + 63) / 64) * 64); }
-template <typename T> size_t two_lds(const TwoPlan &p, int lg) {
-    return sizeof(c2_t<T>) * (size_t)two_lds_points(p, 1 << lg);
-}
 
 template <typename T, bool CONTIG>
 __global__ void __launch_bounds__(kThreads)
@@ -128,7 +131,7 @@ k_two_divergence(const c2_t<T> *in0, const c2_t<T> *in1, const c2_t<T> *in2, c2_
 template <typename T>
 int two_pass(const TwoPlan &p, Three<c2_t<T> *> data, int k, const LineMap &m, const double2 *tw, int inv,
              bool contig, hipStream_t st) {
-    const int lg = two_lg(k * m.nlines);
+    const int lg = two_lg<T>(p, k * m.nlines);
     const dim3 grid(two_blocks(m.nlines, lg), (unsigned)k), block(two_block(p, lg));
     if (contig)
         hipLaunchKernelGGL((k_two_pass<T, true>), grid, block, two_lds<T>(p, lg), st, data, m, p, tw, inv, lg);
@@ -140,7 +143,7 @@ int two_pass(const TwoPlan &p, Three<c2_t<T> *> data, int k, const LineMap &m, c
 template <typename T>
 int two_r2c(const TwoPlan &p, Three<const T *> in, Three<c2_t<T> *> out, int k, long nlines, const double2 *tw,
             hipStream_t st) {
-    const int lg = two_lg(k * nlines);
+    const int lg = two_lg<T>(p, k * nlines);
     hipLaunchKernelGGL(k_two_r2c<T>, dim3(two_blocks(nlines, lg), (unsigned)k), dim3(two_block(p, lg)), two_lds<T>(p, lg), st,
                        in, out, nlines, p, tw, lg);
     return p3mk_launch_check("fft r2c");
@@ -149,7 +152,7 @@ int two_r2c(const TwoPlan &p, Three<const T *> in, Three<c2_t<T> *> out, int k, 
 template <typename T>
 int two_c2r(const TwoPlan &p, Three<const c2_t<T> *> in, Three<T *> out, int k, long nlines, const double2 *tw,
             hipStream_t st) {
-    const int lg = two_lg(k * nlines);
+    const int lg = two_lg<T>(p, k * nlines);
     hipLaunchKernelGGL(k_two_c2r<T>, dim3(two_blocks(nlines, lg), (unsigned)k), dim3(two_block(p, lg)), two_lds<T>(p, lg), st,
                        in, out, nlines, p, tw, lg);
     return p3mk_launch_check("fft c2r");
@@ -158,7 +161,7 @@ int two_c2r(const TwoPlan &p, Three<const c2_t<T> *> in, Three<T *> out, int k, 
 template <typename T>
 int two_convolve(const TwoPlan &p, const c2_t<T> *in, c2_t<T> *const out[3], int nout, long nl, int W,
                  const double2 *tw, const double *G, const double *Dn, double twopi_L, hipStream_t st) {
-    const int lg = two_lg(nl);
+    const int lg = two_lg<T>(p, nl);
     const dim3 grid(two_blocks(nl, lg)), block(two_block(p, lg));
     if (nout == 1)
         hipLaunchKernelGGL((k_two_convolve<1, T>), grid, block, two_lds<T>(p, lg), st, in, out[0], nullptr, nullptr,
@@ -172,7 +175,7 @@ int two_convolve(const TwoPlan &p, const c2_t<T> *in, c2_t<T> *const out[3], int
 template <typename T>
 int two_divergence(const TwoPlan &p, const c2_t<T> *const in[3], c2_t<T> *out, long nl, int W,
                    const double2 *tw, const double *G, const double *Dn, double twopi_L, hipStream_t st) {
-    const int lg = two_lg(nl);
+    const int lg = two_lg<T>(p, nl);
     hipLaunchKernelGGL(k_two_divergence<T>, dim3(two_blocks(nl, lg)), dim3(two_block(p, lg)), two_lds<T>(p, lg), st,
                        in[0], in[1], in[2], out, nl, W, p, tw, G, Dn, twopi_L, lg);
     return p3mk_launch_check("divergence");

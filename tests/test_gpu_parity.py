@@ -329,6 +329,7 @@ def _fft_api(pkg):
     for name, res, args in [
         ("p3mk_fft_forward_zy", ctypes.c_int, [ctypes.c_void_p] * 4),
         ("p3mk_fft_backward_yz", ctypes.c_int, [ctypes.c_void_p] * 4),
+        ("p3mk_divergence", ctypes.c_int, [ctypes.c_void_p] * 6),
     ]:
         f = getattr(L, name)
         f.restype, f.argtypes = res, args
@@ -516,6 +517,41 @@ def test_fft_factor_splits(pkg, M, fp32):
             assert eb < 2 * tol
         finally:
             rig.close()
+
+
+@pytest.mark.parametrize("M,fp32", [(18, 0), (90, 0), (240, 0), (256, 0), (256, 1)])
+def test_divergence_vs_numpy(pkg, M, fp32):
+    """The adjoint's x pass (three spectra in, one out, the multiply between
+    the transforms) on the first y rows of r2c spectra against numpy in FP64,
+    up to 256 points (the largest two-factor mesh and the most LDS).  FP64
+    2e-14, two of the other transforms' 1e-14; FP32 storage with FP64
+    arithmetic 4e-7 as theirs."""
+    fn = _fft_api(pkg)
+    rng = np.random.default_rng(500 + M)
+    cdt = np.complex64 if fp32 else np.complex128
+    H = M // 2 + 1
+    # [x][y][z]; one random plane per x repeated along y keeps the host work small
+    ins = [np.repeat((rng.uniform(-1, 1, (M, 1, H)) + 1j * rng.uniform(-1, 1, (M, 1, H))), M, 1).astype(cdt)
+           for _ in range(3)]
+    G = np.ascontiguousarray(np.broadcast_to(rng.uniform(0.5, 1.5, (M, M, 1)), (M, M, M)))
+    Dn = rng.uniform(-1.0, 1.0, M)
+    rig = _FftRig(fn, M, 1, fp32, [a.nbytes for a in ins] + [ins[0].nbytes, G.nbytes, Dn.nbytes])
+    try:
+        for k, a in enumerate(ins + [None, G, Dn]):
+            if a is not None:
+                rig.put(k, a)
+        spectra = (ctypes.c_void_p * 3)(*[b.value for b in rig.bufs[:3]])
+        assert fn["p3mk_divergence"](rig.plan, rig.bufs[4], rig.bufs[5], spectra, rig.bufs[3], rig.q) == 0
+        got = rig.get(3, np.empty_like(ins[0]))
+        for j in (0, 1, M // 2, M - 1):
+            X = [np.fft.fft(a[:, j].astype(np.complex128), axis=0) for a in ins]
+            D = [Dn[:, None], Dn[j], Dn[None, :H]]
+            s = sum(-2j * np.pi * d * x for d, x in zip(D, X)) * G[:, j, :H]
+            err = rel_err(got[:, j].astype(np.complex128), np.fft.ifft(s, axis=0) * M)
+            print("M %d fp32 %d y %d: %.2e" % (M, fp32, j, err))
+            assert err < (4e-7 if fp32 else 2e-14)
+    finally:
+        rig.close()
 
 
 @pytest.mark.parametrize("method,M", [(0, 10), (0, 26), (3, 90), (1, 28), (6, 44), (6, 150), (6, 110)])
