@@ -225,39 +225,6 @@ extern "C" int p3mk_copy_d2d(void *dst, const void *src, size_t bytes, p3mk_queu
     return copy(dst, src, bytes, hipMemcpyDeviceToDevice, q);
 }
 
-__global__ void k_fill_zero16(uint4 *p, size_t n16) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    const uint4 z = make_uint4(0u, 0u, 0u, 0u);
-    for (; i < n16; i += stride)
-        p[i] = z;
-}
-
-__global__ void k_fill_zero1(unsigned char *p, size_t n) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n)
-        p[i] = 0;
-}
-
-extern "C" int p3mk_fill_zero(void *p, size_t bytes, p3mk_queue *q) {
-    if (bytes == 0)
-        return P3MK_OK;
-    // hipMalloc returns 256-byte aligned memory; all callers pass such
-    // pointers, so the 16-byte body below covers bytes - bytes % 16.
-    const size_t n16 = bytes / 16, rem = bytes % 16;
-    if (n16) {
-        size_t blocks = (n16 + 255) / 256;
-        if (blocks > 8192)
-            blocks = 8192;
-        hipLaunchKernelGGL(k_fill_zero16, dim3((unsigned)blocks), dim3(256), 0, q->stream,
-                           (uint4 *)p, n16);
-    }
-    if (rem)
-        hipLaunchKernelGGL(k_fill_zero1, dim3(1), dim3(64), 0, q->stream,
-                           (unsigned char *)p + 16 * n16, rem);
-    return p3mk_launch_check("fill_zero");
-}
-
 __global__ void k_axpy(size_t n, double a, const double *__restrict__ x, double *__restrict__ y) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -275,9 +242,11 @@ extern "C" int p3mk_axpy(size_t n, double a, const double *x, double *y, p3mk_qu
     return p3mk_launch_check("axpy");
 }
 
+// p: the 16-byte unit each range begins in; the range is [lo, hi) from there
 struct FillRanges {
     unsigned char *p[P3MK_MAX_RANGES];
-    unsigned long long bytes[P3MK_MAX_RANGES], first[P3MK_MAX_RANGES + 1]; // first 16-byte unit of each
+    unsigned long long hi[P3MK_MAX_RANGES], first[P3MK_MAX_RANGES + 1]; // first unit of each
+    unsigned char lo[P3MK_MAX_RANGES];
 };
 
 __global__ void k_fill_many(FillRanges r, int k) {
@@ -290,19 +259,20 @@ __global__ void k_fill_many(FillRanges r, int k) {
         for (int j = 1; j < P3MK_MAX_RANGES; j++)
             s += (j < k && u >= r.first[j]) ? 1 : 0;
         unsigned char *base = r.p[0];
-        unsigned long long bytes = r.bytes[0], first = r.first[0];
+        unsigned long long lo = r.lo[0], hi = r.hi[0], first = r.first[0];
 #pragma unroll
         for (int j = 1; j < P3MK_MAX_RANGES; j++)
             if (s == j) {
                 base = r.p[j];
-                bytes = r.bytes[j];
+                lo = r.lo[j];
+                hi = r.hi[j];
                 first = r.first[j];
             }
         const unsigned long long at = (u - first) * 16;
-        if (at + 16 <= bytes) {
+        if (at >= lo && at + 16 <= hi) {
             *reinterpret_cast<uint4 *>(base + at) = z;
-        } else {
-            for (unsigned long long b = at; b + 4 <= bytes; b += 4)
+        } else { // a range's first or last unit
+            for (unsigned long long b = at > lo ? at : lo; b < at + 16 && b < hi; b += 4)
                 *reinterpret_cast<unsigned int *>(base + b) = 0u;
         }
     }
@@ -310,7 +280,8 @@ __global__ void k_fill_many(FillRanges r, int k) {
 
 // One launch for all the buffers a force evaluation starts from zero (a
 // launch each, and one more for a size that is no multiple of 16 bytes, were
-// a third of a small system's launches).
+// a third of a small system's launches).  A range may begin at any word: the
+// callers' force arrays and the parts of one array are 8-byte aligned.
 extern "C" int p3mk_fill_zero_many(int k, const p3mk_range *ranges, p3mk_queue *q) {
     FillRanges r = {};
     int n = 0;
@@ -318,12 +289,14 @@ extern "C" int p3mk_fill_zero_many(int k, const p3mk_range *ranges, p3mk_queue *
     for (int j = 0; j < k; j++) {
         if (ranges[j].bytes == 0)
             continue;
-        if (n == P3MK_MAX_RANGES || ranges[j].bytes % 4 != 0)
-            return p3mk_fail(P3MK_EINVAL, "zero fill: too many ranges or an odd size", 0);
-        r.p[n] = (unsigned char *)ranges[j].p;
-        r.bytes[n] = ranges[j].bytes;
+        const unsigned long long p = (unsigned long long)ranges[j].p, lo = p % 16;
+        if (n == P3MK_MAX_RANGES || ranges[j].bytes % 4 != 0 || p % 4 != 0)
+            return p3mk_fail(P3MK_EINVAL, "zero fill: too many ranges, or one not of whole words", 0);
+        r.p[n] = (unsigned char *)ranges[j].p - lo;
+        r.lo[n] = (unsigned char)lo;
+        r.hi[n] = lo + ranges[j].bytes;
         r.first[n] = units;
-        units += (ranges[j].bytes + 15) / 16;
+        units += (r.hi[n] + 15) / 16;
         n++;
     }
     if (n == 0)
@@ -333,6 +306,11 @@ extern "C" int p3mk_fill_zero_many(int k, const p3mk_range *ranges, p3mk_queue *
     const unsigned blocks = (unsigned)(units > 8192ull * 256 ? 8192 : (units + 255) / 256);
     hipLaunchKernelGGL(k_fill_many, dim3(blocks), dim3(256), 0, q->stream, r, n);
     return p3mk_launch_check("fill_zero");
+}
+
+extern "C" int p3mk_fill_zero(void *p, size_t bytes, p3mk_queue *q) {
+    const p3mk_range r = {p, bytes};
+    return p3mk_fill_zero_many(1, &r, q);
 }
 
 // The reference's sum (common.c:315-319): f_k + f_r rounded, then added to f.

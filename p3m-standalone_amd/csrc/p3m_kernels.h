@@ -52,10 +52,10 @@ void p3mk_release_host(void *p);
 int p3mk_copy_h2d(void *dst, const void *src, size_t bytes, p3mk_queue *q);
 int p3mk_copy_d2h(void *dst, const void *src, size_t bytes, p3mk_queue *q);
 int p3mk_copy_d2d(void *dst, const void *src, size_t bytes, p3mk_queue *q);
-/* zero fill by a kernel (safe inside captured graphs) */
+/* zero fill by a kernel (safe inside captured graphs); address and size
+ * multiples of 4 bytes */
 int p3mk_fill_zero(void *p, size_t bytes, p3mk_queue *q);
-/* the same over up to P3MK_MAX_RANGES ranges (sizes multiples of 4 bytes) in
- * one launch */
+/* the same over up to P3MK_MAX_RANGES ranges in one launch */
 typedef struct {
     void *p;
     size_t bytes;

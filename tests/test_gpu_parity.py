@@ -479,6 +479,74 @@ def test_calculate_forces_writes_everything(pkg, orc, method, n, L, M, cao, rcut
     solver.close()
 
 
+@pytest.mark.parametrize("method,n,L,M,cao,rcut", [
+    (2, 333, 8.0, 16, 5, 3.9),   # nearest images: f_r is zero-filled too
+    (7, 1001, 30.0, 32, 4, 3.0),
+])
+def test_calculate_forces_into_parts_of_one_array(pkg, orc, method, n, L, M, cao, rcut):
+    """f, f_k, f_r and the energy as neighbouring parts of one array that
+    begins 8 bytes off a 16-byte boundary (odd n: so do some of the parts):
+    each is written whole and nothing beside them."""
+    import torch
+
+    alpha = 1.0
+    s = random_system(n, L, seed=n + 1, charges="normal")
+    fk_ref, f_self = orc.kspace_force(method, s, M, cao, alpha)
+    fr_ref, e_ref = orc.realteil(s, rcut, alpha, cells=True)
+    solver = pkg.Solver(method, pkg.HostSystem.from_dict(s), pkg.parameters(M, cao, alpha, rcut))
+    dev = {k: torch.tensor(s[k], dtype=torch.float64, device="cuda") for k in "xyzq"}
+    block = torch.full((9 * n + 3,), float("nan"), dtype=torch.float64, device="cuda")
+    at = [block.data_ptr() + 8 * (1 + 3 * n * k) for k in range(4)]
+    torch.cuda.synchronize()
+    solver.calculate_forces_device(n, L, *[dev[k].data_ptr() for k in "xyzq"], rcut, alpha, *at)
+    solver.synchronize()
+    got = block.cpu().numpy()
+    f, fk, fr = (got[1 + 3 * n * k:1 + 3 * n * (k + 1)].reshape(3, n) for k in range(3))
+    assert np.isnan(got[0]) and np.isnan(got[-1])
+    assert rel_err(fk, fk_ref) < 1e-12
+    assert rel_err(f, f_self + (fk_ref + fr_ref)) < 1e-12
+    assert rel_err(fr, fr_ref) < 1e-13
+    assert abs(got[9 * n + 1] - e_ref) <= 1e-12 * abs(e_ref)
+    solver.close()
+
+
+def test_zero_fill_ranges(pkg):
+    """Ranges that begin and end at any word of a 16-byte unit, empty ones,
+    ones within one unit and long ones: exactly their words are cleared; an
+    address or a size that is no whole word is refused."""
+    import torch
+
+    class Range(ctypes.Structure):
+        _fields_ = [("p", ctypes.c_void_p), ("bytes", ctypes.c_size_t)]
+
+    fn, lib = _fft_api(pkg), pkg.lib()
+    lib.p3mk_fill_zero_many.argtypes = [ctypes.c_int, ctypes.POINTER(Range), ctypes.c_void_p]
+    lib.p3mk_fill_zero.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+    q = ctypes.c_void_p()
+    assert fn["p3mk_queue_create"](ctypes.byref(q)) == 0
+    buf = torch.empty(200000, dtype=torch.int32, device="cuda")
+    sizes = [0, 1, 2, 3, 4, 5, 8, 1023, 40000]
+    for shift in range(4):
+        buf.fill_(-1)
+        torch.cuda.synchronize()
+        want = np.full(buf.numel(), -1, np.int32)
+        parts, at = [], 4
+        for k, w in enumerate(sizes[:8] if shift % 2 else sizes[1:]):
+            lo = at + (shift + k) % 4
+            parts.append((lo, w))
+            want[lo:lo + w] = 0
+            at = lo + w + 9
+        r = (Range * 8)(*[Range(buf.data_ptr() + 4 * lo, 4 * w) for lo, w in parts])
+        assert lib.p3mk_fill_zero_many(8, r, q) == 0
+        want[at + 1:at + 6] = 0
+        assert lib.p3mk_fill_zero(buf.data_ptr() + 4 * (at + 1), 20, q) == 0
+        assert lib.p3mk_fill_zero(buf.data_ptr() + 2, 8, q) != 0
+        assert lib.p3mk_fill_zero(buf.data_ptr(), 6, q) != 0
+        assert fn["p3mk_queue_sync"](q) == 0
+        assert np.array_equal(buf.cpu().numpy(), want)
+    fn["p3mk_queue_destroy"](q)
+
+
 @pytest.mark.parametrize("fp32", [0, 1])
 @pytest.mark.parametrize("M", [4, 6, 10, 14, 26, 32, 50, 90, 104, 112, 120, 150, 156, 160, 162, 220, 256])
 def test_fft_factor_splits(pkg, M, fp32):
