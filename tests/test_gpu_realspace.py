@@ -299,16 +299,16 @@ def test_stage_ring_pair_kernel_times(pkg):
 
 
 @pytest.mark.parametrize("prec_name", ["FP64", "MIXED"])
-@pytest.mark.parametrize("cells,per_cell", [(3, 37), (6, 9), (8, 8), (13, 4), (16, 3), (17, 3)])
-def test_items_dealt_to_several_wavefronts(pkg, orc, cells, per_cell, prec_name):
+@pytest.mark.parametrize("cells,per_cell,units", [(3, 37, 16), (6, 9, 8), (7, 8, 4), (8, 8, 2), (13, 4, 1), (16, 3, 1),
+                                                  (17, 3, 1)])
+def test_items_dealt_to_several_wavefronts(pkg, orc, cells, per_cell, units, prec_name):
     """Systems of few work items, whose neighbour cells are dealt out to 16,
     8, 4, 2 or one wavefront per item (items from 27 to above 4096, one cell
     of 150 particles among them so that items of one cell differ in chunks):
-    sums of up to 16 shares per particle, so the tolerance is that of the
-    other real-space tests (FP64 1e-13; mixed 1e-6 by the fixed-point quantum
-    at these densities' closest pairs, kept above 0.05)."""
-    import torch
-
+    sums of up to 16 shares per particle and of the energy, so the tolerances
+    are those of the other real-space tests (FP64 1e-13, energy 1e-12; mixed
+    1e-6 by the fixed-point quantum at these densities' closest pairs, kept
+    above 0.05, energy 1e-5)."""
     rcut, alpha = 3.0, 1.0
     L = rcut * cells * 1.001
     rng = np.random.default_rng(100 + cells)
@@ -322,18 +322,18 @@ def test_items_dealt_to_several_wavefronts(pkg, orc, cells, per_cell, prec_name)
     n = len(p)
     q = np.where(np.arange(n) % 2 == 0, 1.0, -1.0)
     s = {"x": p[:, 0].copy(), "y": p[:, 1].copy(), "z": p[:, 2].copy(), "q": q, "L": float(L)}
-    fr_ref, _ = orc.realteil(s, rcut, alpha, cells=True)
-    solver = pkg.Solver(7, pkg.HostSystem.from_dict(s), pkg.parameters(16, 3, alpha, rcut),
-                        getattr(pkg, prec_name))
-    dev = {k: torch.tensor(s[k], dtype=torch.float64, device="cuda") for k in "xyzq"}
-    fr = torch.zeros(3 * n, dtype=torch.float64, device="cuda")
-    torch.cuda.synchronize()
-    solver.realteil_device(n, L, *[dev[k].data_ptr() for k in "xyzq"], rcut, alpha, fr.data_ptr(), None)
-    solver.synchronize()
-    err = rel_err(fr.cpu().numpy().reshape(3, n), fr_ref)
-    print("cells %d n %d %s rel err %.2e" % (cells, n, prec_name, err))
+    fr_ref, e_ref = orc.realteil(s, rcut, alpha, cells=True)
+    f, e, nc = on_cells(pkg, s, rcut, alpha, 1, prec_name)
+    assert nc == cells
+    items = int(((cell_counts(s, nc) + 63) // 64).sum())
+    dealt = 1
+    while dealt < 16 and items * dealt < 1024:
+        dealt *= 2
+    assert dealt == units
+    err = rel_err(f, fr_ref)
+    print("cells %d n %d items %d %s rel err %.2e energy %.2e" % (cells, n, items, prec_name, err, abs(e / e_ref - 1)))
     assert err < (1e-13 if prec_name == "FP64" else 1e-6)
-    solver.close()
+    assert abs(e - e_ref) <= (1e-12 if prec_name == "FP64" else 1e-5) * abs(e_ref)
 
 
 @pytest.mark.parametrize("prec_name", ["FP64", "MIXED"])
@@ -366,6 +366,7 @@ def test_cell_size_follows_the_clustering(pkg, orc, layout, prec_name):
     solver.synchronize()
     err = rel_err(fr.cpu().numpy().reshape(3, n), fr_ref)
     print("%s %s rel err %.2e" % (layout, prec_name, err))
+    assert cells_of(pkg, solver)[1] == (1 if layout == "sparse" else 2)
     assert err < (1e-13 if prec_name == "FP64" else 1e-6)
     solver.close()
 
