@@ -479,6 +479,21 @@ def test_calculate_forces_writes_everything(pkg, orc, method, n, L, M, cao, rcut
     solver.close()
 
 
+@pytest.mark.parametrize("method,cao", [(3, 7), (0, 7), (2, 6), (6, 4)])
+def test_mixed_charges_of_any_unit(pkg, orc, method, cao):
+    """Charges times 2^100: every FP32 value of the mixed form is a power of
+    two times its usual one (mesh values up to 10^34 here, within FP32), so
+    the forces are 2^200 times the usual ones, to the mixed form's 1e-5."""
+    M, L, alpha, n = 16, 10.0, 1.0, 300
+    s = random_system(n, L, seed=5, charges="normal")
+    fk_ref, _ = orc.kspace_force(method, s, M, cao, alpha)
+    big = dict(s, q=s["q"] * 2.0 ** 100)
+    solver = pkg.Solver(method, pkg.HostSystem.from_dict(big), pkg.parameters(M, cao, alpha), pkg.MIXED)
+    got = solver.kspace_force().kspace() / 2.0 ** 200
+    solver.close()
+    assert rel_err(got, fk_ref) < 1e-5
+
+
 @pytest.mark.parametrize("method,n,L,M,cao,rcut", [
     (2, 333, 8.0, 16, 5, 3.9),   # nearest images: f_r is zero-filled too
     (7, 1001, 30.0, 32, 4, 3.0),
