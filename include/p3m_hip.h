@@ -512,7 +512,11 @@ int p3m_hip_format_out_row(char *buf, size_t size, const double v[8]);
 /* Stage times (ms, HIP events on the library's stream) of the last calls:
  * [0] charge assignment, [1] FFTs + influence-function multiply,
  * [2] back-interpolation, [3] whole Kspace_force, [4] last real-space call
- * (0 if none).  Waits for the stream. */
+ * (0 if none).  Of a Calculate_forces step they leave out what the stages
+ * share: the launch before them that clears the mesh, the counts and the force
+ * arrays, and the one after them that brings the real-space forces to the
+ * caller's order and sums (in a Kspace_force or Realteil call of its own the
+ * stages hold their clearing and reordering).  Waits for the stream. */
 int p3m_hip_stage_times(data_t *d, double out[5]);
 /* Per-step stage times without synchronising between steps: after
  * p3m_hip_stage_ring_start(d, n), each of the next n calls of

@@ -66,7 +66,7 @@ typedef struct {
     double *pos;    /* x, y, z, q blocks of n */
     double *force;  /* fk (3n), f (3n), fr (3n) */
     double *hforce; /* pinned staging, 9n */
-    double *hclust; /* pinned, one word: clustering of the positions */
+    double *hclust; /* the word behind it: clustering of the positions */
     double *energy; /* device scalar */
     int *iscratch;
     p3mk_cells *cells;
@@ -109,7 +109,6 @@ static void ctx_free(p3m_ctx *c) {
     p3mk_release(c->energy);
     p3mk_release(c->iscratch);
     p3mk_release_host(c->hforce);
-    p3mk_release_host(c->hclust);
     p3mk_cells_destroy(c->cells);
     p3mk_psort_destroy(c->psort);
     p3mk_queue_destroy(c->q);
@@ -174,8 +173,8 @@ static int ctx_alloc(p3m_ctx *c) {
     TRYK(p3mk_alloc((void **)&c->force, sizeof(double) * 9 * n), "forces");
     TRYK(p3mk_alloc((void **)&c->energy, sizeof(double)), "energy");
     TRYK(p3mk_alloc((void **)&c->iscratch, sizeof(int) * 16), "int scratch");
-    TRYK(p3mk_alloc_host((void **)&c->hforce, sizeof(double) * 9 * n), "pinned staging");
-    TRYK(p3mk_alloc_host((void **)&c->hclust, sizeof(double)), "pinned staging");
+    TRYK(p3mk_alloc_host((void **)&c->hforce, sizeof(double) * (9 * n + 1)), "pinned staging");
+    c->hclust = c->hforce + 9 * n;
     TRYK(p3mk_fill_zero(c->selfb, sizeof(double) * 81, c->q), "zero");
     TRYK(p3mk_fill_zero(c->G, sizeof(double) * M3, c->q), "zero");
     TRYK(p3mk_queue_sync(c->q), "sync");

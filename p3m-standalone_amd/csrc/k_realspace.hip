@@ -545,16 +545,16 @@ __device__ __forceinline__ int next_item(int *counter, Claims &c) {
     return c.next++;
 }
 
-// Units per work item: when the items are fewer than the GPU has wavefront
-// slots, an item's neighbour cells are dealt out to
-// 2^split_bits wavefronts (each walks every 2^split_bits-th live cell and
-// adds its share of the forces), so that a small system's chain of windows
-// is shared.  With the first claims by block index, whole steps: 1,000
-// particles FP64 159 -> 120 us, 7,777 mixed 192 -> 149 us, 100,000 mixed
-// 240 -> 154 us, a batch of 24 small systems 542 -> 455 us; a million
-// particles 6.26 -> 6.15 ms.
+// Units per work item: when the items are fewer than a wavefront per SIMD, an
+// item's neighbour cells are dealt out to 2^split_bits wavefronts (each walks
+// every 2^split_bits-th live cell and adds its share of the forces), so that a
+// small system's chain of windows is shared.  Real space without and with it,
+// us: 1,000 uniform particles FP64 106 / 60, mixed 87 / 54; 4,000 FP64
+// 102 / 62; 7,777 FP64 151 / 90, mixed 119 / 73; 16,000 FP64 114 / 93.  Dealt
+// until 4096 units, the pair kernel of 32,768 particles FP64 took 78 us, 57 as
+// it is.
 constexpr int kMaxSplitBits = 4;
-constexpr int kSplitUnits = 1024; // a wavefront per SIMD; 4096 took 78 us where 1024 took 57 (32,768 particles FP64)
+constexpr int kSplitUnits = 1024;
 __device__ __forceinline__ int split_bits_of(int total) {
     int b = 0;
     while (b < kMaxSplitBits && (total << b) < kSplitUnits)
@@ -1515,7 +1515,8 @@ realspace_item_half(int home, int chunk, int cell0, const double4 *__restrict__ 
 }
 
 // Persistent grid as k_realspace over the half shell; fs (3 n, sorted order)
-// is zeroed by the caller and added to the forces by k_unsort_add.  Queue
+// is zeroed by the caller and brought to the caller's order by
+// k_finish_forces (Calculate_forces) or k_unsort_add (real space alone).  Queue
 // rounds are evaluated two at a time in both forms; FP32: four waves per
 // SIMD (7.07 ms at the Gaussian 1M workload; five with single rounds 7.35,
 // five with paired rounds 8.06 from spills); FP64: three (12.0 ms against
