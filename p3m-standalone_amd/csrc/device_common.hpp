@@ -66,7 +66,7 @@ __device__ __forceinline__ void locate(double r, double Hi, double pos_shift, do
 }
 
 // Weights (and optionally derivative weights) of the P stencil points along
-// one axis, each over the spline's norm (stencil_norm<P> normalises the
+// one axis, each over the spline's norm (stencil_norm<P, T> normalises the
 // product of three).
 template <int P, typename T>
 __device__ __forceinline__ void axis_weights(double r, double Hi, double half_ii, int M,

@@ -221,7 +221,7 @@ k_collect(int n, int M, double L, const double *x, const double *y, const double
     axis_weights<P, double>(x[i], Hi, 0.0, M, b[0], w[0]);
     axis_weights<P, double>(y[i], Hi, 0.0, M, b[1], w[1]);
     axis_weights<P, double>(z[i], Hi, 0.0, M, b[2], w[2]);
-    const double q2 = q[i] * q[i] * stencil_norm<P>;
+    const double q2 = q[i] * q[i] * stencil_norm<P, double>;
     double acc = 0.0;
     for (int a = 0; a < P; a++) {
         const int ia = wrap1(b[0] + a, M);

@@ -415,7 +415,7 @@ k_adjoint_ik(int n, const double4 *__restrict__ sorted, const int *__restrict__ 
             }
         }
     }
-    const double s = (IL ? 0.5 * prefac : prefac) * stencil_norm<P>;
+    const double s = (IL ? 0.5 * prefac : prefac) * stencil_norm<P, T>;
     dq[i] += -s * aq.value();
     dpos[i] += -s * qi * Hi * ax.value();
     dpos[(long)n + i] += -s * qi * Hi * ay.value();
@@ -486,7 +486,7 @@ k_adjoint_ad(int n, const double4 *__restrict__ sorted, const int *__restrict__ 
             }
         }
     }
-    const double s = (IL ? 0.5 * prefac : prefac) * stencil_norm<P>;
+    const double s = (IL ? 0.5 * prefac : prefac) * stencil_norm<P, T>;
     double dqi = -s * aq.value();
     double dx = -s * qi * Hi * ax.value(), dy = -s * qi * Hi * ay.value(),
            dz = -s * qi * Hi * az.value();

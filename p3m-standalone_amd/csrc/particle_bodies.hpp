@@ -194,7 +194,7 @@ assign_rows_item(const double4 *__restrict__ sorted, int pb, int pe, long tl, in
             const double gq = gn;
             fetch(rd + 1, rn, gn);
             if (lane < nb) {
-                const double qn = r.w * stencil_norm<P>;
+                const double qn = r.w * stencil_norm<P, T>;
                 T qv = (T)qn;
                 if (MODE == kWeighted)
                     qv = (T)(qn * gq);
@@ -286,7 +286,7 @@ assign_item(const double4 *__restrict__ sorted, int pb, int pe, long tl, int nt,
     __syncthreads();
     for (int p = pb + threadIdx.x; p < pe; p += blockDim.x) {
         const double4 r = sorted[p];
-        const double qn = r.w * stencil_norm<P>;
+        const double qn = r.w * stencil_norm<P, T>;
         T qv = (T)qn;
         T g0 = T(0), g1 = T(0), g2 = T(0);
         if (MODE == kWeighted) {
@@ -403,7 +403,7 @@ interp_ik_item(const double4 *__restrict__ sorted, const int *__restrict__ perm,
     const int npts = R * R * R;
     const int tz = (int)(tl % nt), ty = (int)((tl / nt) % nt), tx = (int)(tl / ((long)nt * nt));
     const int t0x = tx * Tt, t0y = ty * Tt, t0z = tz * Tt;
-    const double sc = (IL ? 0.5 * prefac : prefac) * stencil_norm<P>;
+    const double sc = (IL ? 0.5 * prefac : prefac) * stencil_norm<P, T>;
     for (int d = 0; d < 3; d++) {
         const T *F = d == 0 ? F0 : (d == 1 ? F1 : F2);
         for_region(R, M, t0x, t0y, t0z, [&](int lx, int ly, int lz, long g) {
@@ -548,7 +548,7 @@ interp_ad_item(const double4 *__restrict__ sorted, const int *__restrict__ perm,
                 F[2] += (double)w0[a] * (double)sz;
             }
         }
-        const double scale = (IL ? 0.5 * prefac : prefac) * stencil_norm<P> * (r.w * Leni);
+        const double scale = (IL ? 0.5 * prefac : prefac) * stencil_norm<P, T> * (r.w * Leni);
         const int i = perm[p];
         fk[i] -= scale * F[0];
         fk[stride + i] -= scale * F[1];
