@@ -357,6 +357,8 @@ extern "C" int p3mk_batch_configure(p3mk_batch *b, int fp32, int use_self_force,
                                     int rs_grid) {
     if (tile_side != 4 && tile_side != 8)
         return p3mk_fail(P3MK_EINVAL, "assignment tile side must be 4 or 8", 0);
+    if (use_self_force && b->form.interlaced)
+        return p3mk_fail(P3MK_EINVAL, "no self-force correction in the interlaced methods", 0);
     b->form.fp32 = fp32 != 0;
     b->use_self = use_self_force != 0;
     b->tile_side = tile_side;

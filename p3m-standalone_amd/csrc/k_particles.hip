@@ -490,7 +490,7 @@ k_adjoint_ad(int n, const double4 *__restrict__ sorted, const int *__restrict__ 
     double dqi = -s * aq.value();
     double dx = -s * qi * Hi * ax.value(), dy = -s * qi * Hi * ay.value(),
            dz = -s * qi * Hi * az.value();
-    if (selfb != nullptr) {
+    if (!IL && selfb != nullptr) {
         // f_{i,d} -= q_i^2 sum_m' b_d(m') sin(theta), theta = 2 pi m'.r / h
         const double c0 = 2 * 3.14159265358979323846 / h;
         const double q2 = qi * qi;
@@ -957,6 +957,8 @@ extern "C" int p3mk_interp_ad(const p3mk_geom *g, int n, const p3mk_psort *s, co
         return p3mk_fail(P3MK_EINVAL, "interpolation needs the sort of the same particles", 0);
     if (selfb != nullptr && f == nullptr)
         return p3mk_fail(P3MK_EINVAL, "self-force correction needs the total-force array", 0);
+    if (selfb != nullptr && g->interlaced)
+        return p3mk_fail(P3MK_EINVAL, "no self-force correction in the interlaced methods", 0);
     if (g->fp32)
         return g->r2c ? launch_interp_ad<float, true>(g, n, s, phi, prefac, selfb, fk, f, qu)
                       : launch_interp_ad<float, false>(g, n, s, phi, prefac, selfb, fk, f, qu);
@@ -972,6 +974,8 @@ extern "C" int p3mk_adjoint_gather(const p3mk_geom *g, int ad, int n, const p3mk
         return P3MK_OK;
     if (n != s->n)
         return p3mk_fail(P3MK_EINVAL, "adjoint needs the sort of the same particles", 0);
+    if (selfb != nullptr && g->interlaced)
+        return p3mk_fail(P3MK_EINVAL, "no self-force correction in the interlaced methods", 0);
     if (g->fp32)
         return g->r2c ? launch_adjoint<float, true>(g, ad, n, s, q, gv, F, lam, prefac, selfb, dpos, dq, qu)
                       : launch_adjoint<float, false>(g, ad, n, s, q, gv, F, lam, prefac, selfb, dpos, dq, qu);
