@@ -369,7 +369,7 @@ k_interp_ad_tile(const double4 *__restrict__ sorted, const int *__restrict__ per
 // Derivatives are those of the B-spline weights at the quantised offsets
 // (d/dx = Hi d/du); outputs accumulate (+=) in the caller's order.
 template <int P, typename T, bool R2C, bool IL>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(kThreads)
 k_adjoint_ik(int n, const double4 *__restrict__ sorted, const int *__restrict__ perm,
              const double *__restrict__ q, const double *__restrict__ gv, double Hi, int M,
              const T *__restrict__ F0, const T *__restrict__ F1, const T *__restrict__ F2,
@@ -423,7 +423,7 @@ k_adjoint_ik(int n, const double4 *__restrict__ sorted, const int *__restrict__ 
 }
 
 template <int P, typename T, bool R2C, bool IL>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(kThreads)
 k_adjoint_ad(int n, const double4 *__restrict__ sorted, const int *__restrict__ perm,
              const double *__restrict__ q, const double *__restrict__ gv, double Hi, int M,
              const T *__restrict__ phi, const T *__restrict__ lam, double prefac,
@@ -789,9 +789,19 @@ int assign_mode(const p3mk_geom *g, int n, p3mk_psort *s, void *mesh, int mode, 
                   : assign_mode_t<double, false>(g, n, s, mesh, mode, gv, qu);
 }
 
-// Workgroups of the adjoint gather: one wavefront each, so that a system of
-// 10,000 particles reaches most CUs (workgroups of 256 were 48 of them, 78 us).
+// Threads a workgroup of the adjoint gather: one wavefront, so that a system of
+// 10,000 particles reaches most CUs (12,345 particles ad-i FP64 order 5: 50 us
+// against 60 with four).  Interlaced gathers read two points a place; from
+// 65,536 particles on, where four wavefronts a workgroup fill the GPU too, they
+// share what they read in L1: 131,072 particles 99 us against 116 (ad-i FP64
+// order 5), 194 against 251 (FP32 order 7), 620 against 640 (ik-i FP64 order
+// 7).  The FP32 ik-i gather keeps one (524,288 particles order 5: 772 against
+// 880).
 constexpr int kGatherThreads = 64;
+constexpr int kGatherShared = 65536;
+template <typename T> int gather_threads(int n, int ad, int interlaced) {
+    return interlaced && n >= kGatherShared && (ad || sizeof(T) == 8) ? kThreads : kGatherThreads;
+}
 
 template <typename T, bool R2C>
 int launch_adjoint(const p3mk_geom *g, int ad, int n, const p3mk_psort *s, const double *q,
@@ -799,7 +809,8 @@ int launch_adjoint(const p3mk_geom *g, int ad, int n, const p3mk_psort *s, const
                    const double *selfb, double *dpos, double *dq, p3mk_queue *qu) {
     const double Hi = (double)g->M / g->L;
     const double h = g->L / g->M;
-    const dim3 grid((unsigned)((n + kGatherThreads - 1) / kGatherThreads));
+    const int threads = gather_threads<T>(n, ad, g->interlaced);
+    const dim3 grid((unsigned)((n + threads - 1) / threads));
     const T *F0 = (const T *)F[0], *F1 = (const T *)F[1], *F2 = (const T *)F[2];
     const T *la = (const T *)lam;
     hipStream_t st = p3mk_stream(qu);
@@ -809,20 +820,20 @@ int launch_adjoint(const p3mk_geom *g, int ad, int n, const p3mk_psort *s, const
     case P:                                                                                        \
         if (ad) {                                                                                  \
             if (il)                                                                                \
-                hipLaunchKernelGGL((k_adjoint_ad<P, T, R2C, true>), grid, dim3(kGatherThreads), 0, st, n, \
+                hipLaunchKernelGGL((k_adjoint_ad<P, T, R2C, true>), grid, dim3(threads), 0, st, n, \
                                    s->sorted, s->perm, q, gv, Hi, g->M, F0, la, prefac, selfb, h,  \
                                    dpos, dq);                                                      \
             else                                                                                   \
-                hipLaunchKernelGGL((k_adjoint_ad<P, T, R2C, false>), grid, dim3(kGatherThreads), 0, st,  \
+                hipLaunchKernelGGL((k_adjoint_ad<P, T, R2C, false>), grid, dim3(threads), 0, st,  \
                                    n, s->sorted, s->perm, q, gv, Hi, g->M, F0, la, prefac, selfb,  \
                                    h, dpos, dq);                                                   \
         } else {                                                                                   \
             if (il)                                                                                \
-                hipLaunchKernelGGL((k_adjoint_ik<P, T, R2C, true>), grid, dim3(kGatherThreads), 0, st, n, \
+                hipLaunchKernelGGL((k_adjoint_ik<P, T, R2C, true>), grid, dim3(threads), 0, st, n, \
                                    s->sorted, s->perm, q, gv, Hi, g->M, F0, F1, F2, la, prefac,    \
                                    dpos, dq);                                                      \
             else                                                                                   \
-                hipLaunchKernelGGL((k_adjoint_ik<P, T, R2C, false>), grid, dim3(kGatherThreads), 0, st,  \
+                hipLaunchKernelGGL((k_adjoint_ik<P, T, R2C, false>), grid, dim3(threads), 0, st,  \
                                    n, s->sorted, s->perm, q, gv, Hi, g->M, F0, F1, F2, la, prefac, \
                                    dpos, dq);                                                      \
         }                                                                                          \

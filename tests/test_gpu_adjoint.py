@@ -310,3 +310,37 @@ def test_total_force_autograd(pkg, orc):
     assert rel_err(pos.grad.cpu().numpy(), fd_pos) < 2e-7
     assert rel_err(q.grad.cpu().numpy(), fd_q) < 1e-9
     solver.close()
+
+
+@pytest.mark.parametrize("method,cao,prec_name", [(3, 5, "FP64"), (3, 7, "MIXED"), (1, 5, "FP64"), (1, 4, "MIXED")])
+def test_gather_workgroups(pkg, method, cao, prec_name):
+    """Interlaced gathers take larger workgroups from 65,536 particles on: a
+    system of 65,535, and the same with one and with 700 more particles of no
+    charge and no cotangent, have the same adjoint (FP64 1e-12; mixed 1e-5,
+    its FP32 mesh sums in another order)."""
+    import torch
+
+    n0, L, M = 65535, 40.0, 32
+    rng = np.random.default_rng(21)
+    n1 = n0 + 700
+    pos = rng.uniform(0.0, L, (3, n1))
+    q = rng.normal(0.0, 1.0, n1)
+    g = rng.normal(0.0, 1.0, (3, n1))
+    q[n0:] = 0.0
+    g[:, n0:] = 0.0
+    got = []
+    for n in (n0, n0 + 1, n1):
+        system = pkg.HostSystem(pos[0, :n].copy(), pos[1, :n].copy(), pos[2, :n].copy(), q[:n].copy(), L)
+        solver = pkg.Solver(method, system, pkg.parameters(M, cao, 1.0), getattr(pkg, prec_name))
+        dev = [torch.tensor(np.ascontiguousarray(a[:n]), device="cuda") for a in (*pos, q)]
+        cot = torch.tensor(np.ascontiguousarray(g[:, :n]).reshape(-1), device="cuda")
+        dpos = torch.zeros(3 * n, dtype=torch.float64, device="cuda")
+        dq = torch.zeros(n, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        solver.kspace_force_vjp_device(n, L, *[a.data_ptr() for a in dev], cot.data_ptr(), dpos.data_ptr(),
+                                       dq.data_ptr())
+        solver.synchronize()
+        got.append(np.concatenate([dpos.cpu().numpy().reshape(3, n)[:, :n0].ravel(), dq.cpu().numpy()[:n0]]))
+        solver.close()
+    tol = 1e-12 if prec_name == "FP64" else 1e-5
+    assert np.isfinite(got[0]).all() and rel_err(got[1], got[0]) < tol and rel_err(got[2], got[0]) < tol
